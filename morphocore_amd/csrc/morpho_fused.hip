@@ -87,35 +87,93 @@ __device__ __forceinline__ PairWork decode_pair(int ncg, int ntx, int nty)
     return w;
 }
 
-// Strict first-tap scan (reference tap order kh, then kw) of the pixel whose tap (kh, kw) reads
+// First-tap scan (reference tap order kh, then kw) of the pixel whose tap (kh, kw) reads
 // win[r + K - 1 - kh][K - 1 - kw]: the extremum and its first tap; a pixel that never improves on
-// the start value keeps it with tap 0. The running extremum is kept with the NaN-ignoring max / min,
-// which equals the strict scan's up to the sign of a zero, so the strict comparison against it picks
-// the same first tap; a zero result takes the value of that tap, whose sign is the strict scan's.
+// the start value keeps it with tap 0.
+//  * float32: each row of taps folds to its extremum (max3 / min3), the first row holding the overall
+//    extremum and its values are selected, and the first tap of that row equal to it is the strict
+//    scan's; a zero result takes the value of that tap, whose sign is the strict scan's. 2.1 slow
+//    operations per 5x5 tap against the 3 of the running scan below.
+//  * float64, which has no max3 / min3: the running extremum is kept with the NaN-ignoring max / min,
+//    which equals the strict scan's up to the sign of a zero, so the strict comparison against it
+//    picks the same first tap (the row form measured 7-12% slower from 3x3 to 7x7).
+// An opening of (8, 32, 179, 250), float32: 5x5 120 -> 110 us, 7x7 377 -> 233 (with pair_unroll); its
+// quantised inputs, whose zero results read their tap again, 168 -> 103 and 690 -> 211.
 template <int OP, typename T, int K, int WR>
 __device__ __forceinline__ void pair_scan(const T (&win)[WR][K], int r, const T* wk, T& best, int& arg)
 {
     using Tr = OpTraits<OP, T>;
-    T m = Tr::init();
-    arg = 0;
-#pragma unroll
-    for (int kh = 0; kh < K; ++kh)
-#pragma unroll
-        for (int kw = 0; kw < K; ++kw)
-        {
-            const T v = Tr::combine(win[r + K - 1 - kh][K - 1 - kw], wk[kh * K + kw]);
-            arg = Tr::better(v, m) ? kh * K + kw : arg;
-            m = Tr::pick(m, v);
-        }
-    best = m;
-    if (m == T(0))
+    if constexpr (sizeof(T) == 4)
     {
+        T v[K][K], m[K], e = Tr::init();
+#pragma unroll
+        for (int kh = 0; kh < K; ++kh)
+        {
+#pragma unroll
+            for (int kw = 0; kw < K; ++kw) v[kh][kw] = Tr::combine(win[r + K - 1 - kh][K - 1 - kw], wk[kh * K + kw]);
+            m[kh] = v[kh][0];
+#pragma unroll
+            for (int kw = 1; kw < K; ++kw) m[kh] = Tr::pick(m[kh], v[kh][kw]);
+        }
+#pragma unroll
+        for (int kh = 0; kh < K; ++kh) e = Tr::pick(e, m[kh]);
+        // The last row stands when none holds it: then it is the start value.
+        int krow = (K - 1) * K, kcol = 0;
+        T rv[K];
+#pragma unroll
+        for (int kw = 0; kw < K; ++kw) rv[kw] = v[K - 1][kw];
+#pragma unroll
+        for (int kh = K - 2; kh >= 0; --kh)
+        {
+            const bool eq = m[kh] == e;
+            krow = eq ? kh * K : krow;
+#pragma unroll
+            for (int kw = 0; kw < K; ++kw) rv[kw] = eq ? v[kh][kw] : rv[kw];
+        }
+        T first = rv[0];
+#pragma unroll
+        for (int kw = K - 1; kw >= 0; --kw)
+        {
+            const bool eq = rv[kw] == e;
+            kcol = eq ? kw : kcol;
+            first = eq ? rv[kw] : first;
+        }
+        const bool none = e == Tr::init();
+        arg = none ? 0 : krow + kcol;
+        best = none ? e : first;
+    }
+    else
+    {
+        T m = Tr::init();
+        arg = 0;
 #pragma unroll
         for (int kh = 0; kh < K; ++kh)
 #pragma unroll
             for (int kw = 0; kw < K; ++kw)
-                if (arg == kh * K + kw) best = Tr::combine(win[r + K - 1 - kh][K - 1 - kw], wk[kh * K + kw]);
+            {
+                const T v = Tr::combine(win[r + K - 1 - kh][K - 1 - kw], wk[kh * K + kw]);
+                arg = Tr::better(v, m) ? kh * K + kw : arg;
+                m = Tr::pick(m, v);
+            }
+        best = m;
+        if (m == T(0))
+        {
+#pragma unroll
+            for (int kh = 0; kh < K; ++kh)
+#pragma unroll
+                for (int kw = 0; kw < K; ++kw)
+                    if (arg == kh * K + kw) best = Tr::combine(win[r + K - 1 - kh][K - 1 - kw], wk[kh * K + kw]);
+        }
     }
+}
+
+// Rows of pixels whose windows a lane holds in registers together: all of its rows share the window's
+// rows (one LDS read each), except float32 7x7, where that takes 256 registers (one wave per SIMD)
+// and one row at a time takes 160 (three): 330 -> 233 us at the shape above.
+template <typename T, int K>
+constexpr int pair_unroll(int rows)
+{
+    return sizeof(T) == 4 && K == 7 ? 1 : rows;
 }
 
 // Each workgroup walks `chans` consecutive channels of one tile; the next channel's input tile and
@@ -198,26 +256,31 @@ __global__ __launch_bounds__(BLOCK) void morpho_pair_fwd_kernel(const PairFwdPar
 #pragma unroll
             for (int k = 0; k < KK; ++k) wr[k] = ws[buf][k];
             const int r0 = wave * RE;
-            T win[RE + K - 1][K];
-#pragma unroll
-            for (int rr = 0; rr < RE + K - 1; ++rr)
-#pragma unroll
-                for (int kw = 0; kw < K; ++kw) win[rr][kw] = xs[buf][min(r0 + rr, XR - 1) * XC + lane + kw];
-#pragma unroll
-            for (int j = 0; j < RE; ++j)
+            constexpr int U = pair_unroll<T, K>(RE);
+#pragma unroll 1
+            for (int j0 = 0; j0 < RE; j0 += U)
             {
-                const int ly = r0 + j;
-                T best;
-                int arg;
-                pair_scan<OP1, T, K>(win, j, wr, best, arg);
-                const int gy = ey0 + ly;
-                const bool in = gy >= 0 && gy < H && gx1 >= 0 && gx1 < W;
-                // REPLICATE: a column outside the image takes the clamped column's value (another lane
-                // of the same row); rows outside the image are copied after the pass.
-                const T moved = shfl_t(best, src_lane);
-                if (ly < ER) es[ly * TILE_W + lane] = p.replicate ? moved : (in ? best : p.fill2);
-                if (p.taps1 && in && own_col1 && ly >= K - 1 - P && ly < K - 1 - P + TH)
-                    p.taps1[pbase + (int64_t)gy * W + gx1] = (uint8_t)arg;
+                T win[U + K - 1][K];
+#pragma unroll
+                for (int rr = 0; rr < U + K - 1; ++rr)
+#pragma unroll
+                    for (int kw = 0; kw < K; ++kw) win[rr][kw] = xs[buf][min(r0 + j0 + rr, XR - 1) * XC + lane + kw];
+#pragma unroll
+                for (int j = 0; j < U; ++j)
+                {
+                    const int ly = r0 + j0 + j;
+                    T best;
+                    int arg;
+                    pair_scan<OP1, T, K>(win, j, wr, best, arg);
+                    const int gy = ey0 + ly;
+                    const bool in = gy >= 0 && gy < H && gx1 >= 0 && gx1 < W;
+                    // REPLICATE: a column outside the image takes the clamped column's value (another lane
+                    // of the same row); rows outside the image are copied after the pass.
+                    const T moved = shfl_t(best, src_lane);
+                    if (ly < ER) es[ly * TILE_W + lane] = p.replicate ? moved : (in ? best : p.fill2);
+                    if (p.taps1 && in && own_col1 && ly >= K - 1 - P && ly < K - 1 - P + TH)
+                        p.taps1[pbase + (int64_t)gy * W + gx1] = (uint8_t)arg;
+                }
             }
         }
         __syncthreads();
@@ -238,23 +301,28 @@ __global__ __launch_bounds__(BLOCK) void morpho_pair_fwd_kernel(const PairFwdPar
             T wr[KK];
 #pragma unroll
             for (int k = 0; k < KK; ++k) wr[k] = ws[buf][KK + k];
-            T win[RH + K - 1][K];
-#pragma unroll
-            for (int rr = 0; rr < RH + K - 1; ++rr)
-#pragma unroll
-                for (int kw = 0; kw < K; ++kw) win[rr][kw] = es[(wave * RH + rr) * TILE_W + lcol + kw];
-#pragma unroll
-            for (int r = 0; r < RH; ++r)
+            constexpr int U = pair_unroll<T, K>(RH);
+#pragma unroll 1
+            for (int r0 = 0; r0 < RH; r0 += U)
             {
-                const int h = h0 + wave * RH + r;
-                T best;
-                int arg;
-                pair_scan<OP2, T, K>(win, r, wr, best, arg);
-                if (lane < OW && h < H && wc < W)
+                T win[U + K - 1][K];
+#pragma unroll
+                for (int rr = 0; rr < U + K - 1; ++rr)
+#pragma unroll
+                    for (int kw = 0; kw < K; ++kw) win[rr][kw] = es[(wave * RH + r0 + rr) * TILE_W + lcol + kw];
+#pragma unroll
+                for (int r = 0; r < U; ++r)
                 {
-                    const int64_t oi = pbase + (int64_t)h * W + wc;
-                    p.out[oi] = best;
-                    if (p.taps2) p.taps2[oi] = (uint8_t)arg;
+                    const int h = h0 + wave * RH + r0 + r;
+                    T best;
+                    int arg;
+                    pair_scan<OP2, T, K>(win, r, wr, best, arg);
+                    if (lane < OW && h < H && wc < W)
+                    {
+                        const int64_t oi = pbase + (int64_t)h * W + wc;
+                        p.out[oi] = best;
+                        if (p.taps2) p.taps2[oi] = (uint8_t)arg;
+                    }
                 }
             }
         }
@@ -388,27 +456,32 @@ __global__ __launch_bounds__(BLOCK) void morpho_sigma_fwd_kernel(const SigmaPara
         }
         const T s = ws[buf][2 * KK];
         const T oms = T(1) - s;
-        T win[RH + K - 1][K];
-#pragma unroll
-        for (int rr = 0; rr < RH + K - 1; ++rr)
-#pragma unroll
-            for (int kw = 0; kw < K; ++kw) win[rr][kw] = xs[buf][(wave * RH + rr) * XC + lane + kw];
-#pragma unroll
-        for (int r = 0; r < RH; ++r)
+        constexpr int U = pair_unroll<T, K>(RH);
+#pragma unroll 1
+        for (int r0 = 0; r0 < RH; r0 += U)
         {
-            const int h = h0 + wave * RH + r;
-            T e, d;
-            int te, td;
-            pair_scan<EROSION, T, K>(win, r, wer, e, te);
-            pair_scan<DILATION, T, K>(win, r, wdr, d, td);
-            if (h < H && wc < W)
+            T win[U + K - 1][K];
+#pragma unroll
+            for (int rr = 0; rr < U + K - 1; ++rr)
+#pragma unroll
+                for (int kw = 0; kw < K; ++kw) win[rr][kw] = xs[buf][(wave * RH + r0 + rr) * XC + lane + kw];
+#pragma unroll
+            for (int r = 0; r < U; ++r)
             {
-                const int64_t oi = pbase + (int64_t)h * W + wc;
-                p.out[oi] = sigma_blend(e, d, oms, s);
-                if (p.tapse)
+                const int h = h0 + wave * RH + r0 + r;
+                T e, d;
+                int te, td;
+                pair_scan<EROSION, T, K>(win, r, wer, e, te);
+                pair_scan<DILATION, T, K>(win, r, wdr, d, td);
+                if (h < H && wc < W)
                 {
-                    p.tapse[oi] = (uint8_t)te;
-                    p.tapsd[oi] = (uint8_t)td;
+                    const int64_t oi = pbase + (int64_t)h * W + wc;
+                    p.out[oi] = sigma_blend(e, d, oms, s);
+                    if (p.tapse)
+                    {
+                        p.tapse[oi] = (uint8_t)te;
+                        p.tapsd[oi] = (uint8_t)td;
+                    }
                 }
             }
         }
