@@ -899,7 +899,7 @@ static hipError_t launch_fwd(const FwdParams<ST>& p, hipStream_t stream)
 }
 
 template <typename ST, int OP>
-static hipError_t forward_op(int merge, FwdParams<ST> p, hipStream_t stream)
+hipError_t forward_op(int merge, FwdParams<ST> p, hipStream_t stream)
 {
     const bool save = p.idx != nullptr;
     // Output channels sharing each staged input tile: 4 for the value modes; 2 when every pair's tap
@@ -939,32 +939,8 @@ static hipError_t forward_op(int merge, FwdParams<ST> p, hipStream_t stream)
     }
 }
 
-template <typename ST>
-hipError_t morpho_forward(int op, int merge, bool replicate, compute_t<ST> fill, const ST* x, const ST* w, ST* out, void* indices,
-                          const Geom& g, hipStream_t stream)
-{
-    if ((int64_t)g.B * g.Cout * g.plane() == 0) return hipSuccess;
-    if (g.Cin == 0 && merge != MERGE_IDENTITY)
-    {
-        const int64_t n = (int64_t)g.B * g.Cout * g.plane();
-        hipError_t err = fill_async<ST>(out, n, empty_merge_value<ST>(merge), stream);
-        if (err == hipSuccess && indices && packed_winners(merge)) err = fill_async<int32_t>(static_cast<int32_t*>(indices), n, 0, stream);
-        return err;
-    }
-    FwdParams<ST> p{};
-    p.x = x;
-    p.w = w;
-    p.out = out;
-    p.idx = indices;
-    p.g = g;
-    p.replicate = replicate ? 1 : 0;
-    p.fill = fill;
-    p.average = 0;
-    return op == DILATION ? forward_op<ST, DILATION>(merge, p, stream) : forward_op<ST, EROSION>(merge, p, stream);
-}
-
-#define MCA_INSTANTIATE_FWD(ST)                                                                                                        \
-    template hipError_t morpho_forward<ST>(int, int, bool, compute_t<ST>, const ST*, const ST*, ST*, void*, const Geom&, hipStream_t); \
-    template size_t morpho_forward_lds<ST>(const Geom&);
+// The instances of one operation and storage type, each compiled in a source of its own (they take
+// minutes together): morpho_fwd.hip and morpho_fwd_*.hip.
+#define MCA_INSTANTIATE_FWD(ST, OP) template hipError_t forward_op<ST, OP>(int, FwdParams<ST>, hipStream_t);
 
 }  // namespace mca

@@ -1,0 +1,7 @@
+// Dilation / erosion forward for gfx950: float32 dilation instances of the kernels of morpho_fwd.hpp.
+#include "morpho_fwd.hpp"
+
+namespace mca
+{
+MCA_INSTANTIATE_FWD(float, DILATION)
+}  // namespace mca
