@@ -131,10 +131,39 @@ IdentBands ident_bands(const Geom& g, size_t elem_bytes, bool backward);
 template <typename ST>
 hipError_t ident_band_forward(int op, bool replicate, ST fill, const ST* x, const ST* w, ST* out, uint8_t* taps, const Geom& g,
                               hipStream_t stream);
-// Backward from the saved taps: grad_input, and grad_weight's sums per (batch element, band) in
-// part ([B * nbands][Cout][KH * KW], T: double for double storage, else float).
+// Backward of double tensors from the saved taps: grad_input, and grad_weight's sums per (batch element,
+// band) in part ([B * nbands][Cout][KH * KW]).
+hipError_t ident_band_backward(int op, const uint8_t* taps, const double* grad_out, double* grad_in, double* part, const Geom& g,
+                               hipStream_t stream);
+
+// grad_input by tiles summed in LDS (morpho_scatter.hip): each tile's pixels (and input channels, MAX /
+// MIN) by one workgroup, written once. ok: whether the shape takes it.
+struct PackedTiles
+{
+    int cg, ncg;           // input channels per workgroup, their groups
+    int tw, th, ntx, nty;  // tile of grad_input pixels
+    int threads;
+    int64_t blocks;
+    size_t lds;
+    bool ok;
+};
+PackedTiles packed_tiles(const Geom& g);
+// MAX / MIN, grad_input only, from the packed winners.
 template <typename T, typename ST>
-hipError_t ident_band_backward(int op, const uint8_t* taps, const ST* grad_out, ST* grad_in, T* part, const Geom& g, hipStream_t stream);
+hipError_t packed_tile_backward(const int32_t* idx, const ST* grad_out, ST* grad_in, const Geom& g, hipStream_t stream);
+struct IdentTiles
+{
+    int tw, th, ntx, nty;
+    int ncopy_log2;  // copies of each grad_weight bin
+    int64_t blocks;
+    size_t lds;
+    bool ok;
+};
+IdentTiles ident_tiles(const Geom& g);
+// IDENTITY: grad_input, and grad_weight's sums per (batch element, tile) in part
+// ([B * ntx * nty][Cout][KH * KW], T: double for double storage, else float).
+template <typename T, typename ST>
+hipError_t ident_tile_backward(int op, const void* taps, const ST* grad_out, ST* grad_in, T* part, const Geom& g, hipStream_t stream);
 
 // Opening / closing with IDENTITY merges fused into one pass (morpho_fused.hip). g: Cin == Cout == C,
 // Cw == 1; first_op: the first stage's op.

@@ -1,10 +1,11 @@
 // Dilation / erosion backward for gfx950: gradient routing from the winners of the forward pass.
 //
-// MAX / MIN (morpho_bwd_packed_kernel): one workgroup per (output channel, pixel chunk) scatters each
-// output gradient to its packed (channel, tap): grad_input by global double atomics (one per output
-// pixel; a pixel can collect up to Cout * KH * KW of them, which float32 sums would round past the
-// 1e-6 tolerance), rounded once to float32 afterwards, grad_weight into LDS bins that become this
-// workgroup's partial slot. Small problems (whose time is launches) gather grad_input instead, in
+// MAX / MIN (morpho_bwd_packed_kernel): one workgroup per (output channel, pixel chunk) sums each output
+// gradient to its packed (channel, tap) in LDS bins of grad_weight that become this workgroup's partial
+// slot; grad_input is summed by tiles in LDS (morpho_scatter.hip). Elements too large for the tiles
+// scatter it here, by global double atomics (one per output pixel; a pixel can collect up to
+// Cout * KH * KW of them, which float32 sums would round past the 1e-6 tolerance), rounded once to
+// float32 afterwards. Small problems (whose time is launches) gather grad_input instead, in
 // further workgroups of the same launch: each input pixel sums, in double and in (output channel,
 // tap) order, the gradients of the output pixels whose winner it is, written once (no zero fill, no
 // atomics, no rounding pass), and keep at most 32 slots (one reduction launch).
@@ -23,10 +24,11 @@
 //                             structuring-element column, which makes the atomic adds bank-conflict
 //                             free (measured: the scattered adds of one shared tile spend ~3x their
 //                             conflict-free time in bank and address conflicts);
-//   morpho_bwd_ident_gather_kernel  IDENTITY 3x3 / 5x5: grad_input gathered per input pixel from
-//                             the taps of its window, written once (no fill, no atomics);
-//   morpho_bwd_taps_kernel    other IDENTITY and larger structuring elements: one shared tile per
-//                             channel.
+//   morpho_bwd_ident_gather_kernel  IDENTITY 3x3 / 5x5 in float64: grad_input gathered per input pixel
+//                             from the taps of its window, written once (no fill, no atomics); other
+//                             types and elements: morpho_scatter.hip;
+//   morpho_bwd_taps_kernel    larger structuring elements (and IDENTITY ones the tiles do not take): one
+//                             shared tile per channel.
 //
 // A tap that read outside the image (including REPLICATE's clamped edge pixel) sends nothing to
 // grad_input; grad_weight always receives sign * g (sign -1 for erosion).
@@ -134,23 +136,51 @@ __global__ __launch_bounds__(BLOCK) void morpho_bwd_packed_kernel(const PackedPa
     const int64_t n_begin = (int64_t)chunk * p.chunk;
     const int64_t n_end = min(n_begin + p.chunk, total);
     const T sign = (T)OpTraits<OP, T>::sign;
-    for (int64_t n = n_begin + threadIdx.x; n < n_end; n += BLOCK)
-    {
-        const int64_t b = n / plane;
-        const int64_t pix = n - b * plane;
-        const int h = (int)(pix / g.W), wc = (int)(pix - (int64_t)h * g.W);
-        const int64_t gi = (b * g.Cout + o) * plane + pix;
-        const T gv = (T)p.gout[gi];
-        if (gv == T(0)) continue;
-        const int32_t packed = p.idx[gi];
+    auto add_weight = [&](int32_t packed, T gv) {
         const int c = packed >> 16, k = packed & 0xFFFF;
-        const int kh = k / g.KW, kw = k - kh * g.KW;
-        const int iy = h + ph - kh, ix = wc + pw - kw;
-        if (p.gin && iy >= 0 && iy < g.H && ix >= 0 && ix < g.W) global_add(&p.gin[(b * g.Cin + c) * plane + (int64_t)iy * g.W + ix], (Acc)gv);
         if (p.lds_bins)
             lds_add(&bins[(int64_t)c * K + k], (Acc)(sign * gv));
         else
             global_add(&part[(int64_t)c * K + k], sign * gv);
+    };
+    // The chunk's pixels batch element by batch element: contiguous winners and gradients.
+    for (int64_t b = n_begin / plane; b * plane < n_end; ++b)
+    {
+        const int64_t q0 = (b * g.Cout + o) * plane;
+        const int64_t lo = max(n_begin - b * plane, (int64_t)0), hi = min(n_end - b * plane, plane);
+        if (!p.gin)
+        {
+            // grad_weight alone: four pixels' loads in flight together.
+            constexpr int U = 4;
+            for (int64_t pix = lo + threadIdx.x; pix < hi; pix += U * BLOCK)
+            {
+                int32_t packed[U];
+                T gv[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                {
+                    const int64_t q = q0 + min(pix + u * BLOCK, hi - 1);
+                    packed[u] = p.idx[q];
+                    gv[u] = (T)p.gout[q];
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (pix + u * BLOCK < hi && gv[u] != T(0)) add_weight(packed[u], gv[u]);
+            }
+            continue;
+        }
+        for (int64_t pix = lo + threadIdx.x; pix < hi; pix += BLOCK)
+        {
+            const T gv = (T)p.gout[q0 + pix];
+            if (gv == T(0)) continue;
+            const int32_t packed = p.idx[q0 + pix];
+            const int h = (int)(pix / g.W), wc = (int)(pix - (int64_t)h * g.W);
+            const int c = packed >> 16, k = packed & 0xFFFF;
+            const int kh = k / g.KW, kw = k - kh * g.KW;
+            const int iy = h + ph - kh, ix = wc + pw - kw;
+            if (iy >= 0 && iy < g.H && ix >= 0 && ix < g.W) global_add(&p.gin[(b * g.Cin + c) * plane + (int64_t)iy * g.W + ix], (Acc)gv);
+            add_weight(packed, gv);
+        }
     }
     if (p.lds_bins)
     {
@@ -159,12 +189,12 @@ __global__ __launch_bounds__(BLOCK) void morpho_bwd_packed_kernel(const PackedPa
     }
 }
 
-template <typename T, typename ST = T>
+template <typename T>
 struct TapsParams
 {
     const void* __restrict__ taps;
-    const ST* __restrict__ gout;
-    ST* __restrict__ gin;
+    const T* __restrict__ gout;
+    T* __restrict__ gin;
     T* __restrict__ part;
     Geom g;
     Tiling t;
@@ -523,7 +553,7 @@ __global__ __launch_bounds__(BLOCK) void morpho_bwd_planes_kernel(const TapsPara
     }
 }
 
-// IDENTITY with 3x3 and 5x5 structuring elements, in gather form: output channel c reads
+// IDENTITY with 3x3 and 5x5 structuring elements in float64, in gather form: output channel c reads
 // input channel c only, so the grad_input of pixel q is the sum of g(p) over the window pixels
 // p = q + (kh - KH/2, kw - KW/2) whose saved tap is k = kh * KW + kw, the tap that read q (a tap that
 // read outside the image matches no pixel). One workgroup per (batch element, channel, tile)
@@ -531,14 +561,14 @@ __global__ __launch_bounds__(BLOCK) void morpho_bwd_planes_kernel(const TapsPara
 // each grad_input pixel of the tile once: no zero fill, no atomics on grad_input. grad_weight sums
 // sign * g by saved tap in LDS bins with one copy per lane of a half wave (conflict free), one
 // partial slot per (batch element, tile). IDENTITY has no 1 / Cin scale.
-template <typename T, int OP, int KH, int KW, int RH, typename ST = T>
-__global__ __launch_bounds__(BLOCK) void morpho_bwd_ident_gather_kernel(const TapsParams<T, ST> p)
+template <int OP, int KH, int KW, int RH>
+__global__ __launch_bounds__(BLOCK) void morpho_bwd_ident_gather_kernel(const TapsParams<double> p)
 {
     constexpr int K = KH * KW, PH = KH / 2, PW = KW / 2;
     constexpr int TH = NWAVES * RH, ROWS = TH + KH - 1, COLS = TILE_W + KW - 1, WR = RH + KH - 1;
     constexpr int ELEMS = ROWS * COLS, NS = (ELEMS + BLOCK - 1) / BLOCK;
     constexpr int NC = 32;
-    __shared__ T gs[ELEMS];
+    __shared__ double gs[ELEMS];
     __shared__ int ts[ELEMS];
     __shared__ __align__(16) Acc bins[K * NC];
     const Geom g = p.g;
@@ -570,15 +600,15 @@ __global__ __launch_bounds__(BLOCK) void morpho_bwd_ident_gather_kernel(const Ta
         ok[j] = y >= 0 && y < g.H && x >= 0 && x < g.W;
         off[j] = clampi(y, 0, g.H - 1) * g.W + clampi(x, 0, g.W - 1);
     }
-    T pg[NS];
+    double pg[NS];
     int pt[NS];
     auto load = [&](int c) {
-        const ST* __restrict__ gp = p.gout + ((int64_t)b * g.Cout + c) * plane;
+        const double* __restrict__ gp = p.gout + ((int64_t)b * g.Cout + c) * plane;
         const uint8_t* __restrict__ tp = static_cast<const uint8_t*>(p.taps) + ((int64_t)b * g.Cout + c) * plane;
 #pragma unroll
         for (int j = 0; j < NS; ++j)
         {
-            pg[j] = (T)gp[off[j]];
+            pg[j] = gp[off[j]];
             pt[j] = tp[off[j]];
         }
     };
@@ -593,14 +623,14 @@ __global__ __launch_bounds__(BLOCK) void morpho_bwd_ident_gather_kernel(const Ta
             const int idx = threadIdx.x + j * BLOCK;
             if (j < NS - 1 || idx < ELEMS)
             {
-                gs[idx] = ok[j] ? pg[j] : T(0);
+                gs[idx] = ok[j] ? pg[j] : 0.0;
                 ts[idx] = ok[j] ? pt[j] : -1;
             }
         }
         __syncthreads();
         if (c + 1 < c_end) load(c + 1);  // in flight while this channel computes
 
-        T gw[WR][KW];
+        double gw[WR][KW];
         int tw[WR][KW];
 #pragma unroll
         for (int rr = 0; rr < WR; ++rr)
@@ -610,7 +640,7 @@ __global__ __launch_bounds__(BLOCK) void morpho_bwd_ident_gather_kernel(const Ta
                 gw[rr][kw] = gs[(wave * RH + rr) * COLS + lane + kw];
                 tw[rr][kw] = ts[(wave * RH + rr) * COLS + lane + kw];
             }
-        ST* __restrict__ gplane = p.gin + ((int64_t)b * g.Cin + c) * plane;
+        double* __restrict__ gplane = p.gin + ((int64_t)b * g.Cin + c) * plane;
         Acc* bl = bins + (lane & (NC - 1));
 #pragma unroll
         for (int r = 0; r < RH; ++r)
@@ -622,7 +652,7 @@ __global__ __launch_bounds__(BLOCK) void morpho_bwd_ident_gather_kernel(const Ta
 #pragma unroll
                 for (int kw = 0; kw < KW; ++kw) s += tw[r + kh][kw] == kh * KW + kw ? (Acc)gw[r + kh][kw] : Acc(0);
             const int h = h0 + wave * RH + r;
-            if (h < g.H && wc < g.W) gplane[(int64_t)h * g.W + wc] = (ST)(T)s;
+            if (h < g.H && wc < g.W) gplane[(int64_t)h * g.W + wc] = s;
             // grad_weight: this lane's own output pixel (h, wc), staged at (row r + PH, column PW).
             const int k = tw[r + PH][PW];
             if (k >= 0) lds_add(&bl[k * NC], (Acc)(OP == DILATION ? gw[r + PH][PW] : -gw[r + PH][PW]));
@@ -639,7 +669,7 @@ __global__ __launch_bounds__(BLOCK) void morpho_bwd_ident_gather_kernel(const Ta
 #pragma unroll
             for (int d = 4; d >= 1; d /= 2) v += __shfl_xor(v, d, 8);
             if ((threadIdx.x & 7) == 0)
-                p.part[((int64_t)b * t.ntiles() + tile) * g.Cout * K + (int64_t)c * K + (threadIdx.x >> 3)] = (T)v;
+                p.part[((int64_t)b * t.ntiles() + tile) * g.Cout * K + (int64_t)c * K + (threadIdx.x >> 3)] = v;
         }
         // The next channel's staging overwrites gs / ts, and its adds need the cleared bins.
         __syncthreads();
@@ -656,6 +686,7 @@ struct PackedPlan
     int64_t chunk;
     bool lds_bins;
     bool gather;  // grad_input gathered (small problems)
+    bool tile;    // grad_input by packed_tile_backward (morpho_scatter.hip); neither: global atomics
     int gblocks;  // gathering workgroups
     size_t part_bytes;
     size_t lds;
@@ -674,6 +705,7 @@ static PackedPlan plan_packed(const Geom& g)
     const int64_t gin_n = (int64_t)g.B * g.Cin * g.plane();
     s.gather = gin_n > 0 && gin_n * g.Cout * g.taps() <= PACKED_GATHER_READS;
     s.gblocks = s.gather ? (int)((gin_n + BLOCK / GATHER_SLOTS - 1) / (BLOCK / GATHER_SLOTS)) : 0;
+    s.tile = !s.gather && packed_tiles(g).ok;
     int64_t nchunks = (4096 + g.Cout - 1) / std::max(g.Cout, 1);  // (no output channel: an empty launch)
     const int64_t max_chunks = (total + BLOCK - 1) / BLOCK;
     if (nchunks > max_chunks) nchunks = max_chunks;
@@ -699,6 +731,7 @@ struct TapsPlan
     bool planes;  // morpho_bwd_planes_kernel
     bool gather;  // morpho_bwd_ident_gather_kernel (else morpho_bwd_taps_kernel)
     bool band;    // gathered by ident_band_gather (morpho_ident.hip): slots per (batch element, band)
+    bool tile;    // ident_tile_backward (morpho_scatter.hip): slots per (batch element, tile)
     size_t part_bytes;
     size_t lds;
 };
@@ -717,7 +750,29 @@ static TapsPlan plan_taps(int merge, const Geom& g, bool band_ok = true)
     // that share, one launch's maximum otherwise.
     const size_t target = (160 * 1024) / 3 / 1024 * 1024;
     s.part_bytes = (size_t)g.B * s.t.ntiles() * g.Cout * g.Cw * K * sizeof(T);
-    if (ident && g.KH == g.KW && (g.KH == 3 || g.KH == 5))
+    // IDENTITY by tiles in LDS; float64 3x3 / 5x5 by the gathers, in tap order.
+    const bool gathered = ident && sizeof(T) == 8 && g.KH == g.KW && (g.KH == 3 || g.KH == 5);
+    if (ident && !gathered)
+    {
+        const IdentTiles tiles = ident_tiles(g);
+        if (tiles.ok)
+        {
+            s.t = make_tiling(g, 1);
+            s.t.th = tiles.th;
+            s.t.ntx = tiles.ntx;
+            s.t.nty = tiles.nty;
+            s.gather = true;
+            s.tile = true;
+            s.ig = 1;
+            s.nig = g.Cin;
+            s.oc = 1;
+            s.ncopy = 1 << tiles.ncopy_log2;
+            s.part_bytes = (size_t)g.B * s.t.ntiles() * g.Cout * g.Cw * K * sizeof(T);
+            s.lds = tiles.lds;
+            return s;
+        }
+    }
+    if (gathered)
     {
         const IdentBands bands = band_ok ? ident_bands(g, sizeof(T), true) : IdentBands{0, 0, 0};
         if (bands.R > 0)
@@ -738,8 +793,6 @@ static TapsPlan plan_taps(int merge, const Geom& g, bool band_ok = true)
             s.lds = bands.lds;
             return s;
         }
-        // 4 rows per wave for every dtype: 16-row tiles (float32 / 16-bit gathers 18-26% faster than
-        // with 8 rows, measured at configs[3]'s shape).
         s.t = make_tiling(g, GATHER_RH);
         s.part_bytes = (size_t)g.B * s.t.ntiles() * g.Cout * g.Cw * K * sizeof(T);
         // Up to 8 consecutive channels per workgroup, the next channel's loads in flight behind
@@ -879,8 +932,11 @@ size_t morpho_backward_workspace(int merge, bool has_indices, const Geom& g)
         c.B = recompute_batch<T>(merge, g);
         bytes += align_up(indices_bytes(merge, c)) + align_up((size_t)c.B * c.Cout * c.plane() * sizeof(T));
     }
-    if (packed_winners(merge) && sizeof(T) != sizeof(Acc) && !plan_packed<T>(g).gather)
-        bytes += align_up((size_t)g.B * g.Cin * g.plane() * sizeof(Acc));
+    if (packed_winners(merge) && sizeof(T) != sizeof(Acc))
+    {
+        const PackedPlan s = plan_packed<T>(g);
+        if (!s.gather && !s.tile) bytes += align_up((size_t)g.B * g.Cin * g.plane() * sizeof(Acc));
+    }
     return bytes;
 }
 
@@ -894,10 +950,11 @@ static hipError_t backward_op(int merge, bool replicate, T fill, const T* x, con
     const bool nonempty = (int64_t)g.B * g.Cout * g.plane() > 0;
     // Recomputed taps live in the workspace (256-byte aligned).
     const bool band_ok = band_aligned(grad_out, grad_in, indices);
-    // The gather kernels write every grad_input pixel themselves; the others accumulate onto zeros.
-    const bool gather = nonempty && (packed ? plan_packed<T>(g).gather : plan_taps<T>(merge, g, band_ok).gather);
+    // The gather and tile kernels write every grad_input pixel themselves; the others accumulate onto zeros.
+    const PackedPlan pp = plan_packed<T>(g);
+    const bool gather = nonempty && (packed ? pp.gather || pp.tile : plan_taps<T>(merge, g, band_ok).gather);
     const int64_t gin_n = (int64_t)g.B * g.Cin * g.plane();
-    // float32 max / min round their double grad_input accumulator into every pixel at the end.
+    // float32 max / min scatters round their double grad_input accumulator into every pixel at the end.
     const bool rounded = packed && sizeof(T) != sizeof(Acc) && nonempty;
     if (!gather && !rounded)
         if ((err = fill_async<T>(grad_in, gin_n, T(0), stream)) != hipSuccess) return err;
@@ -922,15 +979,16 @@ static hipError_t backward_op(int merge, bool replicate, T fill, const T* x, con
 
     if (packed)
     {
-        const PackedPlan s = plan_packed<T>(g);
+        const PackedPlan& s = pp;
         if (!s.lds_bins)
             if ((err = fill_async<T>(part, (int64_t)s.nchunks * wnumel, T(0), stream)) != hipSuccess) return err;
         // float32: grad_input summed in a double buffer of the workspace, rounded once at the end
-        // (gathered: written directly).
-        Acc* gin_acc = s.gather ? nullptr : reinterpret_cast<Acc*>(grad_in);
+        // (gathered or summed by tiles: written directly).
+        const bool scatter = !s.gather && !s.tile;
+        Acc* gin_acc = scatter ? reinterpret_cast<Acc*>(grad_in) : nullptr;
         if constexpr (sizeof(T) != sizeof(Acc))
         {
-            if (!s.gather)
+            if (scatter)
             {
                 gin_acc = reinterpret_cast<Acc*>(ws);
                 if ((err = fill_async<Acc>(gin_acc, gin_n, Acc(0), stream)) != hipSuccess) return err;
@@ -949,8 +1007,10 @@ static hipError_t backward_op(int merge, bool replicate, T fill, const T* x, con
         p.wblocks = s.nchunks * g.Cout;
         morpho_bwd_packed_kernel<T, OP><<<(unsigned)((int64_t)p.wblocks + s.gblocks), BLOCK, s.lds, stream>>>(p);
         if ((err = hipGetLastError()) != hipSuccess) return err;
+        if (s.tile)
+            if ((err = packed_tile_backward<T, T>(p.idx, grad_out, grad_in, g, stream)) != hipSuccess) return err;
         if constexpr (sizeof(T) != sizeof(Acc))
-            if (!s.gather)
+            if (scatter)
                 if ((err = round_async<T>(gin_acc, grad_in, gin_n, stream)) != hipSuccess) return err;
         return reduce_slots_async<T>(part, nslots, wnumel, grad_w, scratch, stream);
     }
@@ -998,15 +1058,21 @@ static hipError_t backward_op(int merge, bool replicate, T fill, const T* x, con
         const bool wide = pair_tap_bytes(g) == 2;
         if (s.band)
         {
-            if ((err = ident_band_backward<T, T>(OP, static_cast<const uint8_t*>(taps), p.gout, p.gin, p.part, gc, stream)) != hipSuccess)
-                return err;
+            if constexpr (sizeof(T) == 8)
+                if ((err = ident_band_backward(OP, static_cast<const uint8_t*>(taps), p.gout, p.gin, p.part, gc, stream)) != hipSuccess) return err;
+        }
+        else if (s.tile)
+        {
+            if ((err = ident_tile_backward<T, T>(OP, taps, p.gout, p.gin, p.part, gc, stream)) != hipSuccess) return err;
         }
         else if (s.gather)
         {
-            switch (g.KH)
+            if constexpr (sizeof(T) == 8)
             {
-                case 3: morpho_bwd_ident_gather_kernel<T, OP, 3, 3, GATHER_RH><<<blocks, BLOCK, 0, stream>>>(p); break;
-                default: morpho_bwd_ident_gather_kernel<T, OP, 5, 5, GATHER_RH><<<blocks, BLOCK, 0, stream>>>(p); break;
+                if (g.KH == 3)
+                    morpho_bwd_ident_gather_kernel<OP, 3, 3, GATHER_RH><<<blocks, BLOCK, 0, stream>>>(p);
+                else
+                    morpho_bwd_ident_gather_kernel<OP, 5, 5, GATHER_RH><<<blocks, BLOCK, 0, stream>>>(p);
             }
         }
         else if (s.planes)
@@ -1078,18 +1144,16 @@ size_t half_backward_workspace(int merge, bool has_indices, const Geom& g)
 }
 
 // The kernels that read grad_output once per output pixel and write grad_input once per input pixel
-// take the 16-bit data directly: the max / min scatter (double accumulator rounded into grad_input)
-// and the IDENTITY gather. grad_weight is summed in float32 partial slots and rounded at the end.
+// take the 16-bit data directly: the max / min scatter and the IDENTITY tiles. grad_weight is summed in float32 partial slots and rounded at the end.
 template <typename ST, int OP>
 static hipError_t half_direct(int merge, const void* indices, const ST* grad_out, ST* grad_in, ST* grad_w, const Geom& g, unsigned char* ws,
                               float* gw, hipStream_t stream)
 {
     hipError_t err;
     const int64_t wnumel = (int64_t)g.Cout * g.Cw * g.taps();
-    const bool band_ok = band_aligned(grad_out, grad_in, indices);
     size_t part_bytes;
     int nslots;
-    partials<float>(merge, g, part_bytes, nslots, band_ok);
+    partials<float>(merge, g, part_bytes, nslots);
     float* part = reinterpret_cast<float*>(ws);
     ws += align_up(part_bytes);
     float* scratch = reinterpret_cast<float*>(ws);
@@ -1100,8 +1164,9 @@ static hipError_t half_direct(int merge, const void* indices, const ST* grad_out
         const int64_t gin_n = (int64_t)g.B * g.Cin * g.plane();
         if (!s.lds_bins)
             if ((err = fill_async<float>(part, (int64_t)s.nchunks * wnumel, 0.0f, stream)) != hipSuccess) return err;
-        Acc* gin_acc = s.gather ? nullptr : reinterpret_cast<Acc*>(ws);
-        if (!s.gather)
+        const bool scatter = !s.gather && !s.tile;
+        Acc* gin_acc = scatter ? reinterpret_cast<Acc*>(ws) : nullptr;
+        if (scatter)
             if ((err = fill_async<Acc>(gin_acc, gin_n, Acc(0), stream)) != hipSuccess) return err;
         PackedParams<float, ST> p{};
         p.idx = static_cast<const int32_t*>(indices);
@@ -1116,35 +1181,14 @@ static hipError_t half_direct(int merge, const void* indices, const ST* grad_out
         p.wblocks = s.nchunks * g.Cout;
         morpho_bwd_packed_kernel<float, OP, ST><<<(unsigned)((int64_t)p.wblocks + s.gblocks), BLOCK, s.lds, stream>>>(p);
         if ((err = hipGetLastError()) != hipSuccess) return err;
-        if (!s.gather)
+        if (s.tile)
+            if ((err = packed_tile_backward<float, ST>(p.idx, grad_out, grad_in, g, stream)) != hipSuccess) return err;
+        if (scatter)
             if ((err = round_async<ST>(gin_acc, grad_in, gin_n, stream)) != hipSuccess) return err;
     }
     else
     {
-        const TapsPlan s = plan_taps<float>(merge, g, band_ok);
-        if (s.band)
-        {
-            if ((err = ident_band_backward<float, ST>(OP, static_cast<const uint8_t*>(indices), grad_out, grad_in, part, g, stream)) !=
-                hipSuccess)
-                return err;
-            if ((err = reduce_slots_async<float>(part, nslots, wnumel, gw, scratch, stream)) != hipSuccess) return err;
-            return convert_async<float, ST>(gw, grad_w, wnumel, stream);
-        }
-        TapsParams<float, ST> p{};
-        p.taps = indices;
-        p.gout = grad_out;
-        p.gin = grad_in;
-        p.part = part;
-        p.g = g;
-        p.t = s.t;
-        p.ig = s.ig;
-        p.nig = s.nig;
-        const unsigned blocks = (unsigned)((int64_t)g.B * s.t.ntiles() * s.nig);
-        if (g.KH == 3)
-            morpho_bwd_ident_gather_kernel<float, OP, 3, 3, GATHER_RH, ST><<<blocks, BLOCK, 0, stream>>>(p);
-        else
-            morpho_bwd_ident_gather_kernel<float, OP, 5, 5, GATHER_RH, ST><<<blocks, BLOCK, 0, stream>>>(p);
-        if ((err = hipGetLastError()) != hipSuccess) return err;
+        if ((err = ident_tile_backward<float, ST>(OP, indices, grad_out, grad_in, part, g, stream)) != hipSuccess) return err;
     }
     if ((err = reduce_slots_async<float>(part, nslots, wnumel, gw, scratch, stream)) != hipSuccess) return err;
     return convert_async<float, ST>(gw, grad_w, wnumel, stream);
@@ -1178,7 +1222,7 @@ hipError_t half_backward(int op, int merge, bool replicate, float fill, const ST
         if ((err = fill_async<ST>(grad_in, gin_n, ST(0), stream)) != hipSuccess) return err;
         return fill_async<ST>(grad_w, wnumel, ST(0), stream);
     }
-    if (packed_winners(merge) || plan_taps<float>(merge, g).gather)
+    if (packed_winners(merge) || plan_taps<float>(merge, g).tile)
         return op == DILATION ? half_direct<ST, DILATION>(merge, indices, grad_out, grad_in, grad_w, g, ws, gw, stream)
                               : half_direct<ST, EROSION>(merge, indices, grad_out, grad_in, grad_w, g, ws, gw, stream);
     if ((err = convert_async<ST, float>(grad_out, gout, gout_n, stream)) != hipSuccess) return err;
