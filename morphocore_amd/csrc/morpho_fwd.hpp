@@ -101,12 +101,68 @@ __device__ __forceinline__ void merge_pair(T bv, int i, T& acc, int& win)
     }
 }
 
+// The first tap of channel pair (o, c) at output pixel (h, wc) equal to `target` and its value, read from
+// global memory one row of the element at a time: a row's loads are all in flight together, so that the
+// rescan waits at most once a row (all of a 3x3 element's rows at once). Tap 0, and `target`, when no
+// tap is equal.
+template <typename ST, int OP, int KH, int KW>
+__device__ __forceinline__ void rescan_static(const ST* __restrict__ xp, const ST* __restrict__ wp, const Geom& g, int h, int wc, bool replicate,
+                                              compute_t<ST> fill, compute_t<ST> target, int& karg, compute_t<ST>& value)
+{
+    using T = compute_t<ST>;
+    using Tr = OpTraits<OP, T>;
+    constexpr int ROWS = KH * KW <= 9 ? KH : 1;  // rows in flight together
+    int cx[KW];
+    unsigned outc = 0;
+#pragma unroll
+    for (int kw = 0; kw < KW; ++kw)
+    {
+        const int x = wc + KW / 2 - kw;
+        cx[kw] = clampi(x, 0, g.W - 1);
+        if (x != cx[kw]) outc |= 1u << kw;
+    }
+    if (replicate) outc = 0;
+    int found = -1;
+    T fval = target;
+    for (int kh0 = 0; kh0 < KH && found < 0; kh0 += ROWS)
+    {
+        ST xv[ROWS][KW], wv[ROWS][KW];
+        bool outr[ROWS];
+#pragma unroll
+        for (int q = 0; q < ROWS; ++q)
+        {
+            const int y = h + KH / 2 - (kh0 + q), yc = clampi(y, 0, g.H - 1);
+            outr[q] = y != yc && !replicate;
+            const ST* __restrict__ row = xp + (int64_t)yc * g.W;
+#pragma unroll
+            for (int kw = 0; kw < KW; ++kw)
+            {
+                xv[q][kw] = row[cx[kw]];
+                wv[q][kw] = wp[(kh0 + q) * KW + kw];
+            }
+        }
+#pragma unroll
+        for (int q = ROWS - 1; q >= 0; --q)
+#pragma unroll
+            for (int kw = KW - 1; kw >= 0; --kw)
+            {
+                const T v = Tr::combine(outr[q] || ((outc >> kw) & 1) ? fill : (T)xv[q][kw], (T)wv[q][kw]);
+                const bool hit = v == target;
+                found = hit ? (kh0 + q) * KW + kw : found;
+                fval = hit ? v : fval;
+            }
+    }
+    karg = found < 0 ? 0 : found;
+    value = fval;
+}
+
 // Finalises and stores one output pixel; for MAX / MIN / IDENTITY rescans the winning channel when
 // its tap is needed (PACKED) or when the result is zero (sign of the first zero tap). The merged
 // value is the winning channel's extremum, so it is the value to look for, unless it is the merge's
 // clamp (lowest() / max()): then channel 0 won without a strictly better channel after it, and its
 // extremum may lie beyond the clamp (an infinite tap), so that extremum is recomputed and looked for.
-template <typename ST, int OP, int MK, int MODE>
+// KH, KW: the element's size when it is known at compile time (else 0).
+template <typename ST, int OP, int MK, int MODE, int KH = 0, int KW = 0>
 __device__ __forceinline__ void store_output(const FwdParams<ST>& p, int b, int o, int h, int wc, int i_count, compute_t<ST> acc, int win)
 {
     using T = compute_t<ST>;
@@ -143,7 +199,13 @@ __device__ __forceinline__ void store_output(const FwdParams<ST>& p, int b, int 
                         }
                 }
             }
-            if (target != Tr::init())
+            if (KH > 0 && target != Tr::init())
+            {
+                T fval = target;
+                if constexpr (KH > 0) rescan_static<ST, OP, KH, KW>(xp, wp, g, h, wc, p.replicate != 0, p.fill, target, karg, fval);
+                if (v == T(0)) v = fval;
+            }
+            else if (target != Tr::init())
             {
                 // Taps in chunks of 4 whose loads are all in flight together (the rescan is a chain of
                 // dependent global loads otherwise); the first equal tap of the first chunk holding
@@ -338,6 +400,10 @@ struct StaticTile
 // global memory, which costs fewer staging passes than it saves.
 constexpr int BUCKET_MIN_TAPS = 25;
 constexpr int BUCKET_MAX_CIN = 256;
+// A workgroup of one output channel sorts only up to this many input channels: its few items share too
+// little of each staged tile. Bucket against per-pixel rescan (us): 7x7 at (8, 64 -> 3, 256, 256) 422 / 319,
+// at (8, 3 -> 3, 512, 512) 150 / 229; 5x5 at (4, 8 -> 8, 128, 128) 23.2 / 23.4.
+constexpr int BUCKET_MAX_CIN_ONE = 8;
 
 // Structuring-element values of the workgroup's OB output channels for one input channel, staged
 // with the input tile and read by every lane at the same LDS address (a broadcast).
@@ -383,22 +449,23 @@ morpho_fwd_static(const FwdParams<ST> p)
     const ST* __restrict__ wb = p.w + (int64_t)b * g.wbs;
     const int wc = w0 + lane;
 
-    // Staging plan, the same for every input channel: plane offset of each element this thread
-    // stages (-1: the fill value).
+    // Staging plan, the same for every input channel: the clamped in-image offset of each element this
+    // thread stages (loaded unconditionally) and whether the fill value replaces it (bit j). The values
+    // stay in their storage type until they are staged: a conversion, or a load under a condition, next
+    // to the load waits for it there, one memory latency per element instead of one per channel
+    // (bfloat16 3x3 min at (16, 64 -> 64, 57, 57): 212 -> 168 us with the 3x3 fold and rescan below).
     int off[NS];
+    unsigned fills = 0;
 #pragma unroll
     for (int j = 0; j < NS; ++j)
     {
         const int idx = threadIdx.x + j * BLOCK;
         const int ly = idx / COLS, lx = idx - ly * COLS;
         const int y = y0 + ly, x = x0 + lx;
-        if (y >= 0 && y < g.H && x >= 0 && x < g.W)
-            off[j] = y * g.W + x;
-        else if (p.replicate)
-            off[j] = clampi(y, 0, g.H - 1) * g.W + clampi(x, 0, g.W - 1);
-        else
-            off[j] = -1;
+        off[j] = clampi(y, 0, g.H - 1) * g.W + clampi(x, 0, g.W - 1);
+        if (!p.replicate && !(y >= 0 && y < g.H && x >= 0 && x < g.W)) fills |= 1u << j;
     }
+    static_assert(NS <= 32, "one bit per staged element");
     // Structuring-element rows this thread stages: output channel o0 + ob, tap k (clamped to a
     // valid channel past Cout; those values are never used).
     int woff[NW];
@@ -410,27 +477,27 @@ morpho_fwd_static(const FwdParams<ST> p)
         woff[j] = ident ? k : (min(o0 + ob, g.Cout - 1) * g.Cw) * K + k;
     }
     const ST* __restrict__ xb = p.x + (int64_t)b * g.Cin * plane;
-    T pre[NS], wpre[NW];
+    ST pre[NS], wpre[NW];
     auto load = [&](int i) {
         const ST* __restrict__ pl = xb + (int64_t)i * plane;
 #pragma unroll
-        for (int j = 0; j < NS; ++j) pre[j] = off[j] >= 0 ? (T)pl[off[j]] : p.fill;
+        for (int j = 0; j < NS; ++j) pre[j] = pl[off[j]];
         const ST* __restrict__ wi = wb + (int64_t)i * K;  // IDENTITY: channel i's own element
 #pragma unroll
-        for (int j = 0; j < NW; ++j) wpre[j] = (T)wi[woff[j]];
+        for (int j = 0; j < NW; ++j) wpre[j] = wi[woff[j]];
     };
     auto store = [&](int buf) {
 #pragma unroll
         for (int j = 0; j < NS; ++j)
         {
             const int idx = threadIdx.x + j * BLOCK;
-            if (j < NS - 1 || idx < S::ELEMS) tiles[buf][idx] = pre[j];
+            if (j < NS - 1 || idx < S::ELEMS) tiles[buf][idx] = (fills >> j) & 1 ? p.fill : (T)pre[j];
         }
 #pragma unroll
         for (int j = 0; j < NW; ++j)
         {
             const int idx = threadIdx.x + j * BLOCK;
-            if (idx < SW::ELEMS) wts[buf][idx] = wpre[j];
+            if (idx < SW::ELEMS) wts[buf][idx] = (T)wpre[j];
         }
     };
 
@@ -567,12 +634,18 @@ morpho_fwd_static(const FwdParams<ST> p)
         else
         {
             // Values only: the order of the taps does not matter, so one column of the window is
-            // live at a time (kw outer) and pairs of taps fold into one max3 / min3.
-            T best[OB][RH];
+            // live at a time (kw outer) and pairs of taps fold into one max3 / min3; a column's odd tap
+            // waits for the next column's (3x3: 5 slow operations per window instead of 6; larger
+            // elements lose a wave per SIMD to the waiting values).
+            constexpr bool CARRY = K == 9;
+            T best[OB][RH], odd[OB][RH];
+            // The start value in a register: max3 / min3 take no infinity as a literal.
+            T start = Tr::init();
+            if constexpr (CARRY) asm volatile("" : "+v"(start));
 #pragma unroll
             for (int ob = 0; ob < OB; ++ob)
 #pragma unroll
-                for (int r = 0; r < RH; ++r) best[ob][r] = Tr::init();
+                for (int r = 0; r < RH; ++r) best[ob][r] = start;
 #pragma unroll
             for (int kw = 0; kw < KW; ++kw)
             {
@@ -595,7 +668,16 @@ morpho_fwd_static(const FwdParams<ST> p)
                         for (int kh = 0; kh + 1 < KH; kh += 2)
                             m = Tr::pick(m, Tr::pick(Tr::combine(col[r + KH - 1 - kh], wp[kh * KW + kw]),
                                                      Tr::combine(col[r + KH - 2 - kh], wp[(kh + 1) * KW + kw])));
-                        if constexpr (KH % 2 == 1) m = Tr::pick(m, Tr::combine(col[r], wp[(KH - 1) * KW + kw]));
+                        if constexpr (KH % 2 == 1)
+                        {
+                            const T v = Tr::combine(col[r], wp[(KH - 1) * KW + kw]);
+                            if (!CARRY || kw == KW - 1)
+                                m = Tr::pick(m, v);
+                            else if (kw % 2 == 0)
+                                odd[ob][r] = v;
+                            else
+                                m = Tr::pick(m, Tr::pick(odd[ob][r], v));
+                        }
                         best[ob][r] = m;
                     }
                 }
@@ -618,7 +700,7 @@ morpho_fwd_static(const FwdParams<ST> p)
             for (int r = 0; r < RH; ++r)
             {
                 const int h = h0 + wave * RH + r;
-                if (h < g.H && wc < g.W) store_output<ST, OP, MK, MODE>(p, b, i, h, wc, 1, acc[0][r], win[0][r]);
+                if (h < g.H && wc < g.W) store_output<ST, OP, MK, MODE, KH, KW>(p, b, i, h, wc, 1, acc[0][r], win[0][r]);
             }
         }
         if (more) store(buf ^ 1);
@@ -627,7 +709,7 @@ morpho_fwd_static(const FwdParams<ST> p)
 
     if constexpr (BUCKET)
     {
-        if (g.Cin >= 1 && g.Cin <= BUCKET_MAX_CIN)
+        if (g.Cin >= 1 && g.Cin <= (OB > 1 ? BUCKET_MAX_CIN : BUCKET_MAX_CIN_ONE))
         {
             // The winning tap of every output pixel, found channel by channel from LDS instead of one
             // lane at a time from global memory (whose scattered loads, one plane per lane, bound the
@@ -788,7 +870,7 @@ morpho_fwd_static(const FwdParams<ST> p)
             {
                 const int o = o0 + ob, h = h0 + wave * RH + r;
                 if (o >= g.Cout || h >= g.H || wc >= g.W) continue;
-                store_output<ST, OP, MK, MODE>(p, b, o, h, wc, i_end - i_begin, acc[ob][r], win[ob][r]);
+                store_output<ST, OP, MK, MODE, KH, KW>(p, b, o, h, wc, i_end - i_begin, acc[ob][r], win[ob][r]);
             }
     }
 }
@@ -804,7 +886,7 @@ static bool has_static(const Geom& g)
     using T = compute_t<ST>;
     if (g.KH != g.KW) return false;
     if constexpr (sizeof(T) == 8) return g.KH == 3;
-    return g.KH == 3 || g.KH == 5 || g.KH == 7 || g.KH == 11;
+    return g.KH == 3 || g.KH == 5 || g.KH == 7 || g.KH == 9 || g.KH == 11;
 }
 
 // Rows per wave of the static kernel: 4 for every size and mode. Fewer registers and more waves beat
@@ -840,10 +922,16 @@ static hipError_t launch_generic(FwdParams<ST> p, hipStream_t stream)
     return hipGetLastError();
 }
 
-// Below this many workgroups the chip is mostly idle and every workgroup's serial latency (its channel
-// loop, the winner rescans of its pixels) is the kernel time: such launches take one row per wave and
-// one output channel per workgroup instead, for up to RH * OB times more workgroups.
+// Below this many workgroups of the full shape (RH rows per wave, OB output channels) the chip is mostly
+// idle and every workgroup's serial latency (its channel loop, the winner rescans of its pixels) is the
+// kernel time: such launches take one output channel per workgroup and 4, 2 or 1 rows per wave, the
+// most that leaves MEDIUM_GRID (4 rows) or TWO_ROW_GRID (2) workgroups. More rows per wave share each LDS
+// read of the window and of the element; fewer make more workgroups. Measured (us), values only:
+// 7x7 at (4, 8 -> 8, 128, 128): 4 rows (512 workgroups) 18.8, 2 (1024) 20.6, 1 (2048) 30.4; 5x5 at
+// (2, 32 -> 32, 64, 64): 4 (256) 34.4, 2 (512) 27.2, 1 (1024) 35.9; (1, 16 -> 16, 64, 64): 4 (64) 17.8,
+// 2 (128) 12.9, 1 (256) 10.6; 11x11 at (1, 51 -> 51, 32, 28): 4 (102) 193, 2 (204) 117, 1 (408) 119.
 constexpr int64_t SMALL_GRID = 1024;
+constexpr int64_t MEDIUM_GRID = 448, TWO_ROW_GRID = 192;
 constexpr int IDENT_CHANS = 8;
 
 template <typename ST, int OP, int MK, int OB, int MODE, int KS>
@@ -863,11 +951,21 @@ static hipError_t launch_static(FwdParams<ST> p, hipStream_t stream)
     {
         if (blocks < SMALL_GRID)
         {
-            p.t = make_tiling(p.g, 1);
             p.nog = p.g.Cout;
             p.chans = 1;
-            blocks = (int64_t)p.g.B * p.t.nty * p.t.ntx * p.nog;
-            morpho_fwd_static<ST, OP, MK, KS, KS, 1, 1, MODE><<<(unsigned)blocks, BLOCK, 0, stream>>>(p);
+            auto with_rows = [&](int rh) {
+                p.t = make_tiling(p.g, rh);
+                return blocks = (int64_t)p.g.B * p.t.nty * p.t.ntx * p.nog;
+            };
+            if (with_rows(RH) >= MEDIUM_GRID)
+                morpho_fwd_static<ST, OP, MK, KS, KS, 1, RH, MODE><<<(unsigned)blocks, BLOCK, 0, stream>>>(p);
+            else if (with_rows(2) >= TWO_ROW_GRID)
+                morpho_fwd_static<ST, OP, MK, KS, KS, 1, 2, MODE><<<(unsigned)blocks, BLOCK, 0, stream>>>(p);
+            else
+            {
+                with_rows(1);
+                morpho_fwd_static<ST, OP, MK, KS, KS, 1, 1, MODE><<<(unsigned)blocks, BLOCK, 0, stream>>>(p);
+            }
             return hipGetLastError();
         }
     }
@@ -891,6 +989,7 @@ static hipError_t launch_fwd(const FwdParams<ST>& p, hipStream_t stream)
                 case 3: return launch_static<ST, OP, MK, OB, MODE, 3>(p, stream);
                 case 5: return launch_static<ST, OP, MK, OB, MODE, 5>(p, stream);
                 case 7: return launch_static<ST, OP, MK, OB, MODE, 7>(p, stream);
+                case 9: return launch_static<ST, OP, MK, OB, MODE, 9>(p, stream);
                 default: return launch_static<ST, OP, MK, OB, MODE, 11>(p, stream);
             }
         }
