@@ -40,51 +40,75 @@ __device__ __forceinline__ bool tap_in_image(int iy, int ix, int kh, int kw, con
 
 // ref, S and W of one pair for the RH pixels of this lane (rows iy0 + r, column ix in input
 // coordinates of the first tap), from the staged tile.
-template <typename T, int RH>
+// KWS: the element's row length when it is known at compile time (else 0): a row's taps are then unrolled,
+// whose exponentials are independent chains of some twenty dependent operations each (one tap at a time
+// a wave waits on every step of its own chain, and small problems have one or two waves per SIMD). EDGE: some
+// tap of the tile may read outside the image (else every tap is taken without a test).
+template <typename T, int RH, int KWS, bool EDGE>
 __device__ __forceinline__ void smorph_pair_stats(const T* tbase, int pitch, const T* __restrict__ wp, T a, const Geom& g, int iy0, int ix,
                                                   T (&ref)[RH], T (&S)[RH], T (&Wsum)[RH])
 {
 #pragma clang fp contract(off)  // S = S + e and W fused as the reference rounds them (written as fma)
     const bool dilation_like = a >= T(0);
     const T lo = ExpConsts<T>::min_input;
+    const int KW = KWS > 0 ? KWS : g.KW;
+    auto refs = [&](int kh, int kw) {
+        const T wk = wp[kh * KW + kw];
 #pragma unroll
-    for (int r = 0; r < RH; ++r) ref[r] = dilation_like ? -std::numeric_limits<T>::infinity() : std::numeric_limits<T>::infinity();
-    for (int kh = 0; kh < g.KH; ++kh)
-        for (int kw = 0; kw < g.KW; ++kw)
+        for (int r = 0; r < RH; ++r)
         {
-            const T wk = wp[kh * g.KW + kw];
+            const T v = tbase[(r - kh) * pitch - kw] + wk;
+            // Strict replacement: a NaN never wins, as in the reference.
+            const bool better = dilation_like ? v > ref[r] : v < ref[r];
+            if (better && (!EDGE || tap_in_image(iy0 + r, ix, kh, kw, g))) ref[r] = v;
+        }
+    };
+    auto sums = [&](int kh, int kw) {
+        const T wk = wp[kh * KW + kw];
 #pragma unroll
-            for (int r = 0; r < RH; ++r)
+        for (int r = 0; r < RH; ++r)
+        {
+            const T v = tbase[(r - kh) * pitch - kw] + wk;
+            const bool valid = !EDGE || tap_in_image(iy0 + r, ix, kh, kw, g);
+            const T e = valid ? exp_ref((v - ref[r]) * a, lo) : T(0);
+            S[r] = S[r] + e;
+            Wsum[r] = fma(e, valid ? v : T(0), Wsum[r]);
+        }
+    };
+    auto each_tap = [&](auto&& f) {
+        for (int kh = 0; kh < g.KH; ++kh)
+        {
+            if constexpr (KWS > 0)
             {
-                const T v = tbase[(r - kh) * pitch - kw] + wk;
-                // Strict replacement: a NaN never wins, as in the reference.
-                const bool better = dilation_like ? v > ref[r] : v < ref[r];
-                if (better && tap_in_image(iy0 + r, ix, kh, kw, g)) ref[r] = v;
+#pragma unroll
+                for (int kw = 0; kw < KWS; ++kw) f(kh, kw);
+            }
+            else
+            {
+                for (int kw = 0; kw < g.KW; ++kw) f(kh, kw);
             }
         }
+    };
+#pragma unroll
+    for (int r = 0; r < RH; ++r) ref[r] = dilation_like ? -std::numeric_limits<T>::infinity() : std::numeric_limits<T>::infinity();
+    each_tap(refs);
 #pragma unroll
     for (int r = 0; r < RH; ++r)
     {
         S[r] = T(0);
         Wsum[r] = T(0);
     }
-    for (int kh = 0; kh < g.KH; ++kh)
-        for (int kw = 0; kw < g.KW; ++kw)
-        {
-            const T wk = wp[kh * g.KW + kw];
-#pragma unroll
-            for (int r = 0; r < RH; ++r)
-            {
-                const T v = tbase[(r - kh) * pitch - kw] + wk;
-                const bool valid = tap_in_image(iy0 + r, ix, kh, kw, g);
-                const T e = valid ? exp_ref((v - ref[r]) * a, lo) : T(0);
-                S[r] = S[r] + e;
-                Wsum[r] = fma(e, valid ? v : T(0), Wsum[r]);
-            }
-        }
+    each_tap(sums);
 }
 
-template <typename T, int MK, int RH, bool STATS>
+// Whether every tap of every pixel of a tile staged from row y0 and column x0 reads the image (the same for
+// the whole workgroup).
+__device__ __forceinline__ bool tile_inside(const Geom& g, const Tiling& t, int y0, int x0)
+{
+    return y0 >= 0 && x0 >= 0 && y0 + t.rows <= g.H && x0 + t.cols <= g.W;
+}
+
+template <typename T, int MK, int RH, bool STATS, int KWS>
 __global__ __launch_bounds__(BLOCK) void smorph_fwd_kernel(const SmorphFwdParams<T> p)
 {
 #pragma clang fp contract(off)  // fused only where the reference fuses (written as fma)
@@ -124,6 +148,7 @@ __global__ __launch_bounds__(BLOCK) void smorph_fwd_kernel(const SmorphFwdParams
 
     const int i_begin = MK == MK_IDENT ? o : 0;
     const int i_end = MK == MK_IDENT ? o + 1 : g.Cin;
+    const bool inside = tile_inside(g, t, y0, x0);
     const T* tbase = tile + (wave * RH + g.KH - 1) * t.pitch + lane + g.KW - 1;
     for (int i = i_begin; i < i_end; ++i)
     {
@@ -134,7 +159,10 @@ __global__ __launch_bounds__(BLOCK) void smorph_fwd_kernel(const SmorphFwdParams
         const T a = p.alpha[pair];
         const T* __restrict__ wp = p.w + ((int64_t)o * g.Cw + (MK == MK_IDENT ? 0 : i)) * K;
         T ref[RH], S[RH], Wsum[RH];
-        smorph_pair_stats<T, RH>(tbase, t.pitch, wp, a, g, iy0, ix, ref, S, Wsum);
+        if (inside)
+            smorph_pair_stats<T, RH, KWS, false>(tbase, t.pitch, wp, a, g, iy0, ix, ref, S, Wsum);
+        else
+            smorph_pair_stats<T, RH, KWS, true>(tbase, t.pitch, wp, a, g, iy0, ix, ref, S, Wsum);
 #pragma unroll
         for (int r = 0; r < RH; ++r)
         {
@@ -188,7 +216,7 @@ __global__ __launch_bounds__(BLOCK) void smorph_fwd_kernel(const SmorphFwdParams
 
 // GGIN: grad_input is summed in global memory (p.gacc, double atomics per routed tap) instead of an LDS
 // copy of the tile flushed per tile: for elements whose tile and its double copy exceed the LDS.
-template <typename T, int MK, int RH, bool GGIN = false>
+template <typename T, int MK, int RH, bool GGIN, int KWS>
 __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams<T> p)
 {
 #pragma clang fp contract(off)  // fused only where the reference fuses (written as fma)
@@ -206,6 +234,8 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
     Acc* bbins = abins + p.ncopy;
     const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
     int work = xcd_work_index(blockIdx.x, gridDim.x);
+    const int oslice = work % p.oslices;  // the workgroups of a strip share its tiles in L2
+    work /= p.oslices;
     const int strip = work % p.nstrips;
     work /= p.nstrips;
     const int i = work % g.Cin;
@@ -237,8 +267,9 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
         __syncthreads();
         Acc* __restrict__ gacc_plane = GGIN ? p.gacc + ((int64_t)b * g.Cin + i) * plane : nullptr;
 
-        const int o_begin = MK == MK_IDENT ? i : 0;
-        const int o_end = MK == MK_IDENT ? i + 1 : g.Cout;
+        const int o_begin = MK == MK_IDENT ? i : oslice * p.oper;
+        const int o_end = MK == MK_IDENT ? i + 1 : min(o_begin + p.oper, g.Cout);
+        const bool inside = tile_inside(g, t, y0, x0);
         for (int o = o_begin; o < o_end; ++o)
         {
             const int wi = MK == MK_IDENT ? 0 : i;
@@ -248,7 +279,10 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
             T ref[RH], S[RH], Wsum[RH], outp[RH], scaled[RH], asum[RH];
             bool in[RH];
             T bsum = T(0);
-            smorph_pair_stats<T, RH>(tbase, t.pitch, wp, a, g, iy0, ix, ref, S, Wsum);
+            if (inside)
+                smorph_pair_stats<T, RH, KWS, false>(tbase, t.pitch, wp, a, g, iy0, ix, ref, S, Wsum);
+            else
+                smorph_pair_stats<T, RH, KWS, true>(tbase, t.pitch, wp, a, g, iy0, ix, ref, S, Wsum);
 #pragma unroll
             for (int r = 0; r < RH; ++r)
             {
@@ -283,38 +317,53 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
                 scaled[r] = gv * inv;
                 asum[r] = T(0);
             }
-            for (int kh = 0; kh < g.KH; ++kh)
-                for (int kw = 0; kw < g.KW; ++kw)
-                {
-                    const int k = kh * g.KW + kw;
-                    const T wk = wp[k];
+            const int KW = KWS > 0 ? KWS : g.KW;
+            auto route = [&](int kh, int kw) {
+                const int k = kh * KW + kw;
+                const T wk = wp[k];
 #pragma unroll
-                    for (int r = 0; r < RH; ++r)
+                for (int r = 0; r < RH; ++r)
+                {
+                    // Every in-image tap of an in-image pixel routes, also with a zero gradient
+                    // (so that a NaN of the pair reaches the gradients, as in the reference).
+                    const bool routes = in[r] && (inside || tap_in_image(iy0 + r, ix, kh, kw, g));
+                    const T v = tbase[(r - kh) * t.pitch - kw] + wk;
+                    // The routing's exponential: the hardware one in float32 (the sums above,
+                    // and so the output, use the reference's).
+                    T e;
+                    if constexpr (sizeof(T) == 4)
+                        e = exp_route((v - ref[r]) * a);
+                    else
+                        e = exp_ref((v - ref[r]) * a, lo);
+                    const T pg = e * scaled[r];
+                    const T centered = v - outp[r];
+                    // c = pg (1 + a centered) and the alpha term pg (v - ref) centered share pg centered.
+                    const T q = pg * centered;
+                    const T c = fma(a, q, pg);
+                    const T as = fma(q, v - ref[r], asum[r]);
+                    asum[r] = routes ? as : asum[r];
+                    if (routes)
                     {
-                        // Every in-image tap of an in-image pixel routes, also with a zero gradient
-                        // (so that a NaN of the pair reaches the gradients, as in the reference).
-                        if (!in[r] || !tap_in_image(iy0 + r, ix, kh, kw, g)) continue;
-                        const T v = tbase[(r - kh) * t.pitch - kw] + wk;
-                        // The routing's exponential: the hardware one in float32 (the sums above,
-                        // and so the output, use the reference's).
-                        T e;
-                        if constexpr (sizeof(T) == 4)
-                            e = exp_route((v - ref[r]) * a);
-                        else
-                            e = exp_ref((v - ref[r]) * a, lo);
-                        const T pg = e * scaled[r];
-                        const T centered = v - outp[r];
-                        // c = pg (1 + a centered) and the alpha term pg (v - ref) centered share pg centered.
-                        const T q = pg * centered;
-                        const T c = fma(a, q, pg);
                         if constexpr (GGIN)
                             global_add(&gacc_plane[(int64_t)(iy0 + r - kh) * g.W + (ix - kw)], (Acc)c);
                         else
                             lds_add(&gtile[(wave * RH + r + g.KH - 1 - kh) * t.pitch + lane + g.KW - 1 - kw], (Acc)c);
                         lds_add(&bins[k * p.ncopy + copy], (Acc)c);
-                        asum[r] = fma(q, v - ref[r], asum[r]);
                     }
                 }
+            };
+            for (int kh = 0; kh < g.KH; ++kh)
+            {
+                if constexpr (KWS > 0)
+                {
+#pragma unroll
+                    for (int kw = 0; kw < KWS; ++kw) route(kh, kw);
+                }
+                else
+                {
+                    for (int kw = 0; kw < g.KW; ++kw) route(kh, kw);
+                }
+            }
             T as = T(0);
 #pragma unroll
             for (int r = 0; r < RH; ++r) as += asum[r];
@@ -453,16 +502,24 @@ struct SmorphBwdPlan
     int tps;
     int ncopy;
     int npairs;
+    int oslices, oper;  // generic kernel: output-channel slices, one workgroup each, and their channels
     bool ggin;  // generic kernel with grad_input summed in global memory (smorph_bwd_kernel<..., true>)
     size_t part_w_bytes, part_a_bytes, part_b_bytes, counts_bytes, gacc_bytes;
     size_t lds;
 };
 
-// Rows per wave of the generic forward: the default while its tile fits the tuned LDS budget, else one
-// (a shorter tile, for large elements).
+// Element widths whose rows the generic kernels unroll (any height): they run one row per wave, whose taps
+// hide each other's latency. Other widths take the default rows per wave, one after the other. Float64
+// 5x5 at (2, 8 -> 8, 64, 60): forward 168 -> 60 us, backward 288 -> 61 (with the output-channel slices);
+// its training step 528 -> 133 (with smorph_element).
+static bool smorph_unrolled(const Geom& g) { return g.KW <= 11 && g.KW >= 3 && g.KW % 2 == 1; }
+
+// Rows per wave of the generic forward: one where the element's rows are unrolled, else the default while its
+// tile fits the tuned LDS budget, else one (a shorter tile, for large elements).
 template <typename T>
 static int smorph_fwd_rh(const Geom& g)
 {
+    if (smorph_unrolled(g)) return 1;
     const Tiling t = make_tiling(g, rows_per_wave<T>());
     return (size_t)t.rows * t.pitch * sizeof(T) <= LDS_LIMIT ? rows_per_wave<T>() : 1;
 }
@@ -494,7 +551,7 @@ static SmorphBwdPlan plan_smorph_bwd(int merge, const Geom& g, bool saved = fals
         {
             const size_t budget = budgets[attempt < 2 ? 0 : 1];
             const bool ggin = attempt == 4;
-            rh = (attempt == 0 || attempt == 2) ? rows_per_wave<T>() : 1;
+            rh = (attempt == 0 || attempt == 2) && !smorph_unrolled(g) ? rows_per_wave<T>() : 1;
             const Tiling t = make_tiling(g, rh);
             const size_t cells = (size_t)t.rows * t.pitch;
             const size_t fixed = align16(cells * sizeof(T)) + (ggin ? 0 : cells * sizeof(Acc));
@@ -517,6 +574,14 @@ static SmorphBwdPlan plan_smorph_bwd(int merge, const Geom& g, bool saved = fals
     while (nstrips > 1 && (size_t)g.B * nstrips * (wnumel + s.npairs) * sizeof(T) > ((size_t)256 << 20)) nstrips = (nstrips + 1) / 2;
     s.tps = std::max(1, (int)((ntiles + nstrips - 1) / nstrips));
     s.nstrips = (int)((ntiles + s.tps - 1) / s.tps);
+    // Problems of few tiles split a strip's output channels over several workgroups (each adds its share
+    // of the strip's grad_input), up to about 1024.
+    s.oslices = 1;
+    if (!stat && merge != MERGE_IDENTITY && g.Cout > 0)
+        s.oslices = (int)std::max<int64_t>(1, std::min<int64_t>(g.Cout, 1024 / (units * s.nstrips)));
+    s.oper = std::max(1, (g.Cout + s.oslices - 1) / s.oslices);
+    s.oslices = std::max(1, (g.Cout + s.oper - 1) / s.oper);
+    if (merge == MERGE_IDENTITY) s.oslices = 1;
     const size_t nslots = (size_t)g.B * s.nstrips;
     s.part_w_bytes = nslots * wnumel * sizeof(T);
     s.part_a_bytes = nslots * s.npairs * sizeof(T);
@@ -568,13 +633,21 @@ template <typename T, int MK>
 static hipError_t launch_smorph_bwd_generic(const SmorphBwdPlan& s, const SmorphBwdParams<T>& p, hipStream_t stream)
 {
     constexpr int RH = rows_per_wave<T>();
-    const unsigned blocks = (unsigned)((int64_t)p.g.B * p.g.Cin * s.nstrips);
+    const unsigned blocks = (unsigned)((int64_t)p.g.B * p.g.Cin * s.nstrips * s.oslices);
     if (s.ggin)
-        smorph_bwd_kernel<T, MK, 1, true><<<blocks, BLOCK, s.lds, stream>>>(p);
+        smorph_bwd_kernel<T, MK, 1, true, 0><<<blocks, BLOCK, s.lds, stream>>>(p);
     else if (s.t.rh == 1)
-        smorph_bwd_kernel<T, MK, 1, false><<<blocks, BLOCK, s.lds, stream>>>(p);
+        switch (smorph_unrolled(p.g) ? p.g.KW : 0)
+        {
+            case 3: smorph_bwd_kernel<T, MK, 1, false, 3><<<blocks, BLOCK, s.lds, stream>>>(p); break;
+            case 5: smorph_bwd_kernel<T, MK, 1, false, 5><<<blocks, BLOCK, s.lds, stream>>>(p); break;
+            case 7: smorph_bwd_kernel<T, MK, 1, false, 7><<<blocks, BLOCK, s.lds, stream>>>(p); break;
+            case 9: smorph_bwd_kernel<T, MK, 1, false, 9><<<blocks, BLOCK, s.lds, stream>>>(p); break;
+            case 11: smorph_bwd_kernel<T, MK, 1, false, 11><<<blocks, BLOCK, s.lds, stream>>>(p); break;
+            default: smorph_bwd_kernel<T, MK, 1, false, 0><<<blocks, BLOCK, s.lds, stream>>>(p); break;
+        }
     else
-        smorph_bwd_kernel<T, MK, RH, false><<<blocks, BLOCK, s.lds, stream>>>(p);
+        smorph_bwd_kernel<T, MK, RH, false, 0><<<blocks, BLOCK, s.lds, stream>>>(p);
     return hipGetLastError();
 }
 
@@ -615,9 +688,17 @@ static hipError_t launch_smorph_fwd(const SmorphFwdParams<T>& p, hipStream_t str
     const int64_t blocks = (int64_t)p.g.B * p.t.nty * p.t.ntx * p.g.Cout;
     const size_t lds = (size_t)p.t.rows * p.t.pitch * sizeof(T);
     if (p.t.rh == 1)
-        smorph_fwd_kernel<T, MK, 1, STATS><<<(unsigned)blocks, BLOCK, lds, stream>>>(p);
+        switch (smorph_unrolled(p.g) ? p.g.KW : 0)
+        {
+            case 3: smorph_fwd_kernel<T, MK, 1, STATS, 3><<<(unsigned)blocks, BLOCK, lds, stream>>>(p); break;
+            case 5: smorph_fwd_kernel<T, MK, 1, STATS, 5><<<(unsigned)blocks, BLOCK, lds, stream>>>(p); break;
+            case 7: smorph_fwd_kernel<T, MK, 1, STATS, 7><<<(unsigned)blocks, BLOCK, lds, stream>>>(p); break;
+            case 9: smorph_fwd_kernel<T, MK, 1, STATS, 9><<<(unsigned)blocks, BLOCK, lds, stream>>>(p); break;
+            case 11: smorph_fwd_kernel<T, MK, 1, STATS, 11><<<(unsigned)blocks, BLOCK, lds, stream>>>(p); break;
+            default: smorph_fwd_kernel<T, MK, 1, STATS, 0><<<(unsigned)blocks, BLOCK, lds, stream>>>(p); break;
+        }
     else
-        smorph_fwd_kernel<T, MK, RH, STATS><<<(unsigned)blocks, BLOCK, lds, stream>>>(p);
+        smorph_fwd_kernel<T, MK, RH, STATS, 0><<<(unsigned)blocks, BLOCK, lds, stream>>>(p);
     return hipGetLastError();
 }
 
@@ -728,6 +809,8 @@ hipError_t smorph_backward(int merge, const T* x, const T* w, const T* alpha, co
     p.t = s.t;
     p.nstrips = s.nstrips;
     p.tps = s.tps;
+    p.oslices = s.oslices;
+    p.oper = s.oper;
     p.ncopy = s.ncopy;
     p.npairs = s.npairs;
     p.scale = merge == MERGE_AVERAGE ? T(1) / (T)g.Cin : T(1);
@@ -894,6 +977,8 @@ hipError_t smorph_scm_backward(const T* x, const T* w, const T* alpha, const T* 
     p.t = s.t;
     p.nstrips = s.nstrips;
     p.tps = s.tps;
+    p.oslices = s.oslices;
+    p.oper = s.oper;
     p.ncopy = s.ncopy;
     p.npairs = s.npairs;
     p.scale = T(1);

@@ -215,6 +215,7 @@ struct SmorphBwdParams
     Tiling t;
     int nstrips;
     int tps;
+    int oslices, oper;  // generic kernel: output-channel slices per strip, channels of each
     int ncopy;
     int npairs;
     T scale;
