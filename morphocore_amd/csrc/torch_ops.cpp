@@ -32,6 +32,7 @@
 #include <vector>
 
 #include "../../include/morphocore_amd.h"
+#include "smorph_element.hpp"
 
 namespace
 {
@@ -1280,6 +1281,70 @@ PyMethodDef g_methods[] = {
     {nullptr, nullptr, 0, nullptr},
 };
 
+// ------------------------------------------------------------------------------------------------
+// The smorph element: the reference's blend of w with its flip by t = tanh(alpha)
+// (functional/smorph.py:56-70), as one launch forward and one backward.
+// ------------------------------------------------------------------------------------------------
+
+class SmorphElementFunction : public torch::autograd::Function<SmorphElementFunction>
+{
+public:
+    static Tensor forward(AutogradContext* ctx, const Tensor& w_in, const Tensor& t_in)
+    {
+        const c10::DeviceGuard guard(w_in.device());
+        const Tensor w = w_in.contiguous(), t = t_in.contiguous();
+        Tensor out = torch::empty(w.sizes(), w.options());
+        const int64_t pairs = t.numel(), K = w.size(2) * w.size(3);
+        const hipStream_t stream = (hipStream_t)stream_of(w);
+        const hipError_t err =
+            w.scalar_type() == c10::kFloat
+                ? mca::smorph_element_forward<float>(w.data_ptr<float>(), t.data_ptr<float>(), out.data_ptr<float>(), pairs, K, stream)
+                : mca::smorph_element_forward<double>(w.data_ptr<double>(), t.data_ptr<double>(), out.data_ptr<double>(), pairs, K, stream);
+        TORCH_CHECK(err == hipSuccess, hipGetErrorString(err));
+        ctx->save_for_backward({w, t});
+        return out;
+    }
+
+    static tensor_list backward(AutogradContext* ctx, tensor_list grad_outputs)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &w = saved[0], &t = saved[1];
+        const Tensor g = grad_outputs[0].contiguous();
+        TORCH_CHECK(g.sizes() == w.sizes() && g.device() == w.device() && g.scalar_type() == w.scalar_type(),
+                    "grad_output must match the element");
+        const c10::DeviceGuard guard(w.device());
+        if (torch::GradMode::is_enabled())
+        {
+            // The caller keeps the backward's own graph: in torch operations, which record it.
+            const Tensor t4 = t.reshape({w.size(0), w.size(1), 1, 1});
+            const Tensor same = (1 + t4) / 2, flipped = (1 - t4) / 2, wf = w.flip({-2, -1}), gs = g * t4;
+            return {gs * same + (gs * flipped).flip({-2, -1}),
+                    (g * (flipped * wf + same * w) + gs * (w - wf) / 2).sum({-2, -1}).reshape(t.sizes())};
+        }
+        Tensor gw = ctx->needs_input_grad(0) ? torch::empty_like(w) : Tensor();
+        Tensor gt = ctx->needs_input_grad(1) ? torch::empty_like(t) : Tensor();
+        const int64_t pairs = t.numel(), K = w.size(2) * w.size(3);
+        const hipStream_t stream = (hipStream_t)stream_of(w);
+        auto run = [&](auto zero) {
+            using T = decltype(zero);
+            return mca::smorph_element_backward<T>(w.data_ptr<T>(), t.data_ptr<T>(), g.data_ptr<T>(), gw.defined() ? gw.data_ptr<T>() : nullptr,
+                                                   gt.defined() ? gt.data_ptr<T>() : nullptr, pairs, K, stream);
+        };
+        const hipError_t err = w.scalar_type() == c10::kFloat ? run(0.0f) : run(0.0);
+        TORCH_CHECK(err == hipSuccess, hipGetErrorString(err));
+        return {gw, gt};
+    }
+};
+
+// w [Cout, Cw, KH, KW] and t with one value per channel pair (Cout * Cw values), float32 or float64.
+Tensor smorph_element(const Tensor& w, const Tensor& t)
+{
+    TORCH_CHECK(w.dim() == 4, "smorph_element: w must be [out_channels, in_channels, kernel_height, kernel_width]");
+    TORCH_CHECK(t.numel() == w.size(0) * w.size(1), "smorph_element: t must have one value per channel pair");
+    check_device("smorph_element", w, {t});
+    return SmorphElementFunction::apply(w, t);
+}
+
 }  // namespace
 
 // Same namespace, names and schemas as the reference (bindings.cpp:130-138).
@@ -1300,6 +1365,8 @@ TORCH_LIBRARY(morphocore, m)
     // No reference counterpart: a chain of dilation / erosion / smorph layers as one operator.
     m.def("morpho_stack(Tensor input, Tensor[] weights, Tensor[] alphas, int[] kinds, int[] merges, int[] paddings, "
           "float[] padding_values, bool save_indices=True, int chunk=0) -> Tensor");
+    // No reference counterpart: the element blend of the reference's Python smorph, from tanh(alpha).
+    m.def("smorph_element(Tensor w, Tensor t) -> Tensor");
 }
 
 // CompositeImplicitAutograd, as the reference (bindings.cpp:142-148): the kernels run above autograd
@@ -1313,6 +1380,7 @@ TORCH_LIBRARY_IMPL(morphocore, CompositeImplicitAutograd, m)
     m.impl("opening_closing", &opening_closing);
     m.impl("sigma_identity", &sigma_identity);
     m.impl("morpho_stack", &morpho_stack);
+    m.impl("smorph_element", &smorph_element);
 }
 
 // Importing morphocore_amd._C loads this library, which runs the registrations above.

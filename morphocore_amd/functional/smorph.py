@@ -18,6 +18,17 @@ def w_tilde(w: torch.Tensor, alpha: torch.Tensor, channel_merge_mode: str = "sum
     return tanh_alpha * (term2 * w.flip(dims=(-2, -1)) + term1 * w)
 
 
+def element(w: torch.Tensor, alpha: torch.Tensor, channel_merge_mode: str = "sum") -> torch.Tensor:
+    """:func:`w_tilde` as one launch forward and one backward (``torch.ops.morphocore.smorph_element``), with
+    the same roundings, for float32 / float64 elements on a HIP device with one alpha per channel pair;
+    other forms run the torch operations."""
+    per_pair = (w.dim() == 4 and w.shape[1] == 1 and alpha.numel() == w.shape[0] if channel_merge_mode == 'identity' or alpha.dim() == 1
+                else alpha.shape == w.shape[:2] and w.dim() == 4)
+    if per_pair and w.is_cuda and alpha.device == w.device and alpha.dtype == w.dtype and w.dtype in (torch.float32, torch.float64):
+        return ops.smorph_element(w, torch.tanh(alpha))
+    return w_tilde(w, alpha, channel_merge_mode)
+
+
 def smorph(x: torch.Tensor, w: torch.Tensor, alpha: torch.Tensor, beta: torch.Tensor = None,
            channel_merge_mode: str = "sum") -> torch.Tensor:
     """Smooth morphology: an alpha-softmax over each window, dilation-like for alpha -> +inf and
@@ -40,7 +51,7 @@ def smorph(x: torch.Tensor, w: torch.Tensor, alpha: torch.Tensor, beta: torch.Te
         min-like for beta < 0, their mean at 0); ``channel_merge_mode`` is then ignored.
     channel_merge_mode : 'sum', 'mean', 'max', 'min' or 'identity'.
     """
-    w_tilde_alpha = w_tilde(w, alpha, channel_merge_mode)
+    w_tilde_alpha = element(w, alpha, channel_merge_mode)
     if beta is not None:
         return ops.smorph_scm(x, w_tilde_alpha, alpha, beta)
     return ops.smorph(x, w_tilde_alpha, alpha, str_to_merge(channel_merge_mode))

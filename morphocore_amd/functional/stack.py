@@ -13,7 +13,7 @@ import torch
 
 from ._ops import ops
 from .merge_enum import str_to_merge, str_to_padding
-from .smorph import w_tilde
+from .smorph import element
 
 _KINDS = {"dilation": 0, "erosion": 1, "smorph": 2}
 
@@ -27,7 +27,7 @@ def _spec(layer):
             raise ValueError("A smorph layer is ('smorph', w, alpha[, channel_merge_mode])")
         merge = layer[3] if len(layer) > 3 else "sum"
         w, alpha = layer[1], layer[2]
-        return _KINDS[kind], w_tilde(w, alpha, merge), alpha, str_to_merge(merge), 0, 0.0
+        return _KINDS[kind], element(w, alpha, merge), alpha, str_to_merge(merge), 0, 0.0
     if not 2 <= len(layer) <= 5:
         raise ValueError(f"A {kind} layer is ('{kind}', w[, channel_merge_mode[, padding_mode[, padding_value]]])")
     merge, padding, value = (tuple(layer[2:]) + ("sum", "replicate", 0.0)[len(layer) - 2:])[:3]

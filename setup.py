@@ -32,9 +32,9 @@ ROCM_INCLUDE = "/opt/rocm/include"
 
 # The longest compiles first.
 KERNEL_SOURCES = ["morpho_fwd_f32_dilation.hip", "morpho_fwd_f32_erosion.hip", "morpho_fwd_f16.hip", "morpho_fwd_bf16.hip", "smorph_static.hip",
-                  "morpho_fwd_f64.hip", "morpho_fused.hip", "morpho_bwd.hip", "smorph.hip", "morpho_ident.hip", "morpho_scatter.hip", "morpho_fwd.hip", "util.hip",
+                  "morpho_fwd_f64.hip", "morpho_fused.hip", "morpho_bwd.hip", "smorph.hip", "smorph_element.hip", "morpho_ident.hip", "morpho_scatter.hip", "morpho_fwd.hip", "util.hip",
                   "capi.cpp", "stack.cpp"]
-KERNEL_HEADERS = ["common.hpp", "launch.hpp", "morpho_fwd.hpp", "smorph_common.hpp", os.path.join("..", "..", "include", "morphocore_amd.h")]
+KERNEL_HEADERS = ["common.hpp", "launch.hpp", "morpho_fwd.hpp", "smorph_common.hpp", "smorph_element.hpp", os.path.join("..", "..", "include", "morphocore_amd.h")]
 # Packed FP32 instructions stay disabled: only scalar fp32 VALU forms are emitted.
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-munsafe-fp-atomics", "-Wall", "-Wno-unused-function",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
@@ -88,7 +88,7 @@ class HipBuildExt(build_ext):
         target = self.get_ext_fullpath(ext.name)
         os.makedirs(os.path.dirname(target), exist_ok=True)
         torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
-        deps = list(ext.sources) + [os.path.join(ROOT, "include", "morphocore_amd.h"), KERNEL_LIB]
+        deps = list(ext.sources) + [os.path.join(CSRC, "smorph_element.hpp"), os.path.join(ROOT, "include", "morphocore_amd.h"), KERNEL_LIB]
         if not _stale(target, deps, self.force):
             return
         abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)

@@ -1,0 +1,83 @@
+"""The generic smorph kernels' unrolled rows (float64, and float32 elements without static kernels) and their
+output-channel slices, on planes with tiles inside the image and at its edges; and the element blend
+(torch.ops.morphocore.smorph_element) against the torch operations it replaces, bit for bit.
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from tests.helpers import TOL, normwise_error, seeded
+
+pytestmark = pytest.mark.gpu
+
+import morphocore_amd as mca  # noqa: E402
+from morphocore_amd.functional.smorph import element, w_tilde  # noqa: E402
+
+
+@pytest.mark.parametrize("merge", ["sum", "mean", "max", "identity"])
+@pytest.mark.parametrize("dtype,shape", [
+    (torch.float64, (1, 2, 5, 13, 200, 5, 5)),   # one slice per output channel
+    (torch.float64, (2, 3, 7, 40, 150, 3, 3)),
+    (torch.float64, (1, 1, 1, 9, 64, 7, 7)),
+    (torch.float64, (1, 2, 3, 21, 140, 11, 11)),
+    (torch.float32, (1, 3, 5, 33, 210, 9, 9)),
+    (torch.float32, (2, 2, 3, 30, 130, 4, 5)),   # even height
+    (torch.float32, (1, 2, 4, 1, 70, 3, 7)),     # a plane of one row
+    (torch.float32, (40, 8, 6, 8, 70, 5, 3)),    # enough tiles: one slice
+    (torch.float64, (1, 2, 3, 20, 70, 6, 6)),    # not unrolled
+])
+def test_generic_kernels(dtype, shape, merge):
+    B, Cin, Cout, H, W, KH, KW = shape
+    Cout = Cin if merge == "identity" else Cout
+    Cw = 1 if merge == "identity" else Cin
+    x = seeded(51, B, Cin, H, W, dtype=dtype, kind="randn")
+    w = seeded(52, Cout, Cw, KH, KW, dtype=dtype, kind="randn", scale=0.2)
+    alpha = seeded(53, Cout, Cw, dtype=dtype, kind="randn", scale=2.0)
+    alpha[0, 0] = 0.0
+    g = seeded(54, B, Cout, H, W, dtype=dtype, kind="randn")
+    m = O.MERGES[merge]
+    xd, wd, ad = (t.cuda().requires_grad_() for t in (x, w, alpha))
+    out = torch.ops.morphocore.smorph(xd, wd, ad, m)
+    out.backward(g.cuda())
+    a_np = alpha.numpy() if merge != "identity" else alpha.numpy().reshape(-1)
+    ref = O.smorph_forward(m, x.numpy(), w.numpy(), a_np)
+    assert np.array_equal(out.detach().cpu().numpy(), ref)
+    gx, gw, ga = O.smorph_backward(m, x.numpy(), w.numpy(), a_np, g.numpy())
+    for got, want in ((xd.grad, gx), (wd.grad, gw), (ad.grad, ga)):
+        assert normwise_error(got.cpu().numpy().reshape(np.shape(want)), want) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("mode,wshape,ashape", [("sum", (4, 3, 5, 5), (4, 3)), ("mean", (1, 1, 1, 1), (1, 1)), ("identity", (7, 1, 11, 11), (7, 1)),
+                                                ("identity", (5, 1, 3, 4), (5,)), ("sum", (6, 1, 9, 9), (6,))])
+def test_element_matches_torch(dtype, mode, wshape, ashape):
+    w = seeded(61, *wshape, dtype=dtype, kind="randn").cuda()
+    alpha = seeded(62, *ashape, dtype=dtype, kind="randn", scale=2.0).cuda()
+    g = seeded(63, *wshape, dtype=dtype, kind="randn").cuda()
+    w1, a1, w2, a2 = (t.clone().requires_grad_() for t in (w, alpha, w, alpha))
+    e1, e2 = element(w1, a1, mode), w_tilde(w2, a2, mode)
+    assert type(e1.grad_fn).__name__ != type(e2.grad_fn).__name__  # the fused operator ran
+    assert torch.equal(e1, e2)
+    # Gradients in 64 bits: each differs by roundings of the element's own type.
+    w64, a64 = (t.double().requires_grad_() for t in (w, alpha))
+    ref = torch.autograd.grad(w_tilde(w64, a64, mode), (w64, a64), g.double())
+    for got, want in zip(torch.autograd.grad(e1, (w1, a1), g), ref):
+        assert got.shape == want.shape and normwise_error(got.cpu().numpy(), want.cpu().numpy()) <= TOL[dtype]
+
+
+def test_element_other_forms():
+    """Forms the operator does not take run the torch operations; a graph of the backward is kept."""
+    w = seeded(64, 3, 2, 3, 3).cuda()
+    for alpha, mode in ((seeded(65, 1).cuda(), "sum"), (seeded(65, 3, 2, dtype=torch.float64).cuda(), "sum"), (seeded(65, 3).cuda(), "mean")):
+        assert torch.equal(element(w, alpha, mode), w_tilde(w, alpha, mode))
+    wp = w.permute(0, 1, 3, 2)
+    alpha = seeded(66, 3, 2).cuda()
+    assert torch.equal(element(wp, alpha), w_tilde(wp, alpha))
+    a1, a2, w1, w2 = (t.double().clone().requires_grad_() for t in (alpha, alpha, w, w))
+    seconds = []
+    for f, a, v in ((element, a1, w1), (w_tilde, a2, w2)):
+        first = torch.autograd.grad(f(v, a).square().sum(), (v, a), create_graph=True)
+        seconds.append(torch.autograd.grad(sum(t.square().sum() for t in first), (v, a)))
+    for got, want in zip(*seconds):
+        assert normwise_error(got.cpu().numpy(), want.cpu().numpy()) <= 1e-12
