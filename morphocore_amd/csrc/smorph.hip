@@ -578,7 +578,7 @@ static SmorphBwdPlan plan_smorph_bwd(int merge, const Geom& g, bool saved = fals
     // of the strip's grad_input), up to about 1024.
     s.oslices = 1;
     if (!stat && merge != MERGE_IDENTITY && g.Cout > 0)
-        s.oslices = (int)std::max<int64_t>(1, std::min<int64_t>(g.Cout, 1024 / (units * s.nstrips)));
+        s.oslices = (int)std::max<int64_t>(1, std::min<int64_t>(g.Cout, 1024 / std::max<int64_t>(1, units * s.nstrips)));
     s.oper = std::max(1, (g.Cout + s.oslices - 1) / s.oslices);
     s.oslices = std::max(1, (g.Cout + s.oper - 1) / s.oper);
     if (merge == MERGE_IDENTITY) s.oslices = 1;
