@@ -42,6 +42,35 @@ __global__ __launch_bounds__(BLOCK) void reduce_slots_kernel(const T* __restrict
         out[j] = (T)sum_slots(part, 0, nslots, n, j);
 }
 
+// The same sums in one launch for a few hundred slots: COLS consecutive columns per workgroup, each by
+// BLOCK / COLS threads that take every (BLOCK / COLS)-th slot; their sums are then added in thread order
+// (a fixed order, in double, rounded once).
+template <typename T, int COLS>
+__global__ __launch_bounds__(BLOCK) void reduce_joint_kernel(const T* __restrict__ part, int nslots, int64_t n, T* __restrict__ out)
+{
+    constexpr int Q = BLOCK / COLS, U = 8;  // U loads in flight per thread
+    __shared__ Acc sums[Q][COLS];
+    const int c = threadIdx.x % COLS, q = threadIdx.x / COLS;
+    const int64_t j = (int64_t)blockIdx.x * COLS + c;
+    Acc s = Acc(0);
+    if (j < n)
+        for (int b = q; b < nslots; b += U * Q)
+        {
+            T v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = part[(int64_t)min(b + u * Q, nslots - 1) * n + j];
+#pragma unroll
+            for (int u = 0; u < U; ++u) s += b + u * Q < nslots ? (Acc)v[u] : Acc(0);
+        }
+    sums[q][c] = s;
+    __syncthreads();
+    if (q != 0 || j >= n) return;
+    s = Acc(0);
+#pragma unroll
+    for (int k = 0; k < Q; ++k) s += sums[k][c];
+    out[j] = (T)s;
+}
+
 // First stage of a long reduction: group blockIdx.y sums slots [y * REDUCE_GROUP, (y + 1) *
 // REDUCE_GROUP) in slot order into tmp[y * n + j]; the groups are then summed in group order.
 template <typename T>
@@ -107,6 +136,10 @@ hipError_t fill_async(T* p, int64_t n, T v, hipStream_t stream)
     return hipGetLastError();
 }
 
+// Up to this many slots are summed by one launch (two took ~5 us each on the few thousand columns of a
+// layer); more by groups first, which spread the slots over more workgroups.
+constexpr int JOINT_SLOTS = 2048;
+
 template <typename T>
 size_t reduce_slots_scratch(int nslots, int64_t n)
 {
@@ -120,6 +153,15 @@ hipError_t reduce_slots_async(const T* part, int nslots, int64_t n, T* out, T* s
     if (nslots <= REDUCE_GROUP)
     {
         reduce_slots_kernel<T><<<grid_for(n), BLOCK, 0, stream>>>(part, nslots, n, out);
+        return hipGetLastError();
+    }
+    if (nslots <= JOINT_SLOTS)
+    {
+        // Few columns: 8 per workgroup, so that enough workgroups run.
+        if (n < 16384)
+            reduce_joint_kernel<T, 8><<<(unsigned)((n + 7) / 8), BLOCK, 0, stream>>>(part, nslots, n, out);
+        else
+            reduce_joint_kernel<T, 32><<<(unsigned)((n + 31) / 32), BLOCK, 0, stream>>>(part, nslots, n, out);
         return hipGetLastError();
     }
     const int groups = (nslots + REDUCE_GROUP - 1) / REDUCE_GROUP;
