@@ -37,6 +37,7 @@
 #include <algorithm>
 #include <cstdlib>
 
+#include "../../include/morphocore_amd.h"
 #include "launch.hpp"
 
 namespace mca
@@ -721,6 +722,8 @@ static PackedPlan plan_packed(const Geom& g)
     return s;
 }
 
+// Rows per wave of the sum / mean taps kernel's small launches.
+constexpr int SMALL_TAPS_RH = 2;
 // Rows per wave of the IDENTITY gather kernel.
 constexpr int GATHER_RH = 4;
 
@@ -735,6 +738,10 @@ struct TapsPlan
     size_t part_bytes;
     size_t lds;
 };
+
+// Workspace of a backward that recomputes its winners: the winners and a scratch output.
+template <typename T>
+static size_t recompute_workspace(int merge, const Geom& g);
 
 // band_ok: the row-band gather may run (its pointers are aligned; see ident_band_backward).
 template <typename T>
@@ -828,6 +835,33 @@ static TapsPlan plan_taps(int merge, const Geom& g, bool band_ok = true)
             return s;
         }
     }
+    // Sum / mean launches of few workgroups take 8-row tiles and one input channel each instead (9x9 at
+    // (4, 16 -> 24, 97, 131): 384 workgroups -> 2496).
+    // Their slots, four times as many, may not take a workspace past the fixed one of
+    // mca_morpho_backward_noalloc_f32 that the larger tiles' would fit.
+    if (!ident && (int64_t)g.B * s.t.ntiles() * ((g.Cin + 1) / 2) < 1024)
+    {
+        const Tiling t = make_tiling(g, SMALL_TAPS_RH);
+        const size_t cells = (size_t)t.rows * t.pitch * sizeof(Acc);
+        const size_t per_oc = K * 4 * sizeof(Acc);
+        const int64_t wnumel = (int64_t)g.Cout * g.Cw * g.taps();
+        auto slots_bytes = [&](int ntiles) {
+            return align_up((size_t)g.B * ntiles * wnumel * sizeof(T)) + align_up(reduce_slots_scratch<T>(g.B * ntiles, wnumel));
+        };
+        const bool fits = slots_bytes(t.ntiles()) + recompute_workspace<T>(merge, g) <= MCA_NOALLOC_SCRATCH_BYTES ||
+                          slots_bytes(s.t.ntiles()) > MCA_NOALLOC_SCRATCH_BYTES;
+        if (cells + per_oc + table <= target && fits)
+        {
+            s.t = t;
+            s.ncopy = 4;
+            s.ig = 1;
+            s.nig = g.Cin;
+            s.oc = std::max(1, std::min(g.Cout, (int)((target - cells - table) / per_oc)));
+            s.lds = cells + (size_t)s.oc * per_oc + table;
+            s.part_bytes = (size_t)g.B * t.ntiles() * g.Cout * g.Cw * K * sizeof(T);
+            return s;
+        }
+    }
     auto need = [&](int ig, int oc, int ncopy) { return ig * tile + (size_t)oc * ig * K * ncopy * sizeof(Acc) + table; };
     s.ncopy = 4;
     s.ig = ident ? 4 : 2;
@@ -917,6 +951,14 @@ static int recompute_batch(int merge, const Geom& g)
     return (int)std::max<int64_t>(1, std::min<int64_t>(fit, g.B));
 }
 
+template <typename T>
+static size_t recompute_workspace(int merge, const Geom& g)
+{
+    Geom c = g;
+    c.B = recompute_batch<T>(merge, g);
+    return align_up(indices_bytes(merge, c)) + align_up((size_t)c.B * c.Cout * c.plane() * sizeof(T));
+}
+
 // Workspace layout: [partial slots | reduction scratch | (recomputed winners | scratch output, for
 // recompute_batch batch elements)].
 template <typename T>
@@ -926,12 +968,7 @@ size_t morpho_backward_workspace(int merge, bool has_indices, const Geom& g)
     int nslots;
     partials_bound<T>(merge, g, part_bytes, nslots);
     size_t bytes = align_up(part_bytes) + align_up(reduce_slots_scratch<T>(nslots, (int64_t)g.Cout * g.Cw * g.taps()));
-    if (!has_indices)
-    {
-        Geom c = g;
-        c.B = recompute_batch<T>(merge, g);
-        bytes += align_up(indices_bytes(merge, c)) + align_up((size_t)c.B * c.Cout * c.plane() * sizeof(T));
-    }
+    if (!has_indices) bytes += recompute_workspace<T>(merge, g);
     if (packed_winners(merge) && sizeof(T) != sizeof(Acc))
     {
         const PackedPlan s = plan_packed<T>(g);
@@ -1088,6 +1125,13 @@ static hipError_t backward_op(int merge, bool replicate, T fill, const T* x, con
                 morpho_bwd_taps_kernel<T, OP, uint16_t, true, RH, 1><<<blocks, BLOCK, s.lds, stream>>>(p);
             else
                 morpho_bwd_taps_kernel<T, OP, uint8_t, true, RH, 1><<<blocks, BLOCK, s.lds, stream>>>(p);
+        }
+        else if (s.t.rh == SMALL_TAPS_RH)
+        {
+            if (wide)
+                morpho_bwd_taps_kernel<T, OP, uint16_t, false, SMALL_TAPS_RH, 1><<<blocks, BLOCK, s.lds, stream>>>(p);
+            else
+                morpho_bwd_taps_kernel<T, OP, uint8_t, false, SMALL_TAPS_RH, 1><<<blocks, BLOCK, s.lds, stream>>>(p);
         }
         else if (s.ig == 2)
         {
