@@ -31,76 +31,6 @@
 namespace mca
 {
 
-// Whether tap (kh, kw) of the output pixel whose first tap reads input row `iy` and column `ix`
-// (iy = h + KH / 2, ix = w + KW / 2) reads an in-image pixel.
-__device__ __forceinline__ bool tap_in_image(int iy, int ix, int kh, int kw, const Geom& g)
-{
-    return (unsigned)(iy - kh) < (unsigned)g.H && (unsigned)(ix - kw) < (unsigned)g.W;
-}
-
-// ref, S and W of one pair for the RH pixels of this lane (rows iy0 + r, column ix in input
-// coordinates of the first tap), from the staged tile.
-// KWS: the element's row length when it is known at compile time (else 0): a row's taps are then unrolled,
-// whose exponentials are independent chains of some twenty dependent operations each (one tap at a time
-// a wave waits on every step of its own chain, and small problems have one or two waves per SIMD). EDGE: some
-// tap of the tile may read outside the image (else every tap is taken without a test).
-template <typename T, int RH, int KWS, bool EDGE>
-__device__ __forceinline__ void smorph_pair_stats(const T* tbase, int pitch, const T* __restrict__ wp, T a, const Geom& g, int iy0, int ix,
-                                                  T (&ref)[RH], T (&S)[RH], T (&Wsum)[RH])
-{
-#pragma clang fp contract(off)  // S = S + e and W fused as the reference rounds them (written as fma)
-    const bool dilation_like = a >= T(0);
-    const T lo = ExpConsts<T>::min_input;
-    const int KW = KWS > 0 ? KWS : g.KW;
-    auto refs = [&](int kh, int kw) {
-        const T wk = wp[kh * KW + kw];
-#pragma unroll
-        for (int r = 0; r < RH; ++r)
-        {
-            const T v = tbase[(r - kh) * pitch - kw] + wk;
-            // Strict replacement: a NaN never wins, as in the reference.
-            const bool better = dilation_like ? v > ref[r] : v < ref[r];
-            if (better && (!EDGE || tap_in_image(iy0 + r, ix, kh, kw, g))) ref[r] = v;
-        }
-    };
-    auto sums = [&](int kh, int kw) {
-        const T wk = wp[kh * KW + kw];
-#pragma unroll
-        for (int r = 0; r < RH; ++r)
-        {
-            const T v = tbase[(r - kh) * pitch - kw] + wk;
-            const bool valid = !EDGE || tap_in_image(iy0 + r, ix, kh, kw, g);
-            const T e = valid ? exp_ref((v - ref[r]) * a, lo) : T(0);
-            S[r] = S[r] + e;
-            Wsum[r] = fma(e, valid ? v : T(0), Wsum[r]);
-        }
-    };
-    auto each_tap = [&](auto&& f) {
-        for (int kh = 0; kh < g.KH; ++kh)
-        {
-            if constexpr (KWS > 0)
-            {
-#pragma unroll
-                for (int kw = 0; kw < KWS; ++kw) f(kh, kw);
-            }
-            else
-            {
-                for (int kw = 0; kw < g.KW; ++kw) f(kh, kw);
-            }
-        }
-    };
-#pragma unroll
-    for (int r = 0; r < RH; ++r) ref[r] = dilation_like ? -std::numeric_limits<T>::infinity() : std::numeric_limits<T>::infinity();
-    each_tap(refs);
-#pragma unroll
-    for (int r = 0; r < RH; ++r)
-    {
-        S[r] = T(0);
-        Wsum[r] = T(0);
-    }
-    each_tap(sums);
-}
-
 // Whether every tap of every pixel of a tile staged from row y0 and column x0 reads the image (the same for
 // the whole workgroup).
 __device__ __forceinline__ bool tile_inside(const Geom& g, const Tiling& t, int y0, int x0)
@@ -682,6 +612,8 @@ static hipError_t finish_gacc(const SmorphBwdPlan& s, const Geom& g, const Acc* 
 template <typename T, int MK, bool STATS>
 static hipError_t launch_smorph_fwd(const SmorphFwdParams<T>& p, hipStream_t stream)
 {
+    if constexpr (!STATS)
+        if (smorph_rows_supported<T>(MK, p.g)) return launch_smorph_fwd_rows(MK, p, stream);
     if constexpr (sizeof(T) == 4)
         if (smorph_static_supported<T>(p.g)) return launch_smorph_fwd_static(MK, STATS, p, stream);
     constexpr int RH = rows_per_wave<T>();

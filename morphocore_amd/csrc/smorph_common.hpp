@@ -221,6 +221,84 @@ struct SmorphBwdParams
     T scale;
 };
 
+// Whether tap (kh, kw) of the output pixel whose first tap reads input row `iy` and column `ix`
+// (iy = h + KH / 2, ix = w + KW / 2) reads an in-image pixel.
+__device__ __forceinline__ bool tap_in_image(int iy, int ix, int kh, int kw, const Geom& g)
+{
+    return (unsigned)(iy - kh) < (unsigned)g.H && (unsigned)(ix - kw) < (unsigned)g.W;
+}
+
+// v when keep, +0 otherwise, by its bits: a select of an exponential becomes a branch around it, one a tap,
+// behind which no other tap's chain overlaps.
+__device__ __forceinline__ float keep_if(float v, bool keep) { return __uint_as_float(__float_as_uint(v) & (keep ? ~0u : 0u)); }
+__device__ __forceinline__ double keep_if(double v, bool keep)
+{
+    return __longlong_as_double(__double_as_longlong(v) & (keep ? ~0ll : 0ll));
+}
+
+// ref, S and W of one pair for the RH pixels of this lane (rows iy0 + r, column ix in input
+// coordinates of the first tap), from the staged tile.
+// KWS: the element's row length when it is known at compile time (else 0): a row's taps are then unrolled,
+// whose exponentials are independent chains of some twenty dependent operations each (one tap at a time
+// a wave waits on every step of its own chain, and small problems have one or two waves per SIMD). EDGE: some
+// tap of the tile may read outside the image (else every tap is taken without a test).
+template <typename T, int RH, int KWS, bool EDGE>
+__device__ __forceinline__ void smorph_pair_stats(const T* tbase, int pitch, const T* wp, T a, const Geom& g, int iy0, int ix,
+                                                  T (&ref)[RH], T (&S)[RH], T (&Wsum)[RH])
+{
+#pragma clang fp contract(off)  // S = S + e and W fused as the reference rounds them (written as fma)
+    const bool dilation_like = a >= T(0);
+    const T lo = ExpConsts<T>::min_input;
+    const int KW = KWS > 0 ? KWS : g.KW;
+    auto refs = [&](int kh, int kw) {
+        const T wk = wp[kh * KW + kw];
+#pragma unroll
+        for (int r = 0; r < RH; ++r)
+        {
+            const T v = tbase[(r - kh) * pitch - kw] + wk;
+            // Strict replacement: a NaN never wins, as in the reference.
+            const bool better = dilation_like ? v > ref[r] : v < ref[r];
+            if (better && (!EDGE || tap_in_image(iy0 + r, ix, kh, kw, g))) ref[r] = v;
+        }
+    };
+    auto sums = [&](int kh, int kw) {
+        const T wk = wp[kh * KW + kw];
+#pragma unroll
+        for (int r = 0; r < RH; ++r)
+        {
+            const T v = tbase[(r - kh) * pitch - kw] + wk;
+            const bool valid = !EDGE || tap_in_image(iy0 + r, ix, kh, kw, g);
+            const T e = keep_if(exp_ref((v - ref[r]) * a, lo), valid);
+            S[r] = S[r] + e;
+            Wsum[r] = fma(e, keep_if(v, valid), Wsum[r]);
+        }
+    };
+    auto each_tap = [&](auto&& f) {
+        for (int kh = 0; kh < g.KH; ++kh)
+        {
+            if constexpr (KWS > 0)
+            {
+#pragma unroll
+                for (int kw = 0; kw < KWS; ++kw) f(kh, kw);
+            }
+            else
+            {
+                for (int kw = 0; kw < g.KW; ++kw) f(kh, kw);
+            }
+        }
+    };
+#pragma unroll
+    for (int r = 0; r < RH; ++r) ref[r] = dilation_like ? -std::numeric_limits<T>::infinity() : std::numeric_limits<T>::infinity();
+    each_tap(refs);
+#pragma unroll
+    for (int r = 0; r < RH; ++r)
+    {
+        S[r] = T(0);
+        Wsum[r] = T(0);
+    }
+    each_tap(sums);
+}
+
 // Structuring-element sizes with static-size smorph kernels (smorph_static.hip).
 template <typename T>
 inline bool smorph_static_supported(const Geom& g)
@@ -260,6 +338,12 @@ inline int64_t smorph_stats_count(int merge, const Geom& g)
 // forward that saves the pair statistics and the backward that reads them.
 hipError_t launch_smorph_fwd_static(int mk, bool stats, const SmorphFwdParams<float>& p, hipStream_t stream);
 hipError_t launch_smorph_bwd_static(int mk, const SmorphBwdParams<float>& p, hipStream_t stream);
+// The forward of launches with few workgroups (smorph_rows.hip): whether it takes the shape, and its launcher
+// (merges SUM, MAX, MIN and SMOOTH; saves the pair statistics when p.pstats is not null).
+template <typename T>
+bool smorph_rows_supported(int mk, const Geom& g);
+template <typename T>
+hipError_t launch_smorph_fwd_rows(int mk, const SmorphFwdParams<T>& p, hipStream_t stream);
 // MAX / MIN merge target and winner counts of every output pixel from the saved W / S values (`outp`).
 hipError_t launch_smorph_counts_saved(const float* outp, const float* out, float* counts, float* target, const Geom& g, hipStream_t stream);
 

@@ -32,7 +32,7 @@ ROCM_INCLUDE = "/opt/rocm/include"
 
 # The longest compiles first.
 KERNEL_SOURCES = ["morpho_fwd_f32_dilation.hip", "morpho_fwd_f32_erosion.hip", "morpho_fwd_f16.hip", "morpho_fwd_bf16.hip", "smorph_static.hip",
-                  "morpho_fwd_f64.hip", "morpho_fused.hip", "morpho_bwd.hip", "smorph.hip", "smorph_element.hip", "morpho_ident.hip", "morpho_scatter.hip", "morpho_fwd.hip", "util.hip",
+                  "morpho_fwd_f64.hip", "morpho_fused.hip", "morpho_bwd.hip", "smorph.hip", "smorph_element.hip", "smorph_rows.hip", "morpho_ident.hip", "morpho_scatter.hip", "morpho_fwd.hip", "util.hip",
                   "capi.cpp", "stack.cpp"]
 KERNEL_HEADERS = ["common.hpp", "launch.hpp", "morpho_fwd.hpp", "smorph_common.hpp", "smorph_element.hpp", os.path.join("..", "..", "include", "morphocore_amd.h")]
 # Packed FP32 instructions stay disabled: only scalar fp32 VALU forms are emitted.
@@ -51,6 +51,15 @@ def _stale(target, deps, force):
         return True
     t = os.path.getmtime(target)
     return any(os.path.getmtime(d) > t for d in deps)
+
+
+def _included(depfile, headers):
+    """The project's headers that the compiler listed for an object (all of them when it listed none)."""
+    if not os.path.exists(depfile):
+        return headers
+    with open(depfile) as f:
+        listed = {os.path.realpath(p) for p in f.read().replace("\\\n", " ").split()}
+    return [h for h in headers if os.path.realpath(h) in listed]
 
 
 class HipBuildExt(build_ext):
@@ -72,8 +81,8 @@ class HipBuildExt(build_ext):
             path = os.path.join(CSRC, src)
             obj = os.path.join(OBJDIR, src + ".o")
             objs.append(obj)
-            if _stale(obj, [path] + headers, self.force):
-                jobs.append([HIPCC] + HIP_FLAGS + ["-c", path, "-o", obj])
+            if _stale(obj, [path] + _included(obj + ".d", headers), self.force):
+                jobs.append([HIPCC] + HIP_FLAGS + ["-MMD", "-MF", obj + ".d", "-c", path, "-o", obj])
         with ThreadPoolExecutor(self._jobs()) as pool:
             for f in [pool.submit(_run, j) for j in jobs]:
                 f.result()
