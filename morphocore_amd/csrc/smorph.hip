@@ -31,6 +31,9 @@
 namespace mca
 {
 
+// Elements of up to this many rows have their rows unrolled (smorph_unrolled).
+constexpr int UNROLLED_KH = 64;
+
 // Whether every tap of every pixel of a tile staged from row y0 and column x0 reads the image (the same for
 // the whole workgroup).
 __device__ __forceinline__ bool tile_inside(const Geom& g, const Tiling& t, int y0, int x0)
@@ -46,6 +49,7 @@ __global__ __launch_bounds__(BLOCK) void smorph_fwd_kernel(const SmorphFwdParams
     T* tile = reinterpret_cast<T*>(smem_raw);
     const Geom g = p.g;
     const Tiling t = p.t;
+    T* wl = tile + t.rows * t.pitch;  // KWS: the pair's element
     const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
     int work = xcd_work_index(blockIdx.x, gridDim.x);
     const int o = work % g.Cout;
@@ -84,10 +88,17 @@ __global__ __launch_bounds__(BLOCK) void smorph_fwd_kernel(const SmorphFwdParams
     {
         __syncthreads();
         stage_tile(tile, p.x + ((int64_t)b * g.Cin + i) * plane, g, t, y0, x0, false, T(0));
+        const T* __restrict__ wg = p.w + ((int64_t)o * g.Cw + (MK == MK_IDENT ? 0 : i)) * K;
+        if constexpr (KWS > 0)
+            for (int k = threadIdx.x; k < K; k += BLOCK) wl[k] = wg[k];
         __syncthreads();
         const int pair = MK == MK_IDENT ? o : o * g.Cin + i;
         const T a = p.alpha[pair];
-        const T* __restrict__ wp = p.w + ((int64_t)o * g.Cw + (MK == MK_IDENT ? 0 : i)) * K;
+        const T* wp;
+        if constexpr (KWS > 0)
+            wp = wl;
+        else
+            wp = wg;
         T ref[RH], S[RH], Wsum[RH];
         if (inside)
             smorph_pair_stats<T, RH, KWS, false>(tbase, t.pitch, wp, a, g, iy0, ix, ref, S, Wsum);
@@ -162,6 +173,7 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
     Acc* bins = GGIN ? gtile : gtile + tile_elems;
     Acc* abins = bins + K * p.ncopy;
     Acc* bbins = abins + p.ncopy;
+    T* wl = reinterpret_cast<T*>(bins + nb * p.ncopy);  // KWS: the current and the next pair's element
     const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
     int work = xcd_work_index(blockIdx.x, gridDim.x);
     const int oslice = work % p.oslices;  // the workgroups of a strip share its tiles in L2
@@ -200,12 +212,35 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
         const int o_begin = MK == MK_IDENT ? i : oslice * p.oper;
         const int o_end = MK == MK_IDENT ? i + 1 : min(o_begin + p.oper, g.Cout);
         const bool inside = tile_inside(g, t, y0, x0);
+        const int wi = MK == MK_IDENT ? 0 : i;
+        auto element = [&](int o) { return p.w + ((int64_t)o * g.Cw + wi) * K; };
+        // The next pair's element is loaded while the current one is routed, and staged before the barrier
+        // that ends it.
+        constexpr int NW = KWS > 0 ? (KWS * UNROLLED_KH + BLOCK - 1) / BLOCK : 1;
+        if constexpr (KWS > 0)
+        {
+            if (o_begin < o_end)
+                for (int k = threadIdx.x; k < K; k += BLOCK) wl[k] = element(o_begin)[k];
+            __syncthreads();
+        }
         for (int o = o_begin; o < o_end; ++o)
         {
-            const int wi = MK == MK_IDENT ? 0 : i;
             const int pair = MK == MK_IDENT ? o : o * g.Cin + i;
             const T a = p.alpha[pair];
-            const T* __restrict__ wp = p.w + ((int64_t)o * g.Cw + wi) * K;
+            const int wbuf = (o - o_begin) & 1;
+            T wnext[NW];
+            const T* wp;
+            if constexpr (KWS > 0)
+            {
+                wp = wl + wbuf * K;
+                const T* __restrict__ wn = element(min(o + 1, o_end - 1));
+#pragma unroll
+                for (int j = 0; j < NW; ++j) wnext[j] = wn[min((int)threadIdx.x + j * BLOCK, K - 1)];
+            }
+            else
+            {
+                wp = element(o);
+            }
             T ref[RH], S[RH], Wsum[RH], outp[RH], scaled[RH], asum[RH];
             bool in[RH];
             T bsum = T(0);
@@ -269,17 +304,18 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
                     const T centered = v - outp[r];
                     // c = pg (1 + a centered) and the alpha term pg (v - ref) centered share pg centered.
                     const T q = pg * centered;
-                    const T c = fma(a, q, pg);
-                    const T as = fma(q, v - ref[r], asum[r]);
-                    asum[r] = routes ? as : asum[r];
-                    if (routes)
+                    // A tap that does not route adds zeros (its own cell and bin exist): no branch per tap.
+                    const T c = keep_if(fma(a, q, pg), routes);
+                    asum[r] = fma(keep_if(q, routes), keep_if(v - ref[r], routes), asum[r]);
+                    if constexpr (GGIN)
                     {
-                        if constexpr (GGIN)
-                            global_add(&gacc_plane[(int64_t)(iy0 + r - kh) * g.W + (ix - kw)], (Acc)c);
-                        else
-                            lds_add(&gtile[(wave * RH + r + g.KH - 1 - kh) * t.pitch + lane + g.KW - 1 - kw], (Acc)c);
-                        lds_add(&bins[k * p.ncopy + copy], (Acc)c);
+                        if (routes) global_add(&gacc_plane[(int64_t)(iy0 + r - kh) * g.W + (ix - kw)], (Acc)c);
                     }
+                    else
+                    {
+                        lds_add(&gtile[(wave * RH + r + g.KH - 1 - kh) * t.pitch + lane + g.KW - 1 - kw], (Acc)c);
+                    }
+                    lds_add(&bins[k * p.ncopy + copy], (Acc)c);
                 }
             };
             for (int kh = 0; kh < g.KH; ++kh)
@@ -300,6 +336,12 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
             if (as != T(0)) lds_add(&abins[copy], (Acc)as);
             if constexpr (MK == MK_SMOOTH)
                 if (bsum != T(0)) lds_add(&bbins[copy], (Acc)bsum);
+            if constexpr (KWS > 0)
+            {
+#pragma unroll
+                for (int j = 0; j < NW; ++j)
+                    if ((int)threadIdx.x + j * BLOCK < K) wl[(wbuf ^ 1) * K + threadIdx.x + j * BLOCK] = wnext[j];
+            }
             __syncthreads();
             for (int j = threadIdx.x; j < nb; j += BLOCK)
             {
@@ -442,7 +484,18 @@ struct SmorphBwdPlan
 // hide each other's latency. Other widths take the default rows per wave, one after the other. Float64
 // 5x5 at (2, 8 -> 8, 64, 60): forward 168 -> 60 us, backward 288 -> 61 (with the output-channel slices);
 // its training step 528 -> 133 (with smorph_element).
-static bool smorph_unrolled(const Geom& g) { return g.KW <= 11 && g.KW >= 3 && g.KW % 2 == 1; }
+// They read the pair's element from LDS, at the same address in every lane: scalar loads share the LDS
+// reads' wait counter, and a scalar operand halves an instruction's rate. With it, and out-of-image taps masked
+// by their bits (a select of an exponential becomes a branch a tap), the backward of float64 11x11 at
+// (3, 7 -> 13, 105, 75) takes 1552 us, 1769 before; 5x5 at (2, 8 -> 8, 64, 60) 55, 62 before. (Elements of more
+// than 64 rows, which need the LDS for their tiles, are not unrolled.)
+static bool smorph_unrolled(const Geom& g) { return g.KW <= 11 && g.KW >= 3 && g.KW % 2 == 1 && g.KH <= UNROLLED_KH; }
+// LDS of that element.
+template <typename T>
+static size_t smorph_element_lds(const Geom& g)
+{
+    return smorph_unrolled(g) ? (size_t)g.taps() * sizeof(T) : 0;
+}
 
 // Rows per wave of the generic forward: one where the element's rows are unrolled, else the default while its
 // tile fits the tuned LDS budget, else one (a shorter tile, for large elements).
@@ -484,7 +537,7 @@ static SmorphBwdPlan plan_smorph_bwd(int merge, const Geom& g, bool saved = fals
             rh = (attempt == 0 || attempt == 2) && !smorph_unrolled(g) ? rows_per_wave<T>() : 1;
             const Tiling t = make_tiling(g, rh);
             const size_t cells = (size_t)t.rows * t.pitch;
-            const size_t fixed = align16(cells * sizeof(T)) + (ggin ? 0 : cells * sizeof(Acc));
+            const size_t fixed = align16(cells * sizeof(T)) + (ggin ? 0 : cells * sizeof(Acc)) + (ggin ? 0 : 2 * smorph_element_lds<T>(g));
             int ncopy = 16;
             while (ncopy > 1 && fixed + nbins * ncopy * sizeof(Acc) > budget) ncopy /= 2;
             s.ncopy = ncopy;
@@ -531,7 +584,7 @@ size_t smorph_lds(int merge, const Geom& g, bool backward)
     if (backward) return plan_smorph_bwd<T>(merge, g).lds;
     if (smorph_static_supported<T>(g)) return 0;  // static LDS
     const Tiling t = make_tiling(g, smorph_fwd_rh<T>(g));
-    return (size_t)t.rows * t.pitch * sizeof(T);
+    return (size_t)t.rows * t.pitch * sizeof(T) + smorph_element_lds<T>(g);
 }
 
 // Workspace bytes of one backward plan: slot partials, MAX / MIN counts and target, reduction scratch.
@@ -618,7 +671,7 @@ static hipError_t launch_smorph_fwd(const SmorphFwdParams<T>& p, hipStream_t str
         if (smorph_static_supported<T>(p.g)) return launch_smorph_fwd_static(MK, STATS, p, stream);
     constexpr int RH = rows_per_wave<T>();
     const int64_t blocks = (int64_t)p.g.B * p.t.nty * p.t.ntx * p.g.Cout;
-    const size_t lds = (size_t)p.t.rows * p.t.pitch * sizeof(T);
+    const size_t lds = (size_t)p.t.rows * p.t.pitch * sizeof(T) + smorph_element_lds<T>(p.g);
     if (p.t.rh == 1)
         switch (smorph_unrolled(p.g) ? p.g.KW : 0)
         {
@@ -815,7 +868,7 @@ size_t smorph_scm_lds(const Geom& g, bool backward)
     if (backward) return plan_smorph_bwd<T>(MERGE_SMOOTH, g).lds;
     if (smorph_static_supported<T>(g)) return 0;  // static LDS
     const Tiling t = make_tiling(g, smorph_fwd_rh<T>(g));
-    return (size_t)t.rows * t.pitch * sizeof(T);
+    return (size_t)t.rows * t.pitch * sizeof(T) + smorph_element_lds<T>(g);
 }
 
 static unsigned elementwise_grid(int64_t n)
