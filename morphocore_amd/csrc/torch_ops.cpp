@@ -1301,14 +1301,15 @@ public:
                 ? mca::smorph_element_forward<float>(w.data_ptr<float>(), t.data_ptr<float>(), out.data_ptr<float>(), pairs, K, stream)
                 : mca::smorph_element_forward<double>(w.data_ptr<double>(), t.data_ptr<double>(), out.data_ptr<double>(), pairs, K, stream);
         TORCH_CHECK(err == hipSuccess, hipGetErrorString(err));
-        ctx->save_for_backward({w, t});
+        // The inputs themselves, whatever their strides: a backward that records its own graph reaches them.
+        ctx->save_for_backward({w_in, t_in});
         return out;
     }
 
     static tensor_list backward(AutogradContext* ctx, tensor_list grad_outputs)
     {
         const auto saved = ctx->get_saved_variables();
-        const Tensor &w = saved[0], &t = saved[1];
+        const Tensor w = saved[0].contiguous(), t = saved[1].contiguous();
         const Tensor g = grad_outputs[0].contiguous();
         TORCH_CHECK(g.sizes() == w.sizes() && g.device() == w.device() && g.scalar_type() == w.scalar_type(),
                     "grad_output must match the element");

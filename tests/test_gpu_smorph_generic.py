@@ -81,3 +81,16 @@ def test_element_other_forms():
         seconds.append(torch.autograd.grad(sum(t.square().sum() for t in first), (v, a)))
     for got, want in zip(*seconds):
         assert normwise_error(got.cpu().numpy(), want.cpu().numpy()) <= 1e-12
+
+
+def test_element_keeps_strided_inputs_in_the_graph():
+    """Second gradients of an element and alpha that are strided views reach both."""
+    w, alpha = seeded(67, 3, 2, 5, 3, dtype=torch.float64).cuda(), seeded(68, 2, 3, dtype=torch.float64).cuda()
+    seconds = []
+    for f in (element, w_tilde):
+        v, a = w.clone().requires_grad_(), alpha.clone().requires_grad_()
+        vt, at = v.permute(0, 1, 3, 2), a.t()
+        first = torch.autograd.grad(f(vt, at).square().sum(), (vt, at), create_graph=True)
+        seconds.append(torch.autograd.grad(sum(t.square().sum() for t in first), (v, a)))
+    for got, want in zip(*seconds):
+        assert normwise_error(got.cpu().numpy(), want.cpu().numpy()) <= 1e-12
