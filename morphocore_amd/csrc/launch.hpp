@@ -155,15 +155,16 @@ struct IdentTiles
 {
     int tw, th, ntx, nty;
     int ncopy_log2;  // copies of each grad_weight bin
-    int64_t blocks;
     size_t lds;
     bool ok;
 };
 IdentTiles ident_tiles(const Geom& g);
 // IDENTITY: grad_input, and grad_weight's sums per (batch element, tile) in part
-// ([B * ntx * nty][Cout][KH * KW], T: double for double storage, else float).
+// ([B * ntx * nty][Cout][KH * KW], T: double for double storage, else float). tiles: the plan of the whole
+// batch, by which the caller laid its slots out; g may be a chunk of that batch, whose own plan can differ.
 template <typename T, typename ST>
-hipError_t ident_tile_backward(int op, const void* taps, const ST* grad_out, ST* grad_in, T* part, const Geom& g, hipStream_t stream);
+hipError_t ident_tile_backward(int op, const IdentTiles& tiles, const void* taps, const ST* grad_out, ST* grad_in, T* part, const Geom& g,
+                               hipStream_t stream);
 
 // Opening / closing with IDENTITY merges fused into one pass (morpho_fused.hip). g: Cin == Cout == C,
 // Cw == 1; first_op: the first stage's op.

@@ -735,6 +735,7 @@ struct TapsPlan
     bool gather;  // morpho_bwd_ident_gather_kernel (else morpho_bwd_taps_kernel)
     bool band;    // gathered by ident_band_gather (morpho_ident.hip): slots per (batch element, band)
     bool tile;    // ident_tile_backward (morpho_scatter.hip): slots per (batch element, tile)
+    IdentTiles ident;  // its tiles, also for a chunk of the batch (the slots' layout)
     size_t part_bytes;
     size_t lds;
 };
@@ -770,6 +771,7 @@ static TapsPlan plan_taps(int merge, const Geom& g, bool band_ok = true)
             s.t.nty = tiles.nty;
             s.gather = true;
             s.tile = true;
+            s.ident = tiles;
             s.ig = 1;
             s.nig = g.Cin;
             s.oc = 1;
@@ -1100,7 +1102,7 @@ static hipError_t backward_op(int merge, bool replicate, T fill, const T* x, con
         }
         else if (s.tile)
         {
-            if ((err = ident_tile_backward<T, T>(OP, taps, p.gout, p.gin, p.part, gc, stream)) != hipSuccess) return err;
+            if ((err = ident_tile_backward<T, T>(OP, s.ident, taps, p.gout, p.gin, p.part, gc, stream)) != hipSuccess) return err;
         }
         else if (s.gather)
         {
@@ -1232,7 +1234,7 @@ static hipError_t half_direct(int merge, const void* indices, const ST* grad_out
     }
     else
     {
-        if ((err = ident_tile_backward<float, ST>(OP, indices, grad_out, grad_in, part, g, stream)) != hipSuccess) return err;
+        if ((err = ident_tile_backward<float, ST>(OP, plan_taps<float>(merge, g).ident, indices, grad_out, grad_in, part, g, stream)) != hipSuccess) return err;
     }
     if ((err = reduce_slots_async<float>(part, nslots, wnumel, gw, scratch, stream)) != hipSuccess) return err;
     return convert_async<float, ST>(gw, grad_w, wnumel, stream);

@@ -278,20 +278,22 @@ IdentTiles ident_tiles(const Geom& g)
     {
         t.nty = (g.H + th - 1) / th;
         t.th = (g.H + t.nty - 1) / t.nty;
-        t.blocks = (int64_t)g.B * g.Cin * t.nty * t.ntx;
-        const bool one_reduction = t.blocks < 256 || (int64_t)g.B * t.ntx * ((g.H + th / 2 - 1) / std::max(th / 2, 1)) <= REDUCE_GROUP;
-        if (t.blocks >= 1024 || th / 2 < std::max(g.KH - 1, 4) || !one_reduction) break;
+        const int64_t blocks = (int64_t)g.B * g.Cin * t.nty * t.ntx;
+        const bool one_reduction = blocks < 256 || (int64_t)g.B * t.ntx * ((g.H + th / 2 - 1) / std::max(th / 2, 1)) <= REDUCE_GROUP;
+        if (blocks >= 1024 || th / 2 < std::max(g.KH - 1, 4) || !one_reduction) break;
     }
     // Copies of every grad_weight bin, one per lane of a half wave while they take at most 16 KiB.
     for (t.ncopy_log2 = 5; t.ncopy_log2 > 0 && ((size_t)g.taps() << t.ncopy_log2) * sizeof(Acc) > 16 * 1024; --t.ncopy_log2) {}
     t.lds = ((size_t)t.tw * t.th + ((size_t)g.taps() << t.ncopy_log2)) * sizeof(Acc);
     const int64_t region = (int64_t)std::min(t.th + g.KH - 1, g.H) * std::min(t.tw + g.KW - 1, g.W);
-    t.ok = t.lds <= LDS_LIMIT && region < 65536 && region <= 8 * (int64_t)t.tw * t.th && t.blocks <= 0x7fffffff;
+    t.ok = t.lds <= LDS_LIMIT && region < 65536 && region <= 8 * (int64_t)t.tw * t.th &&
+           (int64_t)g.B * g.Cin * t.nty * t.ntx <= 0x7fffffff;
     return t;
 }
 
 template <typename T, typename ST>
-hipError_t ident_tile_backward(int op, const void* taps, const ST* grad_out, ST* grad_in, T* part, const Geom& g, hipStream_t stream)
+hipError_t ident_tile_backward(int op, const IdentTiles& tiles, const void* taps, const ST* grad_out, ST* grad_in, T* part, const Geom& g,
+                               hipStream_t stream)
 {
     IdentTileParams<T, ST> p{};
     p.taps = taps;
@@ -299,13 +301,14 @@ hipError_t ident_tile_backward(int op, const void* taps, const ST* grad_out, ST*
     p.gin = grad_in;
     p.part = part;
     p.g = g;
-    p.t = ident_tiles(g);
+    p.t = tiles;
     p.kw_magic = div_magic(g.KW);
-    if (!p.t.ok) return hipErrorInvalidValue;
+    const int64_t blocks = (int64_t)g.B * g.Cin * tiles.nty * tiles.ntx;
+    if (!tiles.ok || blocks > 0x7fffffff) return hipErrorInvalidValue;
     const bool wide = pair_tap_bytes(g) == 2;
     const auto kernel = op == DILATION ? (wide ? ident_tile_kernel<DILATION, T, ST, uint16_t> : ident_tile_kernel<DILATION, T, ST, uint8_t>)
                                        : (wide ? ident_tile_kernel<EROSION, T, ST, uint16_t> : ident_tile_kernel<EROSION, T, ST, uint8_t>);
-    kernel<<<(unsigned)p.t.blocks, BLOCK, p.t.lds, stream>>>(p);
+    kernel<<<(unsigned)blocks, BLOCK, p.t.lds, stream>>>(p);
     return hipGetLastError();
 }
 
@@ -313,9 +316,9 @@ template hipError_t packed_tile_backward<float, float>(const int32_t*, const flo
 template hipError_t packed_tile_backward<double, double>(const int32_t*, const double*, double*, const Geom&, hipStream_t);
 template hipError_t packed_tile_backward<float, _Float16>(const int32_t*, const _Float16*, _Float16*, const Geom&, hipStream_t);
 template hipError_t packed_tile_backward<float, __bf16>(const int32_t*, const __bf16*, __bf16*, const Geom&, hipStream_t);
-template hipError_t ident_tile_backward<float, float>(int, const void*, const float*, float*, float*, const Geom&, hipStream_t);
-template hipError_t ident_tile_backward<double, double>(int, const void*, const double*, double*, double*, const Geom&, hipStream_t);
-template hipError_t ident_tile_backward<float, _Float16>(int, const void*, const _Float16*, _Float16*, float*, const Geom&, hipStream_t);
-template hipError_t ident_tile_backward<float, __bf16>(int, const void*, const __bf16*, __bf16*, float*, const Geom&, hipStream_t);
+template hipError_t ident_tile_backward<float, float>(int, const IdentTiles&, const void*, const float*, float*, float*, const Geom&, hipStream_t);
+template hipError_t ident_tile_backward<double, double>(int, const IdentTiles&, const void*, const double*, double*, double*, const Geom&, hipStream_t);
+template hipError_t ident_tile_backward<float, _Float16>(int, const IdentTiles&, const void*, const _Float16*, _Float16*, float*, const Geom&, hipStream_t);
+template hipError_t ident_tile_backward<float, __bf16>(int, const IdentTiles&, const void*, const __bf16*, __bf16*, float*, const Geom&, hipStream_t);
 
 }  // namespace mca

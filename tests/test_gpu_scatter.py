@@ -5,6 +5,9 @@ input channels, elements larger than the tile, partial last tiles, and an elemen
 count that the global atomics stay. Identity in float32 and 16-bit on planes the row bands do not take:
 one to two tile columns, planes of one row or column, even, rectangular and 17x17 elements (two-byte
 taps). Against the oracle: the operator's contract (1e-6 / 1e-12, one rounding in 16 bits).
+
+Backwards without saved taps walk the batch in chunks over one layout of partial slots: at shapes whose
+tiles depend on the batch, and chunks that do not divide it.
 """
 import numpy as np
 import pytest
@@ -72,3 +75,32 @@ def test_packed_falls_back_to_atomics():
 def test_identity_tiles(op, shape, dtype):
     for padding in ("replicate", "geodesic"):
         _run(op, "identity", padding, dtype, *shape)
+
+
+@pytest.mark.parametrize("op,shape,dtype", [
+    ("dilation", (64, 32, 64, 64, 3, 3), torch.float32),   # 1 tile a plane for the batch, 16 for one element
+    ("erosion", (16, 8, 128, 128, 5, 5), torch.float32),   # 4 and 32
+    ("dilation", (16, 8, 128, 128, 7, 7), torch.float64),
+])
+def test_identity_recomputed_taps_in_chunks_of_one_plan(op, shape, dtype, monkeypatch):
+    """Chunks of the batch take the tiles of the whole batch, which its partial slots are laid out by: the
+    gradients are the oracle's, and the same bit for bit whatever the chunk (the gradient's values are
+    multiples of 1/8 below 32, so that every sum of them is exact)."""
+    B, C, H, W, KH, KW = shape
+    x = seeded(14, B, C, H, W, dtype=dtype)
+    w = seeded(15, C, 1, KH, KW, dtype=dtype, kind="randn", scale=0.1)
+    g = (seeded(16, B, C, H, W, dtype=dtype, kind="randn") * 8).round() / 8
+    o = O.DILATION if op == "dilation" else O.EROSION
+    run = torch.ops.morphocore.dilation if op == "dilation" else torch.ops.morphocore.erosion
+    one = C * H * W * (1 + x.element_size())  # taps and scratch output of one batch element
+    gx, gw = O.morpho_backward(o, O.MERGES["identity"], O.REPLICATE, 0.0, x.numpy(), w.numpy(), g.numpy())
+    grads = []
+    for elements in (B, 1, 3, B - 1):
+        monkeypatch.setenv("MORPHOCORE_AMD_RECOMPUTE_BYTES", str(elements * one))
+        xd, wd = x.cuda().requires_grad_(), w.cuda().requires_grad_()
+        run(xd, wd, O.MERGES["identity"], O.REPLICATE, 0.0, False, 0.0).backward(g.cuda())
+        grads.append((xd.grad, wd.grad))
+        assert normwise_error(xd.grad.cpu().numpy(), gx) <= TOL[dtype], elements
+        assert normwise_error(wd.grad.cpu().numpy(), gw) <= TOL[dtype], elements
+    for gi, wi in grads[1:]:
+        assert torch.equal(gi, grads[0][0]) and torch.equal(wi, grads[0][1])
