@@ -35,7 +35,8 @@ namespace mca
 constexpr int UNROLLED_KH = 64;
 
 // Whether every tap of every pixel of a tile staged from row y0 and column x0 reads the image (the same for
-// the whole workgroup).
+// the whole workgroup). Only the unrolled kernels ask: a second copy of the others' loops takes registers that
+// cost a wave per SIMD (float32 rows of 8: 94 -> 98; 6x6 at (26, 2 -> 21, 20, 102) 141 -> 167 us).
 __device__ __forceinline__ bool tile_inside(const Geom& g, const Tiling& t, int y0, int x0)
 {
     return y0 >= 0 && x0 >= 0 && y0 + t.rows <= g.H && x0 + t.cols <= g.W;
@@ -82,7 +83,7 @@ __global__ __launch_bounds__(BLOCK) void smorph_fwd_kernel(const SmorphFwdParams
 
     const int i_begin = MK == MK_IDENT ? o : 0;
     const int i_end = MK == MK_IDENT ? o + 1 : g.Cin;
-    const bool inside = tile_inside(g, t, y0, x0);
+    const bool inside = KWS > 0 && tile_inside(g, t, y0, x0);
     const T* tbase = tile + (wave * RH + g.KH - 1) * t.pitch + lane + g.KW - 1;
     for (int i = i_begin; i < i_end; ++i)
     {
@@ -94,16 +95,11 @@ __global__ __launch_bounds__(BLOCK) void smorph_fwd_kernel(const SmorphFwdParams
         __syncthreads();
         const int pair = MK == MK_IDENT ? o : o * g.Cin + i;
         const T a = p.alpha[pair];
-        const T* wp;
-        if constexpr (KWS > 0)
-            wp = wl;
-        else
-            wp = wg;
         T ref[RH], S[RH], Wsum[RH];
         if (inside)
-            smorph_pair_stats<T, RH, KWS, false>(tbase, t.pitch, wp, a, g, iy0, ix, ref, S, Wsum);
+            smorph_pair_stats<T, RH, KWS, false>(tbase, t.pitch, wg, wl, a, g, iy0, ix, ref, S, Wsum);
         else
-            smorph_pair_stats<T, RH, KWS, true>(tbase, t.pitch, wp, a, g, iy0, ix, ref, S, Wsum);
+            smorph_pair_stats<T, RH, KWS, true>(tbase, t.pitch, wg, wl, a, g, iy0, ix, ref, S, Wsum);
 #pragma unroll
         for (int r = 0; r < RH; ++r)
         {
@@ -211,7 +207,7 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
 
         const int o_begin = MK == MK_IDENT ? i : oslice * p.oper;
         const int o_end = MK == MK_IDENT ? i + 1 : min(o_begin + p.oper, g.Cout);
-        const bool inside = tile_inside(g, t, y0, x0);
+        const bool inside = KWS > 0 && tile_inside(g, t, y0, x0);
         const int wi = MK == MK_IDENT ? 0 : i;
         auto element = [&](int o) { return p.w + ((int64_t)o * g.Cw + wi) * K; };
         // The next pair's element is loaded while the current one is routed, and staged before the barrier
@@ -229,25 +225,21 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
             const T a = p.alpha[pair];
             const int wbuf = (o - o_begin) & 1;
             T wnext[NW];
-            const T* wp;
+            const T* __restrict__ wg = element(o);
+            const T* wp = wl + wbuf * K;
             if constexpr (KWS > 0)
             {
-                wp = wl + wbuf * K;
                 const T* __restrict__ wn = element(min(o + 1, o_end - 1));
 #pragma unroll
                 for (int j = 0; j < NW; ++j) wnext[j] = wn[min((int)threadIdx.x + j * BLOCK, K - 1)];
-            }
-            else
-            {
-                wp = element(o);
             }
             T ref[RH], S[RH], Wsum[RH], outp[RH], scaled[RH], asum[RH];
             bool in[RH];
             T bsum = T(0);
             if (inside)
-                smorph_pair_stats<T, RH, KWS, false>(tbase, t.pitch, wp, a, g, iy0, ix, ref, S, Wsum);
+                smorph_pair_stats<T, RH, KWS, false>(tbase, t.pitch, wg, wp, a, g, iy0, ix, ref, S, Wsum);
             else
-                smorph_pair_stats<T, RH, KWS, true>(tbase, t.pitch, wp, a, g, iy0, ix, ref, S, Wsum);
+                smorph_pair_stats<T, RH, KWS, true>(tbase, t.pitch, wg, wp, a, g, iy0, ix, ref, S, Wsum);
 #pragma unroll
             for (int r = 0; r < RH; ++r)
             {
@@ -285,13 +277,14 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
             const int KW = KWS > 0 ? KWS : g.KW;
             auto route = [&](int kh, int kw) {
                 const int k = kh * KW + kw;
-                const T wk = wp[k];
+                const T wk = KWS > 0 ? wp[k] : wg[k];
 #pragma unroll
                 for (int r = 0; r < RH; ++r)
                 {
                     // Every in-image tap of an in-image pixel routes, also with a zero gradient
                     // (so that a NaN of the pair reaches the gradients, as in the reference).
                     const bool routes = in[r] && (inside || tap_in_image(iy0 + r, ix, kh, kw, g));
+                    if (KWS == 0 && !routes) continue;  // (not unrolled: no overlap to lose, see smorph_pair_stats)
                     const T v = tbase[(r - kh) * t.pitch - kw] + wk;
                     // The routing's exponential: the hardware one in float32 (the sums above,
                     // and so the output, use the reference's).
@@ -304,12 +297,12 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
                     const T centered = v - outp[r];
                     // c = pg (1 + a centered) and the alpha term pg (v - ref) centered share pg centered.
                     const T q = pg * centered;
-                    // A tap that does not route adds zeros (its own cell and bin exist): no branch per tap.
+                    // Unrolled: a tap that does not route adds zeros (its own cell and bin exist), no branch per tap.
                     const T c = keep_if(fma(a, q, pg), routes);
                     asum[r] = fma(keep_if(q, routes), keep_if(v - ref[r], routes), asum[r]);
                     if constexpr (GGIN)
                     {
-                        if (routes) global_add(&gacc_plane[(int64_t)(iy0 + r - kh) * g.W + (ix - kw)], (Acc)c);
+                        global_add(&gacc_plane[(int64_t)(iy0 + r - kh) * g.W + (ix - kw)], (Acc)c);
                     }
                     else
                     {

@@ -241,34 +241,42 @@ __device__ __forceinline__ double keep_if(double v, bool keep)
 // KWS: the element's row length when it is known at compile time (else 0): a row's taps are then unrolled,
 // whose exponentials are independent chains of some twenty dependent operations each (one tap at a time
 // a wave waits on every step of its own chain, and small problems have one or two waves per SIMD). EDGE: some
-// tap of the tile may read outside the image (else every tap is taken without a test).
+// tap of the tile may read outside the image (else every tap is taken without a test). The element: wl, in LDS,
+// where KWS > 0, else wg, in global memory (restrict: by scalar loads). Rows that are not unrolled have no
+// other tap's chain to overlap: they branch around the exponentials no lane takes, which are most of them on
+// planes smaller than the tile (15x15 at (4, 86 -> 1, 8, 158), float32: 15.7 ms, 23.0 with all of them).
 template <typename T, int RH, int KWS, bool EDGE>
-__device__ __forceinline__ void smorph_pair_stats(const T* tbase, int pitch, const T* wp, T a, const Geom& g, int iy0, int ix,
-                                                  T (&ref)[RH], T (&S)[RH], T (&Wsum)[RH])
+__device__ __forceinline__ void smorph_pair_stats(const T* tbase, int pitch, const T* __restrict__ wg, const T* wl, T a, const Geom& g, int iy0,
+                                                  int ix, T (&ref)[RH], T (&S)[RH], T (&Wsum)[RH])
 {
 #pragma clang fp contract(off)  // S = S + e and W fused as the reference rounds them (written as fma)
     const bool dilation_like = a >= T(0);
     const T lo = ExpConsts<T>::min_input;
     const int KW = KWS > 0 ? KWS : g.KW;
     auto refs = [&](int kh, int kw) {
-        const T wk = wp[kh * KW + kw];
+        const T wk = KWS > 0 ? wl[kh * KW + kw] : wg[kh * KW + kw];
 #pragma unroll
         for (int r = 0; r < RH; ++r)
         {
             const T v = tbase[(r - kh) * pitch - kw] + wk;
             // Strict replacement: a NaN never wins, as in the reference.
             const bool better = dilation_like ? v > ref[r] : v < ref[r];
-            if (better && (!EDGE || tap_in_image(iy0 + r, ix, kh, kw, g))) ref[r] = v;
+            // (bitwise: a logical and becomes a branch a row)
+            ref[r] = better & (!EDGE | tap_in_image(iy0 + r, ix, kh, kw, g)) ? v : ref[r];
         }
     };
     auto sums = [&](int kh, int kw) {
-        const T wk = wp[kh * KW + kw];
+        const T wk = KWS > 0 ? wl[kh * KW + kw] : wg[kh * KW + kw];
 #pragma unroll
         for (int r = 0; r < RH; ++r)
         {
             const T v = tbase[(r - kh) * pitch - kw] + wk;
             const bool valid = !EDGE || tap_in_image(iy0 + r, ix, kh, kw, g);
-            const T e = keep_if(exp_ref((v - ref[r]) * a, lo), valid);
+            T e;
+            if constexpr (KWS > 0)
+                e = keep_if(exp_ref((v - ref[r]) * a, lo), valid);
+            else
+                e = valid ? exp_ref((v - ref[r]) * a, lo) : T(0);
             S[r] = S[r] + e;
             Wsum[r] = fma(e, keep_if(v, valid), Wsum[r]);
         }

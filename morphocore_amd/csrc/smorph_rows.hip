@@ -103,9 +103,9 @@ __global__ __launch_bounds__(BLOCK) void smorph_fwd_rows(const RowsParams<T> q)
         T ref[1], S[1], Wsum[1];
         __builtin_amdgcn_wave_barrier();
         if (inside)
-            smorph_pair_stats<T, 1, KS, false>(tbase, cols, wp, a, g, h + P, wc + P, ref, S, Wsum);
+            smorph_pair_stats<T, 1, KS, false>(tbase, cols, nullptr, wp, a, g, h + P, wc + P, ref, S, Wsum);
         else
-            smorph_pair_stats<T, 1, KS, true>(tbase, cols, wp, a, g, h + P, wc + P, ref, S, Wsum);
+            smorph_pair_stats<T, 1, KS, true>(tbase, cols, nullptr, wp, a, g, h + P, wc + P, ref, S, Wsum);
         const T inv = T(1) / S[0];
         if (in && i0 + wave < g.Cin)
         {
