@@ -241,8 +241,9 @@ constexpr int REDUCE_GROUP = 32;
 template <typename T>
 size_t reduce_slots_scratch(int nslots, int64_t n);
 
-// out[j] = sum of part[s * n + j] over the slots s, in a fixed order (deterministic).
-template <typename T>
-hipError_t reduce_slots_async(const T* part, int nslots, int64_t n, T* out, T* scratch, hipStream_t stream);
+// out[j] = sum of part[s * n + j] over the slots s, in a fixed order (deterministic). PT: the slots' type (T, or
+// double for float results).
+template <typename T, typename PT>
+hipError_t reduce_slots_async(const PT* part, int nslots, int64_t n, T* out, PT* scratch, hipStream_t stream);
 
 }  // namespace mca

@@ -151,10 +151,12 @@ __global__ __launch_bounds__(BLOCK) void smorph_fwd_kernel(const SmorphFwdParams
     }
 }
 
-// GGIN: grad_input is summed in global memory (p.gacc, double atomics per routed tap) instead of an LDS
-// copy of the tile flushed per tile: for elements whose tile and its double copy exceed the LDS.
+// The sums that leave a workgroup stay in double: grad_input (added by every output-channel slice and
+// overlapping tile) and the partial slots (a sum per tile), rounded once at the end in float32.
+// GGIN: grad_input is summed in global memory (p.gin) per routed tap instead of in an LDS copy of the tile
+// flushed per tile: for elements whose tile and its double copy exceed the LDS.
 template <typename T, int MK, int RH, bool GGIN, int KWS>
-__global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams<T> p)
+__global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams<T, Acc> p)
 {
 #pragma clang fp contract(off)  // fused only where the reference fuses (written as fma)
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -181,8 +183,8 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
     const int64_t plane = g.plane();
     const int64_t wnumel = (int64_t)g.Cout * g.Cw * K;
     const int slot = b * p.nstrips + strip;
-    T* part_w = p.part_w + (int64_t)slot * wnumel;
-    T* part_a = p.part_a + (int64_t)slot * p.npairs;
+    Acc* part_w = p.part_w + (int64_t)slot * wnumel;
+    Acc* part_a = p.part_a + (int64_t)slot * p.npairs;
     const int copy = lane & (p.ncopy - 1);
     const T lo = ExpConsts<T>::min_input;
 
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
         if constexpr (!GGIN)
             for (int j = threadIdx.x; j < tile_elems; j += BLOCK) gtile[j] = Acc(0);
         __syncthreads();
-        Acc* __restrict__ gacc_plane = GGIN ? p.gacc + ((int64_t)b * g.Cin + i) * plane : nullptr;
+        Acc* __restrict__ gplane = p.gin + ((int64_t)b * g.Cin + i) * plane;
 
         const int o_begin = MK == MK_IDENT ? i : oslice * p.oper;
         const int o_end = MK == MK_IDENT ? i + 1 : min(o_begin + p.oper, g.Cout);
@@ -302,7 +304,7 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
                     asum[r] = fma(keep_if(q, routes), keep_if(v - ref[r], routes), asum[r]);
                     if constexpr (GGIN)
                     {
-                        global_add(&gacc_plane[(int64_t)(iy0 + r - kh) * g.W + (ix - kw)], (Acc)c);
+                        global_add(&gplane[(int64_t)(iy0 + r - kh) * g.W + (ix - kw)], (Acc)c);
                     }
                     else
                     {
@@ -345,17 +347,16 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
                     bins[j * p.ncopy + c] = Acc(0);
                 }
                 if (j < K)
-                    part_w[((int64_t)o * g.Cw + wi) * K + j] += (T)s;
+                    part_w[((int64_t)o * g.Cw + wi) * K + j] += s;
                 else if (j == K)
-                    part_a[pair] += (T)s;
+                    part_a[pair] += s;
                 else
-                    p.part_b[((int64_t)slot * g.Cin + i) * g.Cout + o] += (T)s;
+                    p.part_b[((int64_t)slot * g.Cin + i) * g.Cout + o] += s;
             }
             __syncthreads();
         }
 
         if constexpr (GGIN) continue;  // nothing staged: grad_input is already in global memory
-        T* gplane = p.gin + ((int64_t)b * g.Cin + i) * plane;
         for (int ly = wave; ly < t.rows; ly += NWAVES)
         {
             const int iy = y0 + ly;
@@ -364,8 +365,8 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
             {
                 const int gx = x0 + lx;
                 if (gx < 0 || gx >= g.W) continue;
-                const T v = (T)gtile[ly * t.pitch + lx];
-                if (v != T(0)) global_add(&gplane[(int64_t)iy * g.W + gx], v);
+                const Acc v = gtile[ly * t.pitch + lx];
+                if (v != Acc(0)) global_add(&gplane[(int64_t)iy * g.W + gx], v);
             }
         }
     }
@@ -469,7 +470,9 @@ struct SmorphBwdPlan
     int npairs;
     int oslices, oper;  // generic kernel: output-channel slices, one workgroup each, and their channels
     bool ggin;  // generic kernel with grad_input summed in global memory (smorph_bwd_kernel<..., true>)
-    size_t part_w_bytes, part_a_bytes, part_b_bytes, counts_bytes, gacc_bytes;
+    // Workspace: grad_weight, grad_alpha and (SMOOTH) grad_beta partials, the double grad_input sums of float
+    // tensors, winner counts and merge target (MAX / MIN), reduction scratch.
+    size_t part_a, part_b, gacc, counts, scratch, bytes;
     size_t lds;
 };
 
@@ -558,16 +561,22 @@ static SmorphBwdPlan plan_smorph_bwd(int merge, const Geom& g, bool saved = fals
     s.oper = std::max(1, (g.Cout + s.oslices - 1) / s.oslices);
     s.oslices = std::max(1, (g.Cout + s.oper - 1) / s.oper);
     if (merge == MERGE_IDENTITY) s.oslices = 1;
-    const size_t nslots = (size_t)g.B * s.nstrips;
-    s.part_w_bytes = nslots * wnumel * sizeof(T);
-    s.part_a_bytes = nslots * s.npairs * sizeof(T);
+    const int nslots = g.B * s.nstrips;
+    const size_t part = stat ? sizeof(T) : sizeof(Acc);  // bytes of a partial sum
+    s.part_a = align_up((size_t)nslots * wnumel * part);
+    s.part_b = s.part_a + align_up((size_t)nslots * s.npairs * part);
     // SMOOTH: grad_beta partials [slot][Cin][Cout], as many values as the grad_alpha ones.
-    s.part_b_bytes = merge == MERGE_SMOOTH ? s.part_a_bytes : 0;
+    const bool smooth = merge == MERGE_SMOOTH;
+    s.gacc = s.part_b + (smooth ? s.part_b - s.part_a : 0);
+    const bool rounded = !stat && sizeof(T) != sizeof(Acc);
+    s.counts = s.gacc + (rounded ? align_up((size_t)g.B * g.Cin * g.plane() * sizeof(Acc)) : 0);
     // MAX / MIN: winner counts, then the merge target, per output pixel.
-    s.counts_bytes = (merge == MERGE_MAX || merge == MERGE_MIN) ? 2 * (size_t)g.B * g.Cout * g.plane() * sizeof(T) : 0;
-    // grad_input summed in global memory: a double buffer, rounded into grad_input afterwards (float
-    // tensors; double ones sum into grad_input itself).
-    s.gacc_bytes = (s.ggin && sizeof(T) != sizeof(Acc)) ? (size_t)g.B * g.Cin * g.plane() * sizeof(Acc) : 0;
+    s.scratch = s.counts + (merge == MERGE_MAX || merge == MERGE_MIN ? align_up(2 * (size_t)g.B * g.Cout * g.plane() * sizeof(T)) : 0);
+    auto reduction = [&](int slots, int64_t n) { return stat ? reduce_slots_scratch<T>(slots, n) : reduce_slots_scratch<Acc>(slots, n); };
+    const size_t red = reduction(nslots, wnumel > s.npairs ? wnumel : s.npairs);
+    // SMOOTH: grad_beta sums nslots * Cin partial rows of Cout values.
+    const size_t red_b = smooth ? reduction(nslots * g.Cin, g.Cout) : 0;
+    s.bytes = s.scratch + align_up(red > red_b ? red : red_b);
     return s;
 }
 
@@ -580,33 +589,20 @@ size_t smorph_lds(int merge, const Geom& g, bool backward)
     return (size_t)t.rows * t.pitch * sizeof(T) + smorph_element_lds<T>(g);
 }
 
-// Workspace bytes of one backward plan: slot partials, MAX / MIN counts and target, reduction scratch.
-template <typename T>
-static size_t smorph_plan_workspace(const SmorphBwdPlan& s, const Geom& g)
-{
-    const int nslots = g.B * s.nstrips;
-    const int64_t wnumel = (int64_t)g.Cout * g.Cw * g.taps();
-    const size_t red = reduce_slots_scratch<T>(nslots, wnumel > s.npairs ? wnumel : s.npairs);
-    // SMOOTH: grad_beta sums nslots * Cin partial rows of Cout values.
-    const size_t red_b = s.part_b_bytes ? reduce_slots_scratch<T>(nslots * g.Cin, g.Cout) : 0;
-    return align_up(s.part_w_bytes) + align_up(s.part_a_bytes) + align_up(s.part_b_bytes) + align_up(s.counts_bytes) +
-           align_up(red > red_b ? red : red_b) + align_up(s.gacc_bytes);
-}
-
 // Enough for either backward (recomputing or from saved statistics): the caller sizes the workspace
 // before it knows which one runs.
 template <typename T>
 size_t smorph_backward_workspace(int merge, const Geom& g)
 {
-    const size_t a = smorph_plan_workspace<T>(plan_smorph_bwd<T>(merge, g, false), g);
-    const size_t b = smorph_static_supported<T>(g) ? smorph_plan_workspace<T>(plan_smorph_bwd<T>(merge, g, true), g) : 0;
+    const size_t a = plan_smorph_bwd<T>(merge, g, false).bytes;
+    const size_t b = smorph_static_supported<T>(g) ? plan_smorph_bwd<T>(merge, g, true).bytes : 0;
     return a > b ? a : b;
 }
 
 // The generic backward kernel of a plan: the default rows per wave or one, grad_input summed in an LDS
 // copy of the tile or in global memory.
 template <typename T, int MK>
-static hipError_t launch_smorph_bwd_generic(const SmorphBwdPlan& s, const SmorphBwdParams<T>& p, hipStream_t stream)
+static hipError_t launch_smorph_bwd_generic(const SmorphBwdPlan& s, const SmorphBwdParams<T, Acc>& p, hipStream_t stream)
 {
     constexpr int RH = rows_per_wave<T>();
     const unsigned blocks = (unsigned)((int64_t)p.g.B * p.g.Cin * s.nstrips * s.oslices);
@@ -627,31 +623,25 @@ static hipError_t launch_smorph_bwd_generic(const SmorphBwdPlan& s, const Smorph
     return hipGetLastError();
 }
 
-// Where the global-memory grad_input sum of a plan goes: grad_input itself for double tensors, the
-// workspace buffer (zero-filled here, rounded into grad_input by finish_gacc) for float ones; null
-// when the plan sums it in LDS.
+// Zeros for everything the generic backward adds to: the partial slots and the grad_input sums behind them (one
+// launch; double tensors sum into grad_input itself).
 template <typename T>
-static hipError_t prepare_gacc(const SmorphBwdPlan& s, const Geom& g, T* grad_in, Acc* buffer, Acc** gacc, hipStream_t stream)
+static hipError_t clear_smorph_sums(const SmorphBwdPlan& s, const Geom& g, unsigned char* ws, T* grad_in, hipStream_t stream)
 {
-    *gacc = nullptr;
-    if (!s.ggin) return hipSuccess;
     if constexpr (sizeof(T) == sizeof(Acc))
     {
-        *gacc = reinterpret_cast<Acc*>(grad_in);  // zero-filled by the caller
-        return hipSuccess;
+        const hipError_t err = fill_async<T>(grad_in, (int64_t)g.B * g.Cin * g.plane(), T(0), stream);
+        if (err != hipSuccess) return err;
     }
-    else
-    {
-        *gacc = buffer;
-        return fill_async<Acc>(buffer, (int64_t)g.B * g.Cin * g.plane(), Acc(0), stream);
-    }
+    return fill_async<Acc>(reinterpret_cast<Acc*>(ws), (int64_t)(s.counts / sizeof(Acc)), Acc(0), stream);
 }
 
+// The double grad_input sums of float tensors, rounded.
 template <typename T>
-static hipError_t finish_gacc(const SmorphBwdPlan& s, const Geom& g, const Acc* buffer, T* grad_in, hipStream_t stream)
+static hipError_t round_smorph_gin(const SmorphBwdPlan& s, const Geom& g, const unsigned char* ws, T* grad_in, hipStream_t stream)
 {
     if constexpr (sizeof(T) != sizeof(Acc))
-        if (s.ggin) return round_async<T>(buffer, grad_in, (int64_t)g.B * g.Cin * g.plane(), stream);
+        return round_async<T>(reinterpret_cast<const Acc*>(ws + s.gacc), grad_in, (int64_t)g.B * g.Cin * g.plane(), stream);
     return hipSuccess;
 }
 
@@ -724,29 +714,18 @@ hipError_t smorph_backward(int merge, const T* x, const T* w, const T* alpha, co
     const int64_t nstat = smorph_stats_count<T>(merge, g);
     const SmorphBwdPlan s = plan_smorph_bwd<T>(merge, g, stats != nullptr);
     // The layout below is this plan's; never lay it out past the buffer.
-    if (workspace_bytes < smorph_plan_workspace<T>(s, g)) return hipErrorInvalidValue;
+    if (workspace_bytes < s.bytes) return hipErrorInvalidValue;
     const int64_t wnumel = (int64_t)g.Cout * g.Cw * g.taps();
-    if ((err = fill_async<T>(grad_in, (int64_t)g.B * g.Cin * g.plane(), T(0), stream)) != hipSuccess) return err;
     if ((int64_t)g.B * g.Cout * g.plane() == 0 || g.Cin == 0)
     {
+        if ((err = fill_async<T>(grad_in, (int64_t)g.B * g.Cin * g.plane(), T(0), stream)) != hipSuccess) return err;
         if ((err = fill_async<T>(grad_w, wnumel, T(0), stream)) != hipSuccess) return err;
         return fill_async<T>(grad_alpha, s.npairs, T(0), stream);
     }
     unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
-    T* part_w = reinterpret_cast<T*>(ws);
-    T* part_a = reinterpret_cast<T*>(ws + align_up(s.part_w_bytes));
-    T* counts = reinterpret_cast<T*>(ws + align_up(s.part_w_bytes) + align_up(s.part_a_bytes));
+    T* counts = reinterpret_cast<T*>(ws + s.counts);
     T* target = counts + (int64_t)g.B * g.Cout * g.plane();
-    Acc* gbuf = reinterpret_cast<Acc*>(ws + align_up(s.part_w_bytes) + align_up(s.part_a_bytes) + align_up(s.counts_bytes));
-    T* scratch = reinterpret_cast<T*>(ws + align_up(s.part_w_bytes) + align_up(s.part_a_bytes) + align_up(s.counts_bytes) +
-                                      align_up(s.gacc_bytes));
     const int nslots = g.B * s.nstrips;
-    // The static kernels that keep their partials in LDS store every slot entry themselves.
-    if (!(smorph_static_supported<T>(g) && smorph_bwd_lds_partials(g, merge == MERGE_IDENTITY)))
-    {
-        if ((err = fill_async<T>(part_w, (int64_t)nslots * wnumel, T(0), stream)) != hipSuccess) return err;
-        if ((err = fill_async<T>(part_a, (int64_t)nslots * s.npairs, T(0), stream)) != hipSuccess) return err;
-    }
 
     if (stats && (merge == MERGE_MAX || merge == MERGE_MIN))
     {
@@ -769,42 +748,59 @@ hipError_t smorph_backward(int merge, const T* x, const T* w, const T* alpha, co
         if (err != hipSuccess) return err;
     }
 
-    SmorphBwdParams<T> p{};
-    p.x = x;
-    p.w = w;
-    p.alpha = alpha;
-    // MAX / MIN compare the pair outputs with the merge target (the forward's output unless channel
-    // 0's pair output is NaN).
-    p.out = (merge == MERGE_MAX || merge == MERGE_MIN) ? target : out;
-    p.counts = counts;
-    p.gout = grad_out;
-    p.gin = grad_in;
-    p.part_w = part_w;
-    p.part_a = part_a;
-    p.pstats = stats;
-    p.nstat = nstat;
-    p.g = g;
-    p.t = s.t;
-    p.nstrips = s.nstrips;
-    p.tps = s.tps;
-    p.oslices = s.oslices;
-    p.oper = s.oper;
-    p.ncopy = s.ncopy;
-    p.npairs = s.npairs;
-    p.scale = merge == MERGE_AVERAGE ? T(1) / (T)g.Cin : T(1);
+    // PT: the partial slots' type.
+    auto params = [&](auto zero) {
+        using PT = decltype(zero);
+        SmorphBwdParams<T, PT> p{};
+        p.x = x;
+        p.w = w;
+        p.alpha = alpha;
+        // MAX / MIN compare the pair outputs with the merge target (the forward's output unless channel
+        // 0's pair output is NaN).
+        p.out = (merge == MERGE_MAX || merge == MERGE_MIN) ? target : out;
+        p.counts = counts;
+        p.gout = grad_out;
+        p.part_w = reinterpret_cast<PT*>(ws);
+        p.part_a = reinterpret_cast<PT*>(ws + s.part_a);
+        p.pstats = stats;
+        p.nstat = nstat;
+        p.g = g;
+        p.t = s.t;
+        p.nstrips = s.nstrips;
+        p.tps = s.tps;
+        p.oslices = s.oslices;
+        p.oper = s.oper;
+        p.ncopy = s.ncopy;
+        p.npairs = s.npairs;
+        p.scale = merge == MERGE_AVERAGE ? T(1) / (T)g.Cin : T(1);
+        return p;
+    };
+    auto reduce = [&](const auto& p) {
+        auto* scratch = reinterpret_cast<decltype(p.part_w)>(ws + s.scratch);
+        const hipError_t e = reduce_slots_async<T>(p.part_w, nslots, wnumel, grad_w, scratch, stream);
+        return e != hipSuccess ? e : reduce_slots_async<T>(p.part_a, nslots, s.npairs, grad_alpha, scratch, stream);
+    };
     const int mk = merge == MERGE_MAX ? MK_MAX : (merge == MERGE_MIN ? MK_MIN : (merge == MERGE_IDENTITY ? MK_IDENT : MK_SUM));
     if constexpr (sizeof(T) == 4)
     {
         if (smorph_static_supported<T>(g))
         {
+            auto p = params(T(0));
+            p.gin = grad_in;
+            if ((err = fill_async<T>(grad_in, (int64_t)g.B * g.Cin * g.plane(), T(0), stream)) != hipSuccess) return err;
+            // The kernels that keep their partials in LDS store every slot entry themselves.
+            if (!smorph_bwd_lds_partials(g, merge == MERGE_IDENTITY))
+            {
+                if ((err = fill_async<T>(p.part_w, (int64_t)nslots * wnumel, T(0), stream)) != hipSuccess) return err;
+                if ((err = fill_async<T>(p.part_a, (int64_t)nslots * s.npairs, T(0), stream)) != hipSuccess) return err;
+            }
             if ((err = launch_smorph_bwd_static(mk, p, stream)) != hipSuccess) return err;
-            if ((err = reduce_slots_async<T>(part_w, nslots, wnumel, grad_w, scratch, stream)) != hipSuccess) return err;
-            return reduce_slots_async<T>(part_a, nslots, s.npairs, grad_alpha, scratch, stream);
+            return reduce(p);
         }
     }
-    Acc* gacc = nullptr;
-    if ((err = prepare_gacc<T>(s, g, grad_in, gbuf, &gacc, stream)) != hipSuccess) return err;
-    p.gacc = gacc;
+    auto p = params(Acc(0));
+    p.gin = sizeof(T) == sizeof(Acc) ? reinterpret_cast<Acc*>(grad_in) : reinterpret_cast<Acc*>(ws + s.gacc);
+    if ((err = clear_smorph_sums<T>(s, g, ws, grad_in, stream)) != hipSuccess) return err;
     switch (merge)
     {
         case MERGE_ADD:
@@ -815,9 +811,8 @@ hipError_t smorph_backward(int merge, const T* x, const T* w, const T* alpha, co
         default: return hipErrorInvalidValue;
     }
     if (err != hipSuccess) return err;
-    if ((err = finish_gacc<T>(s, g, gbuf, grad_in, stream)) != hipSuccess) return err;
-    if ((err = reduce_slots_async<T>(part_w, nslots, wnumel, grad_w, scratch, stream)) != hipSuccess) return err;
-    return reduce_slots_async<T>(part_a, nslots, s.npairs, grad_alpha, scratch, stream);
+    if ((err = round_smorph_gin<T>(s, g, ws, grad_in, stream)) != hipSuccess) return err;
+    return reduce(p);
 }
 
 // The smorph kernels' exponential, elementwise (a test probe of its bits).
@@ -913,76 +908,74 @@ hipError_t smorph_scm_backward(const T* x, const T* w, const T* alpha, const T* 
     if (workspace_bytes < smorph_scm_backward_workspace<T>(g)) return hipErrorInvalidValue;
     const SmorphBwdPlan s = plan_smorph_bwd<T>(MERGE_SMOOTH, g, pstats != nullptr);
     // The layout below is this plan's; never lay it out past the buffer.
-    if (workspace_bytes < smorph_plan_workspace<T>(s, g)) return hipErrorInvalidValue;
+    if (workspace_bytes < s.bytes) return hipErrorInvalidValue;
     const int64_t wnumel = (int64_t)g.Cout * g.Cw * g.taps();
-    if ((err = fill_async<T>(grad_in, (int64_t)g.B * g.Cin * g.plane(), T(0), stream)) != hipSuccess) return err;
     if ((int64_t)g.B * g.Cout * g.plane() == 0 || g.Cin == 0)
     {
+        if ((err = fill_async<T>(grad_in, (int64_t)g.B * g.Cin * g.plane(), T(0), stream)) != hipSuccess) return err;
         if ((err = fill_async<T>(grad_w, wnumel, T(0), stream)) != hipSuccess) return err;
         if ((err = fill_async<T>(grad_alpha, s.npairs, T(0), stream)) != hipSuccess) return err;
         return fill_async<T>(grad_beta, g.Cout, T(0), stream);
     }
     unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
-    T* part_w = reinterpret_cast<T*>(ws);
-    T* part_a = reinterpret_cast<T*>(ws + align_up(s.part_w_bytes));
-    T* part_b = reinterpret_cast<T*>(ws + align_up(s.part_w_bytes) + align_up(s.part_a_bytes));
-    Acc* gbuf = reinterpret_cast<Acc*>(ws + align_up(s.part_w_bytes) + align_up(s.part_a_bytes) + align_up(s.part_b_bytes));
-    T* scratch = reinterpret_cast<T*>(ws + align_up(s.part_w_bytes) + align_up(s.part_a_bytes) + align_up(s.part_b_bytes) +
-                                      align_up(s.gacc_bytes));
     const int nslots = g.B * s.nstrips;
-    const bool stat = smorph_static_supported<T>(g);
-    // The static kernel that keeps its partials in LDS stores every slot entry itself.
-    if (!(stat && smorph_bwd_lds_partials(g, false, true)))
-    {
-        if ((err = fill_async<T>(part_w, (int64_t)nslots * wnumel, T(0), stream)) != hipSuccess) return err;
-        if ((err = fill_async<T>(part_a, (int64_t)nslots * s.npairs, T(0), stream)) != hipSuccess) return err;
-        if ((err = fill_async<T>(part_b, (int64_t)nslots * g.Cin * g.Cout, T(0), stream)) != hipSuccess) return err;
-    }
-
-    SmorphBwdParams<T> p{};
-    p.x = x;
-    p.w = w;
-    p.alpha = alpha;
-    p.out = out;
-    p.gout = grad_out;
-    p.gin = grad_in;
-    p.part_w = part_w;
-    p.part_a = part_a;
-    p.beta = beta;
-    p.sstats = sstats;
-    p.part_b = part_b;
-    p.g = g;
-    p.t = s.t;
-    p.nstrips = s.nstrips;
-    p.tps = s.tps;
-    p.oslices = s.oslices;
-    p.oper = s.oper;
-    p.ncopy = s.ncopy;
-    p.npairs = s.npairs;
-    p.scale = T(1);
-    bool launched = false;
+    auto params = [&](auto zero) {
+        using PT = decltype(zero);
+        SmorphBwdParams<T, PT> p{};
+        p.x = x;
+        p.w = w;
+        p.alpha = alpha;
+        p.out = out;
+        p.gout = grad_out;
+        p.part_w = reinterpret_cast<PT*>(ws);
+        p.part_a = reinterpret_cast<PT*>(ws + s.part_a);
+        p.part_b = reinterpret_cast<PT*>(ws + s.part_b);
+        p.beta = beta;
+        p.sstats = sstats;
+        p.g = g;
+        p.t = s.t;
+        p.nstrips = s.nstrips;
+        p.tps = s.tps;
+        p.oslices = s.oslices;
+        p.oper = s.oper;
+        p.ncopy = s.ncopy;
+        p.npairs = s.npairs;
+        p.scale = T(1);
+        return p;
+    };
+    auto reduce = [&](const auto& p) {
+        auto* scratch = reinterpret_cast<decltype(p.part_w)>(ws + s.scratch);
+        hipError_t e = reduce_slots_async<T>(p.part_w, nslots, wnumel, grad_w, scratch, stream);
+        if (e == hipSuccess) e = reduce_slots_async<T>(p.part_a, nslots, s.npairs, grad_alpha, scratch, stream);
+        // grad_beta[o]: the partial rows [slot][i] summed in (slot, i) order.
+        return e != hipSuccess ? e : reduce_slots_async<T>(p.part_b, nslots * g.Cin, g.Cout, grad_beta, scratch, stream);
+    };
     if constexpr (sizeof(T) == 4)
-        if (stat)
+        if (smorph_static_supported<T>(g))
         {
             // The float32 static kernels: from the saved pair statistics (two rows per wave), or
             // recomputing them (one row per wave).
+            auto p = params(T(0));
+            p.gin = grad_in;
             p.pstats = pstats;
             p.nstat = smorph_stats_count<T>(MERGE_SMOOTH, g);
+            if ((err = fill_async<T>(grad_in, (int64_t)g.B * g.Cin * g.plane(), T(0), stream)) != hipSuccess) return err;
+            // The kernel that keeps its partials in LDS stores every slot entry itself.
+            if (!smorph_bwd_lds_partials(g, false, true))
+            {
+                if ((err = fill_async<T>(p.part_w, (int64_t)nslots * wnumel, T(0), stream)) != hipSuccess) return err;
+                if ((err = fill_async<T>(p.part_a, (int64_t)nslots * s.npairs, T(0), stream)) != hipSuccess) return err;
+                if ((err = fill_async<T>(p.part_b, (int64_t)nslots * g.Cin * g.Cout, T(0), stream)) != hipSuccess) return err;
+            }
             if ((err = launch_smorph_bwd_static(MK_SMOOTH, p, stream)) != hipSuccess) return err;
-            launched = true;
+            return reduce(p);
         }
-    if (!launched)
-    {
-        Acc* gacc = nullptr;
-        if ((err = prepare_gacc<T>(s, g, grad_in, gbuf, &gacc, stream)) != hipSuccess) return err;
-        p.gacc = gacc;
-        if ((err = launch_smorph_bwd_generic<T, MK_SMOOTH>(s, p, stream)) != hipSuccess) return err;
-        if ((err = finish_gacc<T>(s, g, gbuf, grad_in, stream)) != hipSuccess) return err;
-    }
-    if ((err = reduce_slots_async<T>(part_w, nslots, wnumel, grad_w, scratch, stream)) != hipSuccess) return err;
-    if ((err = reduce_slots_async<T>(part_a, nslots, s.npairs, grad_alpha, scratch, stream)) != hipSuccess) return err;
-    // grad_beta[o]: the partial rows [slot][i] summed in (slot, i) order.
-    return reduce_slots_async<T>(part_b, nslots * g.Cin, g.Cout, grad_beta, scratch, stream);
+    auto p = params(Acc(0));
+    p.gin = sizeof(T) == sizeof(Acc) ? reinterpret_cast<Acc*>(grad_in) : reinterpret_cast<Acc*>(ws + s.gacc);
+    if ((err = clear_smorph_sums<T>(s, g, ws, grad_in, stream)) != hipSuccess) return err;
+    if ((err = launch_smorph_bwd_generic<T, MK_SMOOTH>(s, p, stream)) != hipSuccess) return err;
+    if ((err = round_smorph_gin<T>(s, g, ws, grad_in, stream)) != hipSuccess) return err;
+    return reduce(p);
 }
 
 #define MCA_INSTANTIATE_SCM(T)                                                                                                           \

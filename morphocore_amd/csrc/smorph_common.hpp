@@ -188,7 +188,8 @@ __device__ __forceinline__ bool alpha_is_zero(float a)
     return (__builtin_amdgcn_readfirstlane(__builtin_bit_cast(unsigned, a)) & 0x7fffffffu) == 0u;
 }
 
-template <typename T>
+// PT: the type of the partial slots (the generic kernel's are double).
+template <typename T, typename PT = T>
 struct SmorphBwdParams
 {
     const T* __restrict__ x;
@@ -197,20 +198,17 @@ struct SmorphBwdParams
     const T* __restrict__ out;     // forward output (MAX / MIN)
     const T* __restrict__ counts;  // winner counts (MAX / MIN)
     const T* __restrict__ gout;
-    T* __restrict__ gin;
-    T* __restrict__ part_w;
-    T* __restrict__ part_a;
+    PT* __restrict__ gin;          // generic kernel: double sums, [B, Cin, H, W]
+    PT* __restrict__ part_w;
+    PT* __restrict__ part_a;
     const float* __restrict__ pstats;  // the forward's saved pair statistics, or null (recomputed)
     int64_t nstat;
-    // Generic kernel for elements whose tile and grad_input copy exceed the LDS: grad_input summed in
-    // global memory, [B, Cin, H, W] double (grad_input itself for double tensors), else null.
-    Acc* __restrict__ gacc;
     // SMOOTH merge (smorph_scm): beta per output channel, the forward's soft-merge statistics (ref,
     // then 1 / sum, [B, Cout, H, W] each; `out` holds the merged output), and the grad_beta partials
     // [slot][Cin][Cout].
     const T* __restrict__ beta;
     const T* __restrict__ sstats;
-    T* __restrict__ part_b;
+    PT* __restrict__ part_b;
     Geom g;
     Tiling t;
     int nstrips;
@@ -244,7 +242,7 @@ __device__ __forceinline__ double keep_if(double v, bool keep)
 // tap of the tile may read outside the image (else every tap is taken without a test). The element: wl, in LDS,
 // where KWS > 0, else wg, in global memory (restrict: by scalar loads). Rows that are not unrolled have no
 // other tap's chain to overlap: they branch around the exponentials no lane takes, which are most of them on
-// planes smaller than the tile (15x15 at (4, 86 -> 1, 8, 158), float32: 15.7 ms, 23.0 with all of them).
+// planes smaller than the tile (15x15 at (4, 86 -> 1, 8, 158), float32: 15.9 ms, 23.0 with all of them).
 template <typename T, int RH, int KWS, bool EDGE>
 __device__ __forceinline__ void smorph_pair_stats(const T* tbase, int pitch, const T* __restrict__ wg, const T* wl, T a, const Geom& g, int iy0,
                                                   int ix, T (&ref)[RH], T (&S)[RH], T (&Wsum)[RH])

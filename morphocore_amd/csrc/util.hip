@@ -35,8 +35,8 @@ __device__ __forceinline__ Acc sum_slots(const T* __restrict__ part, int s0, int
 
 // out[j] = sum over slots s = 0, 1, ... of part[s * n + j], always in slot order, accumulated in
 // double and rounded once.
-template <typename T>
-__global__ __launch_bounds__(BLOCK) void reduce_slots_kernel(const T* __restrict__ part, int nslots, int64_t n, T* __restrict__ out)
+template <typename T, typename PT>
+__global__ __launch_bounds__(BLOCK) void reduce_slots_kernel(const PT* __restrict__ part, int nslots, int64_t n, T* __restrict__ out)
 {
     for (int64_t j = (int64_t)blockIdx.x * BLOCK + threadIdx.x; j < n; j += (int64_t)gridDim.x * BLOCK)
         out[j] = (T)sum_slots(part, 0, nslots, n, j);
@@ -45,8 +45,8 @@ __global__ __launch_bounds__(BLOCK) void reduce_slots_kernel(const T* __restrict
 // The same sums in one launch for a few hundred slots: COLS consecutive columns per workgroup, each by
 // BLOCK / COLS threads that take every (BLOCK / COLS)-th slot; their sums are then added in thread order
 // (a fixed order, in double, rounded once).
-template <typename T, int COLS>
-__global__ __launch_bounds__(BLOCK) void reduce_joint_kernel(const T* __restrict__ part, int nslots, int64_t n, T* __restrict__ out)
+template <typename T, typename PT, int COLS>
+__global__ __launch_bounds__(BLOCK) void reduce_joint_kernel(const PT* __restrict__ part, int nslots, int64_t n, T* __restrict__ out)
 {
     constexpr int Q = BLOCK / COLS, U = 8;  // U loads in flight per thread
     __shared__ Acc sums[Q][COLS];
@@ -56,7 +56,7 @@ __global__ __launch_bounds__(BLOCK) void reduce_joint_kernel(const T* __restrict
     if (j < n)
         for (int b = q; b < nslots; b += U * Q)
         {
-            T v[U];
+            PT v[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) v[u] = part[(int64_t)min(b + u * Q, nslots - 1) * n + j];
 #pragma unroll
@@ -146,28 +146,28 @@ size_t reduce_slots_scratch(int nslots, int64_t n)
     return nslots > REDUCE_GROUP ? (size_t)((nslots + REDUCE_GROUP - 1) / REDUCE_GROUP) * (size_t)n * sizeof(T) : 0;
 }
 
-template <typename T>
-hipError_t reduce_slots_async(const T* part, int nslots, int64_t n, T* out, T* scratch, hipStream_t stream)
+template <typename T, typename PT>
+hipError_t reduce_slots_async(const PT* part, int nslots, int64_t n, T* out, PT* scratch, hipStream_t stream)
 {
     if (n <= 0) return hipSuccess;
     if (nslots <= REDUCE_GROUP)
     {
-        reduce_slots_kernel<T><<<grid_for(n), BLOCK, 0, stream>>>(part, nslots, n, out);
+        reduce_slots_kernel<T, PT><<<grid_for(n), BLOCK, 0, stream>>>(part, nslots, n, out);
         return hipGetLastError();
     }
     if (nslots <= JOINT_SLOTS)
     {
         // Few columns: 8 per workgroup, so that enough workgroups run.
         if (n < 16384)
-            reduce_joint_kernel<T, 8><<<(unsigned)((n + 7) / 8), BLOCK, 0, stream>>>(part, nslots, n, out);
+            reduce_joint_kernel<T, PT, 8><<<(unsigned)((n + 7) / 8), BLOCK, 0, stream>>>(part, nslots, n, out);
         else
-            reduce_joint_kernel<T, 32><<<(unsigned)((n + 31) / 32), BLOCK, 0, stream>>>(part, nslots, n, out);
+            reduce_joint_kernel<T, PT, 32><<<(unsigned)((n + 31) / 32), BLOCK, 0, stream>>>(part, nslots, n, out);
         return hipGetLastError();
     }
     const int groups = (nslots + REDUCE_GROUP - 1) / REDUCE_GROUP;
     const dim3 grid((unsigned)grid_for(n), (unsigned)groups);
-    reduce_groups_kernel<T><<<grid, BLOCK, 0, stream>>>(part, nslots, n, scratch);
-    reduce_slots_kernel<T><<<grid_for(n), BLOCK, 0, stream>>>(scratch, groups, n, out);
+    reduce_groups_kernel<PT><<<grid, BLOCK, 0, stream>>>(part, nslots, n, scratch);
+    reduce_slots_kernel<T, PT><<<grid_for(n), BLOCK, 0, stream>>>(scratch, groups, n, out);
     return hipGetLastError();
 }
 
@@ -240,7 +240,8 @@ template hipError_t fill_async<__bf16>(__bf16*, int64_t, __bf16, hipStream_t);
 template hipError_t fill_async<int32_t>(int32_t*, int64_t, int32_t, hipStream_t);
 template size_t reduce_slots_scratch<float>(int, int64_t);
 template size_t reduce_slots_scratch<double>(int, int64_t);
-template hipError_t reduce_slots_async<float>(const float*, int, int64_t, float*, float*, hipStream_t);
-template hipError_t reduce_slots_async<double>(const double*, int, int64_t, double*, double*, hipStream_t);
+template hipError_t reduce_slots_async<float, float>(const float*, int, int64_t, float*, float*, hipStream_t);
+template hipError_t reduce_slots_async<float, double>(const double*, int, int64_t, float*, double*, hipStream_t);
+template hipError_t reduce_slots_async<double, double>(const double*, int, int64_t, double*, double*, hipStream_t);
 
 }  // namespace mca

@@ -26,6 +26,7 @@ from morphocore_amd.functional.smorph import element, w_tilde  # noqa: E402
     (torch.float32, (1, 2, 4, 1, 70, 3, 7)),     # a plane of one row
     (torch.float32, (40, 8, 6, 8, 70, 5, 3)),    # enough tiles: one slice
     (torch.float64, (1, 2, 3, 20, 70, 6, 6)),    # not unrolled
+    (torch.float32, (1, 3, 2, 7, 21, 13, 13)),   # not unrolled, most taps outside the image
 ])
 def test_generic_kernels(dtype, shape, merge):
     B, Cin, Cout, H, W, KH, KW = shape
@@ -94,3 +95,45 @@ def test_element_keeps_strided_inputs_in_the_graph():
         seconds.append(torch.autograd.grad(sum(t.square().sum() for t in first), (v, a)))
     for got, want in zip(*seconds):
         assert normwise_error(got.cpu().numpy(), want.cpu().numpy()) <= 1e-12
+
+
+def _gradients(x, w, alpha, g):
+    xd, wd, ad = (t.cuda().requires_grad_() for t in (x, w, alpha))
+    torch.ops.morphocore.smorph(xd, wd, ad, O.MERGES["sum"]).backward(g.cuda())
+    return [t.grad.cpu().numpy() for t in (xd, wd, ad)]
+
+
+BIG = 1e4  # a float32 partial sum of this size loses 6e-4 of terms around 1; a double one 1e-12
+ONCE = 2.0 ** -22  # two results, each the double sum rounded once
+
+
+@pytest.mark.parametrize("KH,KW", [(9, 9), (6, 6)])
+def test_float32_grad_input_of_many_slices_is_rounded_once(KH, KW):
+    """Output channels in equal pairs with opposite large gradients cancel, whichever workgroups sum them:
+    grad_input is that of the two channels left, whose gradients are small."""
+    B, Cin, Cout, H, W = 1, 2, 258, 12, 40
+    x = seeded(81, B, Cin, H, W, kind="randn")
+    w = seeded(82, Cout, Cin, KH, KW, kind="randn", scale=0.2)
+    alpha = seeded(83, Cout, Cin, kind="randn", scale=2.0)
+    large = BIG * seeded(84, B, Cout - 2, H, W, kind="randn")
+    w[1:-2:2], alpha[1:-2:2], large[:, 1::2] = w[:-2:2], alpha[:-2:2], -large[:, ::2]
+    small = seeded(85, B, 2, H, W, kind="randn")
+    got = _gradients(x, w, alpha, torch.cat([large, small], 1))[0]
+    want = _gradients(x, w, alpha, torch.cat([torch.zeros_like(large), small], 1))[0]
+    assert normwise_error(got, want) <= ONCE
+
+
+@pytest.mark.parametrize("KH,KW", [(9, 9), (5, 3)])
+def test_float32_slots_of_many_tiles_are_rounded_once(KH, KW):
+    """Rows that see the same windows, in several tiles of one partial slot, with opposite large gradients
+    cancel: grad_weight and grad_alpha are those of the row between them."""
+    B, Cin, Cout, H, W = 128, 4, 1, 64, 40
+    x = seeded(86, B, Cin, 1, W, kind="randn").expand(B, Cin, H, W).contiguous()
+    w = seeded(87, Cout, Cin, KH, KW, kind="randn", scale=0.2)
+    alpha = seeded(88, Cout, Cin, kind="randn", scale=2.0)
+    small, large = torch.zeros(B, Cout, H, W), torch.zeros(B, Cout, H, W)
+    small[:, :, 38] = seeded(89, B, Cout, W, kind="randn")
+    large[:, :, 33] = BIG * seeded(90, B, Cout, W, kind="randn")
+    large[:, :, 46] = -large[:, :, 33]
+    for got, want in list(zip(_gradients(x, w, alpha, small + large), _gradients(x, w, alpha, small)))[1:]:
+        assert normwise_error(got, want) <= ONCE
