@@ -190,12 +190,13 @@ __global__ __launch_bounds__(BLOCK) void morpho_bwd_packed_kernel(const PackedPa
     }
 }
 
-template <typename T>
+// GT: the type grad_input is summed in across workgroups.
+template <typename T, typename GT = T>
 struct TapsParams
 {
     const void* __restrict__ taps;
     const T* __restrict__ gout;
-    T* __restrict__ gin;
+    GT* __restrict__ gin;
     T* __restrict__ part;
     Geom g;
     Tiling t;
@@ -217,8 +218,8 @@ __device__ __forceinline__ double keep_bits(double v, bool keep)
 
 // NI: channel pairs routed per step (IG input channels of one output channel; 1 for IDENTITY, whose
 // steps walk the group's channels).
-template <typename T, int OP, typename AT, bool IDENT, int RH, int NI>
-__global__ __launch_bounds__(BLOCK) void morpho_bwd_taps_kernel(const TapsParams<T> p)
+template <typename T, int OP, typename AT, bool IDENT, int RH, int NI, typename GT = T>
+__global__ __launch_bounds__(BLOCK) void morpho_bwd_taps_kernel(const TapsParams<T, GT> p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const Geom g = p.g;
@@ -374,7 +375,7 @@ __global__ __launch_bounds__(BLOCK) void morpho_bwd_taps_kernel(const TapsParams
     // with the neighbouring tiles' footprints: atomics onto the zero-filled gradient.
     for (int il = 0; il < ni; ++il)
     {
-        T* gplane = p.gin + ((int64_t)b * g.Cin + i0 + il) * plane;
+        GT* gplane = p.gin + ((int64_t)b * g.Cin + i0 + il) * plane;
         const Acc* gxl = gx + il * tile_elems;
         for (int ly = wave; ly < t.rows; ly += NWAVES)
         {
@@ -384,11 +385,11 @@ __global__ __launch_bounds__(BLOCK) void morpho_bwd_taps_kernel(const TapsParams
             {
                 const int ix = x0 + lx;
                 if (ix < 0 || ix >= g.W) continue;
-                const T v = (T)gxl[ly * t.pitch + lx];
+                const GT v = (GT)gxl[ly * t.pitch + lx];
                 const bool own = ly >= g.KH - 1 && ly < t.th && lx >= g.KW - 1 && lx < TILE_W;
                 if (own)
                     gplane[(int64_t)iy * g.W + ix] = v;
-                else if (v != T(0))
+                else if (v != GT(0))
                     global_add(&gplane[(int64_t)iy * g.W + ix], v);
             }
         }
@@ -722,7 +723,9 @@ static PackedPlan plan_packed(const Geom& g)
     return s;
 }
 
-// Rows per wave of the sum / mean taps kernel's small launches.
+// Rows per wave of the sum / mean taps kernel's small launches. Elements of 9 rows and more leave such a tile no row
+// of grad_input of its own (every pixel is the sum of two or three tiles), so float32 sums them in a double
+// buffer of the workspace, rounded once.
 constexpr int SMALL_TAPS_RH = 2;
 // Rows per wave of the IDENTITY gather kernel.
 constexpr int GATHER_RH = 4;
@@ -736,6 +739,8 @@ struct TapsPlan
     bool band;    // gathered by ident_band_gather (morpho_ident.hip): slots per (batch element, band)
     bool tile;    // ident_tile_backward (morpho_scatter.hip): slots per (batch element, tile)
     IdentTiles ident;  // its tiles, also for a chunk of the batch (the slots' layout)
+    bool small;   // morpho_bwd_taps_kernel in SMALL_TAPS_RH-row tiles
+    size_t gacc_bytes;  // float32's double grad_input sums of those
     size_t part_bytes;
     size_t lds;
 };
@@ -839,28 +844,28 @@ static TapsPlan plan_taps(int merge, const Geom& g, bool band_ok = true)
     }
     // Sum / mean launches of few workgroups take 8-row tiles and one input channel each instead (9x9 at
     // (4, 16 -> 24, 97, 131): 384 workgroups -> 2496).
-    // Their slots, four times as many, may not take a workspace past the fixed one of
-    // mca_morpho_backward_noalloc_f32 that the larger tiles' would fit.
+    // Their slots, four times as many, and grad_input sums may not take a workspace past the fixed one of
+    // mca_morpho_backward_noalloc_f32, which the larger tiles' may fit.
     if (!ident && (int64_t)g.B * s.t.ntiles() * ((g.Cin + 1) / 2) < 1024)
     {
         const Tiling t = make_tiling(g, SMALL_TAPS_RH);
         const size_t cells = (size_t)t.rows * t.pitch * sizeof(Acc);
         const size_t per_oc = K * 4 * sizeof(Acc);
         const int64_t wnumel = (int64_t)g.Cout * g.Cw * g.taps();
-        auto slots_bytes = [&](int ntiles) {
-            return align_up((size_t)g.B * ntiles * wnumel * sizeof(T)) + align_up(reduce_slots_scratch<T>(g.B * ntiles, wnumel));
-        };
-        const bool fits = slots_bytes(t.ntiles()) + recompute_workspace<T>(merge, g) <= MCA_NOALLOC_SCRATCH_BYTES ||
-                          slots_bytes(s.t.ntiles()) > MCA_NOALLOC_SCRATCH_BYTES;
-        if (cells + per_oc + table <= target && fits)
+        const int nslots = g.B * t.ntiles();
+        const size_t gacc = sizeof(T) == sizeof(Acc) ? 0 : (size_t)g.B * g.Cin * g.plane() * sizeof(Acc);
+        const size_t bytes = align_up((size_t)nslots * wnumel * sizeof(T)) + align_up(reduce_slots_scratch<T>(nslots, wnumel)) + align_up(gacc);
+        if (cells + per_oc + table <= target && bytes + recompute_workspace<T>(merge, g) <= MCA_NOALLOC_SCRATCH_BYTES)
         {
             s.t = t;
+            s.small = true;
+            s.gacc_bytes = gacc;
             s.ncopy = 4;
             s.ig = 1;
             s.nig = g.Cin;
             s.oc = std::max(1, std::min(g.Cout, (int)((target - cells - table) / per_oc)));
             s.lds = cells + (size_t)s.oc * per_oc + table;
-            s.part_bytes = (size_t)g.B * t.ntiles() * g.Cout * g.Cw * K * sizeof(T);
+            s.part_bytes = (size_t)nslots * wnumel * sizeof(T);
             return s;
         }
     }
@@ -976,6 +981,7 @@ size_t morpho_backward_workspace(int merge, bool has_indices, const Geom& g)
         const PackedPlan s = plan_packed<T>(g);
         if (!s.gather && !s.tile) bytes += align_up((size_t)g.B * g.Cin * g.plane() * sizeof(Acc));
     }
+    if (!packed_winners(merge)) bytes += align_up(plan_taps<T>(merge, g).gacc_bytes);
     return bytes;
 }
 
@@ -991,10 +997,12 @@ static hipError_t backward_op(int merge, bool replicate, T fill, const T* x, con
     const bool band_ok = band_aligned(grad_out, grad_in, indices);
     // The gather and tile kernels write every grad_input pixel themselves; the others accumulate onto zeros.
     const PackedPlan pp = plan_packed<T>(g);
-    const bool gather = nonempty && (packed ? pp.gather || pp.tile : plan_taps<T>(merge, g, band_ok).gather);
+    const TapsPlan s = packed ? TapsPlan{} : plan_taps<T>(merge, g, band_ok);
+    const bool gather = nonempty && (packed ? pp.gather || pp.tile : s.gather);
     const int64_t gin_n = (int64_t)g.B * g.Cin * g.plane();
-    // float32 max / min scatters round their double grad_input accumulator into every pixel at the end.
-    const bool rounded = packed && sizeof(T) != sizeof(Acc) && nonempty;
+    // float32 max / min scatters and small sum / mean launches round their double grad_input accumulator into
+    // every pixel at the end.
+    const bool rounded = (packed ? sizeof(T) != sizeof(Acc) : s.gacc_bytes > 0) && nonempty;
     if (!gather && !rounded)
         if ((err = fill_async<T>(grad_in, gin_n, T(0), stream)) != hipSuccess) return err;
     if ((int64_t)g.B * g.Cout * g.plane() == 0) return fill_async<T>(grad_w, wnumel, T(0), stream);
@@ -1054,7 +1062,13 @@ static hipError_t backward_op(int merge, bool replicate, T fill, const T* x, con
         return reduce_slots_async<T>(part, nslots, wnumel, grad_w, scratch, stream);
     }
 
-    const TapsPlan s = plan_taps<T>(merge, g, band_ok);
+    Acc* gacc = nullptr;
+    if (s.gacc_bytes > 0)
+    {
+        gacc = reinterpret_cast<Acc*>(ws);
+        ws += align_up(s.gacc_bytes);
+        if ((err = fill_async<Acc>(gacc, gin_n, Acc(0), stream)) != hipSuccess) return err;
+    }
     // Without saved taps, batch chunks: each chunk's taps recomputed into the workspace, then routed
     // into its own grad_input rows and partial slots (slots are per batch element and tile).
     const int chunk = indices ? g.B : recompute_batch<T>(merge, g);
@@ -1128,12 +1142,25 @@ static hipError_t backward_op(int merge, bool replicate, T fill, const T* x, con
             else
                 morpho_bwd_taps_kernel<T, OP, uint8_t, true, RH, 1><<<blocks, BLOCK, s.lds, stream>>>(p);
         }
-        else if (s.t.rh == SMALL_TAPS_RH)
+        else if (s.small)
         {
+            TapsParams<T, Acc> q{};
+            q.taps = p.taps;
+            q.gout = p.gout;
+            q.gin = (gacc ? gacc : reinterpret_cast<Acc*>(grad_in)) + (int64_t)b0 * g.Cin * plane;
+            q.part = p.part;
+            q.g = p.g;
+            q.t = p.t;
+            q.ig = p.ig;
+            q.nig = p.nig;
+            q.oc = p.oc;
+            q.ncopy_log2 = p.ncopy_log2;
+            q.kw_div = p.kw_div;
+            q.scale = p.scale;
             if (wide)
-                morpho_bwd_taps_kernel<T, OP, uint16_t, false, SMALL_TAPS_RH, 1><<<blocks, BLOCK, s.lds, stream>>>(p);
+                morpho_bwd_taps_kernel<T, OP, uint16_t, false, SMALL_TAPS_RH, 1, Acc><<<blocks, BLOCK, s.lds, stream>>>(q);
             else
-                morpho_bwd_taps_kernel<T, OP, uint8_t, false, SMALL_TAPS_RH, 1><<<blocks, BLOCK, s.lds, stream>>>(p);
+                morpho_bwd_taps_kernel<T, OP, uint8_t, false, SMALL_TAPS_RH, 1, Acc><<<blocks, BLOCK, s.lds, stream>>>(q);
         }
         else if (s.ig == 2)
         {
@@ -1151,6 +1178,8 @@ static hipError_t backward_op(int merge, bool replicate, T fill, const T* x, con
         }
         if ((err = hipGetLastError()) != hipSuccess) return err;
     }
+    if (gacc)
+        if ((err = round_async<T>(gacc, grad_in, gin_n, stream)) != hipSuccess) return err;
     return reduce_slots_async<T>(part, nslots, wnumel, grad_w, scratch, stream);
 }
 

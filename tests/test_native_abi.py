@@ -182,6 +182,18 @@ def test_smorph_workspace_covers_the_saved_statistics_plan(merge, geom):
     assert have >= _smorph_saved_plan_bytes(merge, B, C, C, H, W, K)
 
 
+def test_small_taps_launches_keep_the_workspace_bounded():
+    """Sum / mean launches of few workgroups take 8-row tiles (four times the partial slots of 32-row ones)
+    only where that workspace fits the no-allocation backward's scratch: an element of 25 x 25 taps and
+    64 x 64 channels keeps its 28 slots of 10 MB."""
+    lib = _native.lib()
+    slots, wnumel = 4 * 7, 64 * 64 * 25 * 25
+    assert lib.mca_morpho_backward_workspace_size_f32(2, 1, 1, 64, 64, 64, 128, 448, 25, 25) == slots * wnumel * 4
+    # Within it: 16 tiles of 8 rows, and the double grad_input sums.
+    need = 2 * 13 * 3 * 81 * 16 * 24 * 4
+    assert need < lib.mca_morpho_backward_workspace_size_f32(2, 1, 2, 16, 24, 16, 97, 131, 9, 9) <= _native.NOALLOC_SCRATCH_BYTES
+
+
 def test_noalloc_backward_rejects_problems_beyond_its_scratch():
     """The no-allocation backward refuses, before any device work, a problem whose workspace exceeds
     the library's per-GPU scratch (here: configs[4]'s first layer without saved winners)."""
