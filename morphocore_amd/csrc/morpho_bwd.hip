@@ -97,20 +97,14 @@ __device__ __forceinline__ Acc packed_gather_pixel(const PackedParams<T, ST>& p,
     return s;
 }
 
-// Planes of fewer pixels are walked across batch elements (one at a time they leave lanes, and the loads in flight,
-// idle): backward of 3x3 at (1949, 5 -> 8, 4, 4) 21 us, 80 plane by plane.
-constexpr int FLAT_PLANE = 4 * BLOCK;
-
-// WONLY: grad_weight alone (grad_input by packed_tile_backward). Its unrolled loads are not part of the other
-// form, whose gathering workgroups they slow down (5x5 at (1, 3 -> 5, 259, 316) 54 -> 60 us).
-template <typename T, int OP, typename ST, bool WONLY>
+template <typename T, int OP, typename ST = T>
 __global__ __launch_bounds__(BLOCK) void morpho_bwd_packed_kernel(const PackedParams<T, ST> p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     Acc* bins = reinterpret_cast<Acc*>(smem_raw);
     const Geom g = p.g;
     const int work = xcd_work_index(blockIdx.x, gridDim.x);
-    if (!WONLY && work >= p.wblocks)
+    if (work >= p.wblocks)
     {
         // Gathering workgroup: each pixel's slots, then their sum in slot order (deterministic).
         __shared__ Acc slot_sums[BLOCK];
@@ -150,76 +144,43 @@ __global__ __launch_bounds__(BLOCK) void morpho_bwd_packed_kernel(const PackedPa
         else
             global_add(&part[(int64_t)c * K + k], sign * gv);
     };
-    if constexpr (!WONLY)
+    // The chunk's pixels batch element by batch element: contiguous winners and gradients.
+    for (int64_t b = n_begin / plane; b * plane < n_end; ++b)
     {
-        for (int64_t n = n_begin + threadIdx.x; n < n_end; n += BLOCK)
+        const int64_t q0 = (b * g.Cout + o) * plane;
+        const int64_t lo = max(n_begin - b * plane, (int64_t)0), hi = min(n_end - b * plane, plane);
+        if (!p.gin)
         {
-            const int64_t b = n / plane;
-            const int64_t pix = n - b * plane;
-            const int64_t q = (b * g.Cout + o) * plane + pix;
-            const T gv = (T)p.gout[q];
-            if (gv == T(0)) continue;
-            const int32_t packed = p.idx[q];
-            if (p.gin)
-            {
-                const int h = (int)(pix / g.W), wc = (int)(pix - (int64_t)h * g.W);
-                const int c = packed >> 16, k = packed & 0xFFFF;
-                const int kh = k / g.KW, kw = k - kh * g.KW;
-                const int iy = h + ph - kh, ix = wc + pw - kw;
-                if (iy >= 0 && iy < g.H && ix >= 0 && ix < g.W) global_add(&p.gin[(b * g.Cin + c) * plane + (int64_t)iy * g.W + ix], (Acc)gv);
-            }
-            add_weight(packed, gv);
-        }
-    }
-    else
-    {
-        constexpr int U = 4;  // pixels whose loads are in flight together
-        if (plane >= FLAT_PLANE || p.chunk > 0x3fffffff)
-        {
-            // The chunk's pixels batch element by batch element: contiguous winners and gradients.
-            for (int64_t b = n_begin / plane; b * plane < n_end; ++b)
-            {
-                const int64_t q0 = (b * g.Cout + o) * plane;
-                const int64_t lo = max(n_begin - b * plane, (int64_t)0), hi = min(n_end - b * plane, plane);
-                for (int64_t pix = lo + threadIdx.x; pix < hi; pix += U * BLOCK)
-                {
-                    int32_t packed[U];
-                    T gv[U];
-#pragma unroll
-                    for (int u = 0; u < U; ++u)
-                    {
-                        const int64_t q = q0 + min(pix + u * BLOCK, hi - 1);
-                        packed[u] = p.idx[q];
-                        gv[u] = (T)p.gout[q];
-                    }
-#pragma unroll
-                    for (int u = 0; u < U; ++u)
-                        if (pix + u * BLOCK < hi && gv[u] != T(0)) add_weight(packed[u], gv[u]);
-                }
-            }
-        }
-        else if (n_begin < n_end)
-        {
-            // Across batch elements (pixel numbers from the chunk's first one's, in 32 bits).
-            const int64_t b0 = n_begin / plane;
-            const unsigned hi = (unsigned)(n_end - b0 * plane), up = (unsigned)plane;
-            const int64_t q0 = (b0 * g.Cout + o) * plane, skip = (int64_t)(g.Cout - 1) * plane;
-            for (unsigned n = (unsigned)(n_begin - b0 * plane) + threadIdx.x; n < hi; n += U * BLOCK)
+            // grad_weight alone: four pixels' loads in flight together.
+            constexpr int U = 4;
+            for (int64_t pix = lo + threadIdx.x; pix < hi; pix += U * BLOCK)
             {
                 int32_t packed[U];
                 T gv[U];
 #pragma unroll
                 for (int u = 0; u < U; ++u)
                 {
-                    const unsigned m = min(n + u * BLOCK, hi - 1);
-                    const int64_t q = q0 + m + (m / up) * skip;
+                    const int64_t q = q0 + min(pix + u * BLOCK, hi - 1);
                     packed[u] = p.idx[q];
                     gv[u] = (T)p.gout[q];
                 }
 #pragma unroll
                 for (int u = 0; u < U; ++u)
-                    if (n + u * BLOCK < hi && gv[u] != T(0)) add_weight(packed[u], gv[u]);
+                    if (pix + u * BLOCK < hi && gv[u] != T(0)) add_weight(packed[u], gv[u]);
             }
+            continue;
+        }
+        for (int64_t pix = lo + threadIdx.x; pix < hi; pix += BLOCK)
+        {
+            const T gv = (T)p.gout[q0 + pix];
+            if (gv == T(0)) continue;
+            const int32_t packed = p.idx[q0 + pix];
+            const int h = (int)(pix / g.W), wc = (int)(pix - (int64_t)h * g.W);
+            const int c = packed >> 16, k = packed & 0xFFFF;
+            const int kh = k / g.KW, kw = k - kh * g.KW;
+            const int iy = h + ph - kh, ix = wc + pw - kw;
+            if (iy >= 0 && iy < g.H && ix >= 0 && ix < g.W) global_add(&p.gin[(b * g.Cin + c) * plane + (int64_t)iy * g.W + ix], (Acc)gv);
+            add_weight(packed, gv);
         }
     }
     if (p.lds_bins)
@@ -766,9 +727,6 @@ static PackedPlan plan_packed(const Geom& g)
 // of grad_input of its own (every pixel is the sum of two or three tiles), so float32 sums them in a double
 // buffer of the workspace, rounded once.
 constexpr int SMALL_TAPS_RH = 2;
-// Below this many workgroups of the larger tiles: fewer than the CUs, or, where their LDS leaves the bins of a single
-// output channel (float32 9x9: every channel flushes), up to SMALL_GRID's.
-constexpr int64_t SMALL_TAPS_GRID = 192, SMALL_TAPS_GRID_ONE = 1024;
 // Rows per wave of the IDENTITY gather kernel.
 constexpr int GATHER_RH = 4;
 
@@ -884,31 +842,11 @@ static TapsPlan plan_taps(int merge, const Geom& g, bool band_ok = true)
             return s;
         }
     }
-    auto need = [&](int ig, int oc, int ncopy) { return ig * tile + (size_t)oc * ig * K * ncopy * sizeof(Acc) + table; };
-    s.ncopy = 4;
-    s.ig = ident ? 4 : 2;
-    while (s.ig > 1 && s.ig > g.Cin) s.ig /= 2;
-    while (s.ig > 1 && need(s.ig, 1, s.ncopy) > target) s.ig /= 2;
-    while (s.ncopy > 1 && need(s.ig, 1, s.ncopy) > LDS_LIMIT) s.ncopy /= 2;
-    if (ident)
-    {
-        s.oc = 1;
-    }
-    else
-    {
-        const size_t budget = need(s.ig, 1, s.ncopy) <= target ? target : LDS_LIMIT;
-        const size_t per_oc = (size_t)s.ig * K * s.ncopy * sizeof(Acc);
-        const size_t fixed = s.ig * tile + table;
-        s.oc = budget > fixed ? (int)((budget - fixed) / per_oc) : 1;
-        if (s.oc > g.Cout) s.oc = g.Cout;
-        if (s.oc < 1) s.oc = 1;
-    }
-    s.nig = (g.Cin + s.ig - 1) / s.ig;
-    s.lds = need(s.ig, s.oc, s.ncopy);
-    // Sum / mean launches of few workgroups take 8-row tiles and one input channel each instead.
+    // Sum / mean launches of few workgroups take 8-row tiles and one input channel each instead (9x9 at
+    // (4, 16 -> 24, 97, 131): 384 workgroups -> 2496).
     // Their slots, four times as many, and grad_input sums may not take a workspace past the fixed one of
     // mca_morpho_backward_noalloc_f32, which the larger tiles' may fit.
-    if (!ident && (int64_t)g.B * s.t.ntiles() * s.nig < (s.oc == 1 && g.Cout > 1 ? SMALL_TAPS_GRID_ONE : SMALL_TAPS_GRID))
+    if (!ident && (int64_t)g.B * s.t.ntiles() * ((g.Cin + 1) / 2) < 1024)
     {
         const Tiling t = make_tiling(g, SMALL_TAPS_RH);
         const size_t cells = (size_t)t.rows * t.pitch * sizeof(Acc);
@@ -931,6 +869,27 @@ static TapsPlan plan_taps(int merge, const Geom& g, bool band_ok = true)
             return s;
         }
     }
+    auto need = [&](int ig, int oc, int ncopy) { return ig * tile + (size_t)oc * ig * K * ncopy * sizeof(Acc) + table; };
+    s.ncopy = 4;
+    s.ig = ident ? 4 : 2;
+    while (s.ig > 1 && s.ig > g.Cin) s.ig /= 2;
+    while (s.ig > 1 && need(s.ig, 1, s.ncopy) > target) s.ig /= 2;
+    while (s.ncopy > 1 && need(s.ig, 1, s.ncopy) > LDS_LIMIT) s.ncopy /= 2;
+    if (ident)
+    {
+        s.oc = 1;
+    }
+    else
+    {
+        const size_t budget = need(s.ig, 1, s.ncopy) <= target ? target : LDS_LIMIT;
+        const size_t per_oc = (size_t)s.ig * K * s.ncopy * sizeof(Acc);
+        const size_t fixed = s.ig * tile + table;
+        s.oc = budget > fixed ? (int)((budget - fixed) / per_oc) : 1;
+        if (s.oc > g.Cout) s.oc = g.Cout;
+        if (s.oc < 1) s.oc = 1;
+    }
+    s.nig = (g.Cin + s.ig - 1) / s.ig;
+    s.lds = need(s.ig, s.oc, s.ncopy);
     return s;
 }
 
@@ -1093,8 +1052,7 @@ static hipError_t backward_op(int merge, bool replicate, T fill, const T* x, con
         p.lds_bins = s.lds_bins ? 1 : 0;
         p.chunk = s.chunk;
         p.wblocks = s.nchunks * g.Cout;
-        const auto kernel = s.tile ? morpho_bwd_packed_kernel<T, OP, T, true> : morpho_bwd_packed_kernel<T, OP, T, false>;
-        kernel<<<(unsigned)((int64_t)p.wblocks + s.gblocks), BLOCK, s.lds, stream>>>(p);
+        morpho_bwd_packed_kernel<T, OP><<<(unsigned)((int64_t)p.wblocks + s.gblocks), BLOCK, s.lds, stream>>>(p);
         if ((err = hipGetLastError()) != hipSuccess) return err;
         if (s.tile)
             if ((err = packed_tile_backward<T, T>(p.idx, grad_out, grad_in, g, stream)) != hipSuccess) return err;
@@ -1296,8 +1254,7 @@ static hipError_t half_direct(int merge, const void* indices, const ST* grad_out
         p.lds_bins = s.lds_bins ? 1 : 0;
         p.chunk = s.chunk;
         p.wblocks = s.nchunks * g.Cout;
-        const auto kernel = s.tile ? morpho_bwd_packed_kernel<float, OP, ST, true> : morpho_bwd_packed_kernel<float, OP, ST, false>;
-        kernel<<<(unsigned)((int64_t)p.wblocks + s.gblocks), BLOCK, s.lds, stream>>>(p);
+        morpho_bwd_packed_kernel<float, OP, ST><<<(unsigned)((int64_t)p.wblocks + s.gblocks), BLOCK, s.lds, stream>>>(p);
         if ((err = hipGetLastError()) != hipSuccess) return err;
         if (s.tile)
             if ((err = packed_tile_backward<float, ST>(p.idx, grad_out, grad_in, g, stream)) != hipSuccess) return err;
