@@ -400,10 +400,16 @@ struct StaticTile
 // global memory, which costs fewer staging passes than it saves.
 constexpr int BUCKET_MIN_TAPS = 25;
 constexpr int BUCKET_MAX_CIN = 256;
-// A workgroup of one output channel sorts only up to this many input channels: its few items share too
-// little of each staged tile. Bucket against per-pixel rescan (us): 7x7 at (8, 64 -> 3, 256, 256) 422 / 319,
-// at (8, 3 -> 3, 512, 512) 150 / 229; 5x5 at (4, 8 -> 8, 128, 128) 23.2 / 23.4.
-constexpr int BUCKET_MAX_CIN_ONE = 8;
+// A workgroup of one output channel sorts only a few input channels, whose staged tiles its few pixels share:
+// two a row per wave (one of 5x5, whose per-pixel rescan is short). Time of the per-pixel rescan over that of
+// the bucket, medians of small launches at 2-3, 4-7, 8-15 and 16-31 input channels: 4 rows, 5x5 1.38 1.03 0.87
+// 0.71, 7x7 1.68 1.17 1.01 0.79, 9x9 1.71 1.33 1.05 0.86, 11x11 1.64 1.38 1.11 0.88; 2 rows, 5x5 1.09 0.87 0.70
+// 0.58, 7x7 1.28 0.97 0.79 0.66, 9x9 1.37 1.03 0.85 0.71, 11x11 1.44 1.07 0.89 0.77.
+template <int RH, int K>
+constexpr int bucket_max_cin_one()
+{
+    return K == 25 ? RH : 2 * RH;
+}
 
 // Structuring-element values of the workgroup's OB output channels for one input channel, staged
 // with the input tile and read by every lane at the same LDS address (a broadcast).
@@ -709,7 +715,7 @@ morpho_fwd_static(const FwdParams<ST> p)
 
     if constexpr (BUCKET)
     {
-        if (g.Cin >= 1 && g.Cin <= (OB > 1 ? BUCKET_MAX_CIN : BUCKET_MAX_CIN_ONE))
+        if (g.Cin >= 1 && g.Cin <= (OB > 1 ? BUCKET_MAX_CIN : bucket_max_cin_one<RH, K>()))
         {
             // The winning tap of every output pixel, found channel by channel from LDS instead of one
             // lane at a time from global memory (whose scattered loads, one plane per lane, bound the
@@ -925,13 +931,32 @@ static hipError_t launch_generic(FwdParams<ST> p, hipStream_t stream)
 // Below this many workgroups of the full shape (RH rows per wave, OB output channels) the chip is mostly
 // idle and every workgroup's serial latency (its channel loop, the winner rescans of its pixels) is the
 // kernel time: such launches take one output channel per workgroup and 4, 2 or 1 rows per wave, the
-// most that leaves MEDIUM_GRID (4 rows) or TWO_ROW_GRID (2) workgroups. More rows per wave share each LDS
-// read of the window and of the element; fewer make more workgroups. Measured (us), values only:
-// 7x7 at (4, 8 -> 8, 128, 128): 4 rows (512 workgroups) 18.8, 2 (1024) 20.6, 1 (2048) 30.4; 5x5 at
-// (2, 32 -> 32, 64, 64): 4 (256) 34.4, 2 (512) 27.2, 1 (1024) 35.9; (1, 16 -> 16, 64, 64): 4 (64) 17.8,
-// 2 (128) 12.9, 1 (256) 10.6; 11x11 at (1, 51 -> 51, 32, 28): 4 (102) 193, 2 (204) 117, 1 (408) 119.
+// most that leaves small_rows().four or .two workgroups and no wave without rows. More rows per wave share each LDS read of the window and
+// of the element; fewer make more workgroups, and keep fewer windows in registers where every tap is tracked
+// (11x11 is faster by one row at every size).
 constexpr int64_t SMALL_GRID = 1024;
-constexpr int64_t MEDIUM_GRID = 448, TWO_ROW_GRID = 192;
+
+struct SmallRows
+{
+    int64_t four, two;  // workgroups from which 4 and 2 rows per wave are taken
+};
+
+// Measured over 1100 random launches below SMALL_GRID (3x3 to 11x11, float32 and bfloat16): time over that of the
+// best of the three, geometric mean, by these limits | by one row always:
+// values 1.006 | 1.21, identity values 1.005 | 1.13, max / min winners 1.01 | 1.16, taps 1.01 | 1.02,
+// identity taps 1.01 | 1.05. Float32 (us, at 4, 2, 1 rows): values, 7x7 at (4, 8 -> 8, 128, 128) 18.8 20.6 30.4 (512,
+// 1024, 2048 workgroups), 5x5 at (1, 16 -> 16, 64, 64) 17.8 12.9 10.6 (64, 128, 256); taps, 7x7 at
+// (2, 11 -> 38, 94, 14) 35.4 36.1 43.2 (456, 912, 1824), 9x9 at (11, 5 -> 6, 19, 162) 26.9 22.0 19.3
+// (396, 594, 990), 11x11 at (5, 28 -> 8, 60, 75) 186 187 157 (320, 640, 1200).
+template <int MODE, int KS>
+constexpr SmallRows small_rows()
+{
+    constexpr int64_t never = INT64_MAX;
+    if (MODE == FWD_TAPS) return KS <= 5 ? SmallRows{640, 384} : (KS <= 9 ? SmallRows{never, 512} : SmallRows{never, never});
+    if (MODE == FWD_PACKED) return KS <= 5 ? SmallRows{768, 512} : SmallRows{640, 256};
+    return SmallRows{448, KS == 3 ? 384 : 192};
+}
+
 constexpr int IDENT_CHANS = 8;
 
 template <typename ST, int OP, int MK, int OB, int MODE, int KS>
@@ -957,15 +982,21 @@ static hipError_t launch_static(FwdParams<ST> p, hipStream_t stream)
                 p.t = make_tiling(p.g, rh);
                 return blocks = (int64_t)p.g.B * p.t.nty * p.t.ntx * p.nog;
             };
-            if (with_rows(RH) >= MEDIUM_GRID)
-                morpho_fwd_static<ST, OP, MK, KS, KS, 1, RH, MODE><<<(unsigned)blocks, BLOCK, 0, stream>>>(p);
-            else if (with_rows(2) >= TWO_ROW_GRID)
-                morpho_fwd_static<ST, OP, MK, KS, KS, 1, 2, MODE><<<(unsigned)blocks, BLOCK, 0, stream>>>(p);
-            else
-            {
-                with_rows(1);
-                morpho_fwd_static<ST, OP, MK, KS, KS, 1, 1, MODE><<<(unsigned)blocks, BLOCK, 0, stream>>>(p);
-            }
+            constexpr SmallRows rows = small_rows<MODE, KS>();
+            if constexpr (rows.four < INT64_MAX)
+                if (p.g.H > NWAVES * RH / 2 && with_rows(RH) >= rows.four)
+                {
+                    morpho_fwd_static<ST, OP, MK, KS, KS, 1, RH, MODE><<<(unsigned)blocks, BLOCK, 0, stream>>>(p);
+                    return hipGetLastError();
+                }
+            if constexpr (rows.two < INT64_MAX)
+                if (p.g.H > NWAVES && with_rows(2) >= rows.two)
+                {
+                    morpho_fwd_static<ST, OP, MK, KS, KS, 1, 2, MODE><<<(unsigned)blocks, BLOCK, 0, stream>>>(p);
+                    return hipGetLastError();
+                }
+            with_rows(1);
+            morpho_fwd_static<ST, OP, MK, KS, KS, 1, 1, MODE><<<(unsigned)blocks, BLOCK, 0, stream>>>(p);
             return hipGetLastError();
         }
     }

@@ -61,6 +61,37 @@ def test_forward_shapes(K, shape, op, merge, padding):
     assert normwise_error(wd.grad.cpu().numpy(), gw) <= TOL[torch.float32]
 
 
+@pytest.mark.parametrize("K,merge,Cin", [(3, "max", 3), (5, "min", 4), (5, "max", 5), (7, "max", 8), (9, "min", 9), (11, "max", 4), (3, "sum", 3), (5, "mean", 2),
+                                         (7, "sum", 2), (9, "mean", 2), (11, "sum", 2), (3, "identity", 0), (7, "identity", 0)])
+@pytest.mark.parametrize("B,Cout,H,W", [
+    (7, 14, 33, 60),   # 294 workgroups of four rows, 490 of two
+    (13, 14, 30, 60),  # 364 and 728
+    (12, 30, 40, 30),  # 1080 and 1800
+    (90, 9, 8, 20),    # 810 of two rows; four would leave waves without rows
+    (90, 9, 4, 20),    # planes of four rows: one row per wave
+    (16, 3, 60, 200),  # three output channels: one per workgroup in the full shape too
+])
+def test_saving_forward_shapes(K, merge, Cin, B, Cout, H, W):
+    """Rows per wave of the launches that save winners or taps, and the input channels up to which one output
+    channel's winners are sorted (two a row per wave, one of 5x5): values and gradients."""
+    Cin = Cin or Cout
+    Cw = 1 if merge == "identity" else Cin
+    x = seeded(51, B, Cin, H, W, kind="quant") - 0.5
+    w = (seeded(52, Cout, Cw, K, K, kind="quant") * 4).round() / 4 - 0.5
+    g = seeded(53, B, Cout, H, W, kind="randn")
+    m = O.MERGES[merge]
+    packed = merge in ("max", "min")
+    ref, idx = O.morpho_forward(0, m, O.REPLICATE, 0.0, x.numpy(), w.numpy(), save_indices=packed)
+    xd, wd = x.cuda().requires_grad_(), w.cuda().requires_grad_()
+    out = torch.ops.morphocore.dilation(xd, wd, m, O.REPLICATE, 0.0, True, 0.0)
+    got = out.detach().cpu().numpy()
+    assert np.array_equal(got, ref) and np.array_equal(np.signbit(got), np.signbit(ref))
+    out.backward(g.cuda())
+    gx, gw = O.morpho_backward(0, m, O.REPLICATE, 0.0, x.numpy(), w.numpy(), g.numpy(), indices=idx if packed else None)
+    assert normwise_error(xd.grad.cpu().numpy(), gx) <= TOL[torch.float32]
+    assert normwise_error(wd.grad.cpu().numpy(), gw) <= TOL[torch.float32]
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("padding", ["geodesic", "replicate"])
 def test_sixteen_bit_staging(dtype, padding):
