@@ -641,18 +641,14 @@ morpho_fwd_static(const FwdParams<ST> p)
         else
         {
             // Values only: the order of the taps does not matter, so one column of the window is
-            // live at a time (kw outer) and pairs of taps fold into one max3 / min3; a column's odd tap
-            // waits for the next column's (3x3: 5 slow operations per window instead of 6; larger
-            // elements lose a wave per SIMD to the waiting values).
-            constexpr bool CARRY = K == 9;
-            T best[OB][RH], odd[OB][RH];
-            // The start value in a register: max3 / min3 take no infinity as a literal.
-            T start = Tr::init();
-            if constexpr (CARRY) asm volatile("" : "+v"(start));
+            // live at a time (kw outer) and pairs of taps fold into one max3 / min3. (A column's odd tap
+            // kept for the next column's, one operation less per 3x3 window, takes 16 registers more and
+            // with them a wave per SIMD: 3x3 max at (256, 32 -> 32, 16, 16) 115 us instead of 107.)
+            T best[OB][RH];
 #pragma unroll
             for (int ob = 0; ob < OB; ++ob)
 #pragma unroll
-                for (int r = 0; r < RH; ++r) best[ob][r] = start;
+                for (int r = 0; r < RH; ++r) best[ob][r] = Tr::init();
 #pragma unroll
             for (int kw = 0; kw < KW; ++kw)
             {
@@ -675,16 +671,7 @@ morpho_fwd_static(const FwdParams<ST> p)
                         for (int kh = 0; kh + 1 < KH; kh += 2)
                             m = Tr::pick(m, Tr::pick(Tr::combine(col[r + KH - 1 - kh], wp[kh * KW + kw]),
                                                      Tr::combine(col[r + KH - 2 - kh], wp[(kh + 1) * KW + kw])));
-                        if constexpr (KH % 2 == 1)
-                        {
-                            const T v = Tr::combine(col[r], wp[(KH - 1) * KW + kw]);
-                            if (!CARRY || kw == KW - 1)
-                                m = Tr::pick(m, v);
-                            else if (kw % 2 == 0)
-                                odd[ob][r] = v;
-                            else
-                                m = Tr::pick(m, Tr::pick(odd[ob][r], v));
-                        }
+                        if constexpr (KH % 2 == 1) m = Tr::pick(m, Tr::combine(col[r], wp[(KH - 1) * KW + kw]));
                         best[ob][r] = m;
                     }
                 }
