@@ -727,6 +727,12 @@ static PackedPlan plan_packed(const Geom& g)
 // of grad_input of its own (every pixel is the sum of two or three tiles), so float32 sums them in a double
 // buffer of the workspace, rounded once.
 constexpr int SMALL_TAPS_RH = 2;
+// Taken below this many workgroups of the larger tiles: fewer than the CUs, or, where those tiles leave LDS for the
+// bins of one output channel only and flush after each (float32 9x9), more. Backward (us, larger tiles | these):
+// 9x9 at (3, 8 -> 20, 220, 80) 106 | 65 (168 workgroups) and (2, 16 -> 25, 102, 257) 174 | 107 (320); 11x11 at
+// (1, 10 -> 14, 156, 71) 39 | 27 (100) and (1, 17 -> 5, 137, 79) 26 | 20 (170), but (1, 25 -> 5, 213, 203) 41 | 52
+// (700) and (2, 21 -> 6, 239, 69) 39 | 50 (672); 17x17 at (1, 4 -> 9, 142, 152) 38 | 24 (60).
+constexpr int64_t SMALL_TAPS_GRID = 192, SMALL_TAPS_GRID_ONE = 1024;
 // Rows per wave of the IDENTITY gather kernel.
 constexpr int GATHER_RH = 4;
 
@@ -842,11 +848,31 @@ static TapsPlan plan_taps(int merge, const Geom& g, bool band_ok = true)
             return s;
         }
     }
-    // Sum / mean launches of few workgroups take 8-row tiles and one input channel each instead (9x9 at
-    // (4, 16 -> 24, 97, 131): 384 workgroups -> 2496).
+    auto need = [&](int ig, int oc, int ncopy) { return ig * tile + (size_t)oc * ig * K * ncopy * sizeof(Acc) + table; };
+    s.ncopy = 4;
+    s.ig = ident ? 4 : 2;
+    while (s.ig > 1 && s.ig > g.Cin) s.ig /= 2;
+    while (s.ig > 1 && need(s.ig, 1, s.ncopy) > target) s.ig /= 2;
+    while (s.ncopy > 1 && need(s.ig, 1, s.ncopy) > LDS_LIMIT) s.ncopy /= 2;
+    if (ident)
+    {
+        s.oc = 1;
+    }
+    else
+    {
+        const size_t budget = need(s.ig, 1, s.ncopy) <= target ? target : LDS_LIMIT;
+        const size_t per_oc = (size_t)s.ig * K * s.ncopy * sizeof(Acc);
+        const size_t fixed = s.ig * tile + table;
+        s.oc = budget > fixed ? (int)((budget - fixed) / per_oc) : 1;
+        if (s.oc > g.Cout) s.oc = g.Cout;
+        if (s.oc < 1) s.oc = 1;
+    }
+    s.nig = (g.Cin + s.ig - 1) / s.ig;
+    s.lds = need(s.ig, s.oc, s.ncopy);
+    // Sum / mean launches of few workgroups take 8-row tiles and one input channel each instead.
     // Their slots, four times as many, and grad_input sums may not take a workspace past the fixed one of
     // mca_morpho_backward_noalloc_f32, which the larger tiles' may fit.
-    if (!ident && (int64_t)g.B * s.t.ntiles() * ((g.Cin + 1) / 2) < 1024)
+    if (!ident && (int64_t)g.B * s.t.ntiles() * s.nig < (s.oc == 1 && g.Cout > 1 ? SMALL_TAPS_GRID_ONE : SMALL_TAPS_GRID))
     {
         const Tiling t = make_tiling(g, SMALL_TAPS_RH);
         const size_t cells = (size_t)t.rows * t.pitch * sizeof(Acc);
@@ -869,27 +895,6 @@ static TapsPlan plan_taps(int merge, const Geom& g, bool band_ok = true)
             return s;
         }
     }
-    auto need = [&](int ig, int oc, int ncopy) { return ig * tile + (size_t)oc * ig * K * ncopy * sizeof(Acc) + table; };
-    s.ncopy = 4;
-    s.ig = ident ? 4 : 2;
-    while (s.ig > 1 && s.ig > g.Cin) s.ig /= 2;
-    while (s.ig > 1 && need(s.ig, 1, s.ncopy) > target) s.ig /= 2;
-    while (s.ncopy > 1 && need(s.ig, 1, s.ncopy) > LDS_LIMIT) s.ncopy /= 2;
-    if (ident)
-    {
-        s.oc = 1;
-    }
-    else
-    {
-        const size_t budget = need(s.ig, 1, s.ncopy) <= target ? target : LDS_LIMIT;
-        const size_t per_oc = (size_t)s.ig * K * s.ncopy * sizeof(Acc);
-        const size_t fixed = s.ig * tile + table;
-        s.oc = budget > fixed ? (int)((budget - fixed) / per_oc) : 1;
-        if (s.oc > g.Cout) s.oc = g.Cout;
-        if (s.oc < 1) s.oc = 1;
-    }
-    s.nig = (g.Cin + s.ig - 1) / s.ig;
-    s.lds = need(s.ig, s.oc, s.ncopy);
     return s;
 }
 
