@@ -97,14 +97,20 @@ __device__ __forceinline__ Acc packed_gather_pixel(const PackedParams<T, ST>& p,
     return s;
 }
 
-template <typename T, int OP, typename ST = T>
+// Planes of fewer pixels are walked across batch elements (one at a time they leave lanes, and the loads in flight,
+// idle): backward of 3x3 at (1949, 5 -> 8, 4, 4) 21 us, 80 plane by plane.
+constexpr int FLAT_PLANE = 4 * BLOCK;
+
+// WONLY: grad_weight alone (grad_input by packed_tile_backward). Its unrolled loads are not part of the other
+// form, whose gathering workgroups they slow down (5x5 at (1, 3 -> 5, 259, 316) 54 -> 60 us).
+template <typename T, int OP, typename ST, bool WONLY>
 __global__ __launch_bounds__(BLOCK) void morpho_bwd_packed_kernel(const PackedParams<T, ST> p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     Acc* bins = reinterpret_cast<Acc*>(smem_raw);
     const Geom g = p.g;
     const int work = xcd_work_index(blockIdx.x, gridDim.x);
-    if (work >= p.wblocks)
+    if (!WONLY && work >= p.wblocks)
     {
         // Gathering workgroup: each pixel's slots, then their sum in slot order (deterministic).
         __shared__ Acc slot_sums[BLOCK];
@@ -144,43 +150,76 @@ __global__ __launch_bounds__(BLOCK) void morpho_bwd_packed_kernel(const PackedPa
         else
             global_add(&part[(int64_t)c * K + k], sign * gv);
     };
-    // The chunk's pixels batch element by batch element: contiguous winners and gradients.
-    for (int64_t b = n_begin / plane; b * plane < n_end; ++b)
+    if constexpr (!WONLY)
     {
-        const int64_t q0 = (b * g.Cout + o) * plane;
-        const int64_t lo = max(n_begin - b * plane, (int64_t)0), hi = min(n_end - b * plane, plane);
-        if (!p.gin)
+        for (int64_t n = n_begin + threadIdx.x; n < n_end; n += BLOCK)
         {
-            // grad_weight alone: four pixels' loads in flight together.
-            constexpr int U = 4;
-            for (int64_t pix = lo + threadIdx.x; pix < hi; pix += U * BLOCK)
+            const int64_t b = n / plane;
+            const int64_t pix = n - b * plane;
+            const int64_t q = (b * g.Cout + o) * plane + pix;
+            const T gv = (T)p.gout[q];
+            if (gv == T(0)) continue;
+            const int32_t packed = p.idx[q];
+            if (p.gin)
+            {
+                const int h = (int)(pix / g.W), wc = (int)(pix - (int64_t)h * g.W);
+                const int c = packed >> 16, k = packed & 0xFFFF;
+                const int kh = k / g.KW, kw = k - kh * g.KW;
+                const int iy = h + ph - kh, ix = wc + pw - kw;
+                if (iy >= 0 && iy < g.H && ix >= 0 && ix < g.W) global_add(&p.gin[(b * g.Cin + c) * plane + (int64_t)iy * g.W + ix], (Acc)gv);
+            }
+            add_weight(packed, gv);
+        }
+    }
+    else
+    {
+        constexpr int U = 4;  // pixels whose loads are in flight together
+        if (plane >= FLAT_PLANE || p.chunk > 0x3fffffff)
+        {
+            // The chunk's pixels batch element by batch element: contiguous winners and gradients.
+            for (int64_t b = n_begin / plane; b * plane < n_end; ++b)
+            {
+                const int64_t q0 = (b * g.Cout + o) * plane;
+                const int64_t lo = max(n_begin - b * plane, (int64_t)0), hi = min(n_end - b * plane, plane);
+                for (int64_t pix = lo + threadIdx.x; pix < hi; pix += U * BLOCK)
+                {
+                    int32_t packed[U];
+                    T gv[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                    {
+                        const int64_t q = q0 + min(pix + u * BLOCK, hi - 1);
+                        packed[u] = p.idx[q];
+                        gv[u] = (T)p.gout[q];
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        if (pix + u * BLOCK < hi && gv[u] != T(0)) add_weight(packed[u], gv[u]);
+                }
+            }
+        }
+        else if (n_begin < n_end)
+        {
+            // Across batch elements (pixel numbers from the chunk's first one's, in 32 bits).
+            const int64_t b0 = n_begin / plane;
+            const unsigned hi = (unsigned)(n_end - b0 * plane), up = (unsigned)plane;
+            const int64_t q0 = (b0 * g.Cout + o) * plane, skip = (int64_t)(g.Cout - 1) * plane;
+            for (unsigned n = (unsigned)(n_begin - b0 * plane) + threadIdx.x; n < hi; n += U * BLOCK)
             {
                 int32_t packed[U];
                 T gv[U];
 #pragma unroll
                 for (int u = 0; u < U; ++u)
                 {
-                    const int64_t q = q0 + min(pix + u * BLOCK, hi - 1);
+                    const unsigned m = min(n + u * BLOCK, hi - 1);
+                    const int64_t q = q0 + m + (m / up) * skip;
                     packed[u] = p.idx[q];
                     gv[u] = (T)p.gout[q];
                 }
 #pragma unroll
                 for (int u = 0; u < U; ++u)
-                    if (pix + u * BLOCK < hi && gv[u] != T(0)) add_weight(packed[u], gv[u]);
+                    if (n + u * BLOCK < hi && gv[u] != T(0)) add_weight(packed[u], gv[u]);
             }
-            continue;
-        }
-        for (int64_t pix = lo + threadIdx.x; pix < hi; pix += BLOCK)
-        {
-            const T gv = (T)p.gout[q0 + pix];
-            if (gv == T(0)) continue;
-            const int32_t packed = p.idx[q0 + pix];
-            const int h = (int)(pix / g.W), wc = (int)(pix - (int64_t)h * g.W);
-            const int c = packed >> 16, k = packed & 0xFFFF;
-            const int kh = k / g.KW, kw = k - kh * g.KW;
-            const int iy = h + ph - kh, ix = wc + pw - kw;
-            if (iy >= 0 && iy < g.H && ix >= 0 && ix < g.W) global_add(&p.gin[(b * g.Cin + c) * plane + (int64_t)iy * g.W + ix], (Acc)gv);
-            add_weight(packed, gv);
         }
     }
     if (p.lds_bins)
@@ -1057,7 +1096,8 @@ static hipError_t backward_op(int merge, bool replicate, T fill, const T* x, con
         p.lds_bins = s.lds_bins ? 1 : 0;
         p.chunk = s.chunk;
         p.wblocks = s.nchunks * g.Cout;
-        morpho_bwd_packed_kernel<T, OP><<<(unsigned)((int64_t)p.wblocks + s.gblocks), BLOCK, s.lds, stream>>>(p);
+        const auto kernel = s.tile ? morpho_bwd_packed_kernel<T, OP, T, true> : morpho_bwd_packed_kernel<T, OP, T, false>;
+        kernel<<<(unsigned)((int64_t)p.wblocks + s.gblocks), BLOCK, s.lds, stream>>>(p);
         if ((err = hipGetLastError()) != hipSuccess) return err;
         if (s.tile)
             if ((err = packed_tile_backward<T, T>(p.idx, grad_out, grad_in, g, stream)) != hipSuccess) return err;
@@ -1259,7 +1299,8 @@ static hipError_t half_direct(int merge, const void* indices, const ST* grad_out
         p.lds_bins = s.lds_bins ? 1 : 0;
         p.chunk = s.chunk;
         p.wblocks = s.nchunks * g.Cout;
-        morpho_bwd_packed_kernel<float, OP, ST><<<(unsigned)((int64_t)p.wblocks + s.gblocks), BLOCK, s.lds, stream>>>(p);
+        const auto kernel = s.tile ? morpho_bwd_packed_kernel<float, OP, ST, true> : morpho_bwd_packed_kernel<float, OP, ST, false>;
+        kernel<<<(unsigned)((int64_t)p.wblocks + s.gblocks), BLOCK, s.lds, stream>>>(p);
         if ((err = hipGetLastError()) != hipSuccess) return err;
         if (s.tile)
             if ((err = packed_tile_backward<float, ST>(p.idx, grad_out, grad_in, g, stream)) != hipSuccess) return err;

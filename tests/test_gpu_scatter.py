@@ -52,6 +52,7 @@ def _run(op, merge, padding, dtype, B, Cin, Cout, H, W, KH, KW):
     (1, 2, 4, 40, 300, 21, 21),    # tap numbers past 256
     (1, 2, 16, 1, 45000, 1, 31),   # a plane of one row
     (1, 130, 4, 31, 33, 9, 9),     # three channel groups
+    (2500, 8, 16, 4, 5, 3, 3),     # small planes: winners walked across batch elements
 ])
 def test_packed_tiles(shape, dtype):
     _run("erosion" if shape[1] % 2 else "dilation", "max" if shape[2] % 3 else "min", "replicate", dtype, *shape)
