@@ -184,8 +184,8 @@ struct IdentTileParams
     unsigned kw_magic;
 };
 
-template <int OP, typename T, typename ST, typename AT>
-__global__ __launch_bounds__(BLOCK) void ident_tile_kernel(const IdentTileParams<T, ST> p)
+template <int OP, typename T, typename ST, typename AT, int THREADS>
+__global__ __launch_bounds__(THREADS) void ident_tile_kernel(const IdentTileParams<T, ST> p)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const Geom& g = p.g;
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(BLOCK) void ident_tile_kernel(const IdentTileParams
     const int x0 = tx * t.tw, y0 = ty * t.th;
     const int cols = min(t.tw, g.W - x0), rows = min(t.th, g.H - y0);
     const int ncopy = 1 << t.ncopy_log2;
-    for (int j = threadIdx.x; j < t.tw * t.th + K * ncopy; j += BLOCK) acc[j] = Acc(0);
+    for (int j = threadIdx.x; j < t.tw * t.th + K * ncopy; j += THREADS) acc[j] = Acc(0);
     const int ph = g.pad_h(), pw = g.pad_w();
     const int h_lo = max(y0 - ph, 0), h_hi = min(y0 + rows - ph + g.KH - 1, g.H);
     const int w_lo = max(x0 - pw, 0), w_hi = min(x0 + cols - pw + g.KW - 1, g.W);
@@ -215,14 +215,14 @@ __global__ __launch_bounds__(BLOCK) void ident_tile_kernel(const IdentTileParams
     __syncthreads();
 
     constexpr int U = 8;  // pixels whose loads are in flight together
-    for (int i0 = threadIdx.x; i0 < n; i0 += U * BLOCK)
+    for (int i0 = threadIdx.x; i0 < n; i0 += U * THREADS)
     {
         int at[U], k[U], dy[U], dx[U];
         T gv[U];
 #pragma unroll
         for (int u = 0; u < U; ++u)
         {
-            const int i = min(i0 + u * BLOCK, n - 1);
+            const int i = min(i0 + u * THREADS, n - 1);
             const int r = div_by(i, rmagic);
             const int h = h_lo + r, w = w_lo + i - r * rcols;
             at[u] = h * g.W + w;
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(BLOCK) void ident_tile_kernel(const IdentTileParams
 #pragma unroll
         for (int u = 0; u < U; ++u)
         {
-            if (i0 + u * BLOCK >= n) break;
+            if (i0 + u * THREADS >= n) break;
             const int kh = div_by(k[u], p.kw_magic);
             const int iy = dy[u] + ph - kh, ix = dx[u] + pw - (k[u] - kh * g.KW);
             const Acc v = (Acc)gv[u];
@@ -251,13 +251,13 @@ __global__ __launch_bounds__(BLOCK) void ident_tile_kernel(const IdentTileParams
     __syncthreads();
     const unsigned cmagic = cols == 1 ? 0u : (unsigned)(((uint64_t(1) << 32) + cols - 1) / cols);
     ST* __restrict__ gin = p.gin + base + (int64_t)y0 * g.W + x0;
-    for (int j = threadIdx.x; j < rows * cols; j += BLOCK)
+    for (int j = threadIdx.x; j < rows * cols; j += THREADS)
     {
         const int r = div_by(j, cmagic), col = j - r * cols;
         gin[r * g.W + col] = (ST)(T)acc[r * t.tw + col];
     }
     T* __restrict__ part = p.part + (((int64_t)b * t.ntx * t.nty + tile) * g.Cin + c) * K;
-    for (int j = threadIdx.x; j < K; j += BLOCK)
+    for (int j = threadIdx.x; j < K; j += THREADS)
     {
         Acc s = Acc(0);
         for (int q = 0; q < ncopy; ++q) s += bins[(j << t.ncopy_log2) + ((q + j) & (ncopy - 1))];
@@ -291,6 +291,9 @@ IdentTiles ident_tiles(const Geom& g)
     return t;
 }
 
+// Pixels up to which one wave takes a tile: backward of 3x3 at (2114, 10 -> 10, 3, 8) 24 us, 62 by four waves.
+constexpr int IDENT_WAVE_TILE = 256;
+
 template <typename T, typename ST>
 hipError_t ident_tile_backward(int op, const IdentTiles& tiles, const void* taps, const ST* grad_out, ST* grad_in, T* part, const Geom& g,
                                hipStream_t stream)
@@ -306,9 +309,16 @@ hipError_t ident_tile_backward(int op, const IdentTiles& tiles, const void* taps
     const int64_t blocks = (int64_t)g.B * g.Cin * tiles.nty * tiles.ntx;
     if (!tiles.ok || blocks > 0x7fffffff) return hipErrorInvalidValue;
     const bool wide = pair_tap_bytes(g) == 2;
-    const auto kernel = op == DILATION ? (wide ? ident_tile_kernel<DILATION, T, ST, uint16_t> : ident_tile_kernel<DILATION, T, ST, uint8_t>)
-                                       : (wide ? ident_tile_kernel<EROSION, T, ST, uint16_t> : ident_tile_kernel<EROSION, T, ST, uint8_t>);
-    kernel<<<(unsigned)blocks, BLOCK, p.t.lds, stream>>>(p);
+    // Tiles of a few hundred pixels (small planes) by one wave each: four waves would mostly wait for one another.
+    const bool small = tiles.tw * tiles.th <= IDENT_WAVE_TILE;
+    auto launch = [&](auto kernel, int threads) { kernel<<<(unsigned)blocks, threads, p.t.lds, stream>>>(p); };
+    auto sized = [&](auto one, auto four) { small ? launch(one, WAVE) : launch(four, BLOCK); };
+    if (op == DILATION)
+        wide ? sized(ident_tile_kernel<DILATION, T, ST, uint16_t, WAVE>, ident_tile_kernel<DILATION, T, ST, uint16_t, BLOCK>)
+             : sized(ident_tile_kernel<DILATION, T, ST, uint8_t, WAVE>, ident_tile_kernel<DILATION, T, ST, uint8_t, BLOCK>);
+    else
+        wide ? sized(ident_tile_kernel<EROSION, T, ST, uint16_t, WAVE>, ident_tile_kernel<EROSION, T, ST, uint16_t, BLOCK>)
+             : sized(ident_tile_kernel<EROSION, T, ST, uint8_t, WAVE>, ident_tile_kernel<EROSION, T, ST, uint8_t, BLOCK>);
     return hipGetLastError();
 }
 

@@ -72,6 +72,9 @@ def test_packed_falls_back_to_atomics():
     ("erosion", (40, 30, 30, 13, 11, 4, 2)),  # one tile per plane, full-height tiles
     ("dilation", (1, 2, 2, 50, 47, 17, 17)),  # two-byte taps
     ("erosion", (1, 3, 3, 64, 100, 1, 9)),
+    ("dilation", (3, 4, 4, 16, 16, 5, 5)),    # 256 pixels: one wave a tile
+    ("erosion", (3, 4, 4, 16, 17, 5, 5)),     # four
+    ("dilation", (50, 7, 7, 3, 2, 3, 3)),
 ])
 def test_identity_tiles(op, shape, dtype):
     for padding in ("replicate", "geodesic"):
