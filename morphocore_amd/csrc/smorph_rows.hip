@@ -101,7 +101,10 @@ __global__ __launch_bounds__(BLOCK) void smorph_fwd_rows(const RowsParams<T> q)
         const int pair = o * g.Cin + i;
         const T* wp = wts[wave];
         T ref[1], S[1], Wsum[1];
+        // The wave's lanes read what its other lanes staged: in order for the compiler too (no instruction waits).
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         if (inside)
             smorph_pair_stats<T, 1, KS, false>(tbase, cols, nullptr, wp, a, g, h + P, wc + P, ref, S, Wsum);
         else
