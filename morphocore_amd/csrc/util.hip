@@ -42,7 +42,7 @@ __global__ __launch_bounds__(BLOCK) void reduce_slots_kernel(const PT* __restric
         out[j] = (T)sum_slots(part, 0, nslots, n, j);
 }
 
-// The same sums in one launch for a few hundred slots: COLS consecutive columns per workgroup, each by
+// The same sums in one launch for up to JOINT_SLOTS slots: COLS consecutive columns per workgroup, each by
 // BLOCK / COLS threads that take every (BLOCK / COLS)-th slot; their sums are then added in thread order
 // (a fixed order, in double, rounded once).
 template <typename T, typename PT, int COLS>
@@ -136,9 +136,13 @@ hipError_t fill_async(T* p, int64_t n, T v, hipStream_t stream)
     return hipGetLastError();
 }
 
-// Up to this many slots are summed by one launch (two took ~5 us each on the few thousand columns of a
-// layer); more by groups first, which spread the slots over more workgroups.
-constexpr int JOINT_SLOTS = 2048;
+// Up to this many slots are summed by one launch; more by groups first, which spread the slots over more
+// workgroups. 8 columns a workgroup (32 bytes of each 128-byte line of a slot, which four workgroups then read) only
+// where few columns and many slots would leave too few workgroups. Time over that of the two launches (6 us at
+// least), float32 slots, 8 | 32 columns: 400 columns of 128 slots 0.37 | 0.37, of 512 0.41 | 0.62, of 2048
+// 0.56 | 1.40; 1600 of 1024 0.51 | 0.95; 4608 of 256 0.44 | 0.45, of 512 0.94 | 0.54, of 1024 1.54 | 0.71, of 2048
+// 1.92 | 1.31; 16000 of 1024 2.24 | 0.80, 102400 of 1024 - | 1.14 (0.93 of 512).
+constexpr int JOINT_SLOTS = 1024, JOINT_FEW_COLUMNS = 3072;
 
 template <typename T>
 size_t reduce_slots_scratch(int nslots, int64_t n)
@@ -157,8 +161,7 @@ hipError_t reduce_slots_async(const PT* part, int nslots, int64_t n, T* out, PT*
     }
     if (nslots <= JOINT_SLOTS)
     {
-        // Few columns: 8 per workgroup, so that enough workgroups run.
-        if (n < 16384)
+        if (nslots > 128 && n < JOINT_FEW_COLUMNS)
             reduce_joint_kernel<T, PT, 8><<<(unsigned)((n + 7) / 8), BLOCK, 0, stream>>>(part, nslots, n, out);
         else
             reduce_joint_kernel<T, PT, 32><<<(unsigned)((n + 31) / 32), BLOCK, 0, stream>>>(part, nslots, n, out);
