@@ -25,7 +25,10 @@ def element(w: torch.Tensor, alpha: torch.Tensor, channel_merge_mode: str = "sum
     per_pair = (w.dim() == 4 and w.shape[1] == 1 and alpha.numel() == w.shape[0] if channel_merge_mode == 'identity' or alpha.dim() == 1
                 else alpha.shape == w.shape[:2] and w.dim() == 4)
     if per_pair and w.is_cuda and alpha.device == w.device and alpha.dtype == w.dtype and w.dtype in (torch.float32, torch.float64):
-        return ops.smorph_element(w, torch.tanh(alpha))
+        t = torch.tanh(alpha)
+        if channel_merge_mode == 'identity' and alpha.dim() > 1:
+            t = t.view(-1)  # as w_tilde: refuses strides that it cannot view as one value per channel
+        return ops.smorph_element(w, t)
     return w_tilde(w, alpha, channel_merge_mode)
 
 

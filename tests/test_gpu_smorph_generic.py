@@ -84,6 +84,15 @@ def test_element_other_forms():
         assert normwise_error(got.cpu().numpy(), want.cpu().numpy()) <= 1e-12
 
 
+def test_element_refuses_what_the_torch_operations_refuse():
+    """Identity alphas whose strides cannot be viewed as one value per channel."""
+    w, alpha = seeded(69, 6, 1, 3, 3).cuda(), seeded(70, 2, 3).cuda()
+    for f in (element, w_tilde):
+        assert f(w, alpha, "identity").shape == w.shape
+        with pytest.raises(RuntimeError, match="view"):
+            f(w, alpha.t(), "identity")
+
+
 def test_element_keeps_strided_inputs_in_the_graph():
     """Second gradients of an element and alpha that are strided views reach both."""
     w, alpha = seeded(67, 3, 2, 5, 3, dtype=torch.float64).cuda(), seeded(68, 2, 3, dtype=torch.float64).cuda()
