@@ -8,7 +8,7 @@
 // float32 afterwards. Small problems (whose time is launches) gather grad_input instead, in
 // further workgroups of the same launch: each input pixel sums, in double and in (output channel,
 // tap) order, the gradients of the output pixels whose winner it is, written once (no zero fill, no
-// atomics, no rounding pass), and keep at most 32 slots (one reduction launch).
+// atomics, no rounding pass), and keep at most 32 slots.
 // Reference semantics: morpho_op_cpu_backward.hxx:39-88 (run_single_winner).
 //
 // ADD / AVERAGE / IDENTITY: every channel pair routes g * scale to its own first extremal tap
@@ -18,7 +18,7 @@
 // tile's outputs land, atomics on the halo shared with neighbouring tiles) and grad_weight in
 // lane-striped LDS bins, written once per chunk of output channels into the workgroup's partial
 // slot. Partial slots are then summed in a fixed order (reduce_slots_async). LDS accumulators are
-// double (see Acc). Two kernels:
+// double (see Acc). Three kernels:
 //   morpho_bwd_planes_kernel  ADD / AVERAGE whose KW planes of the tile fit in LDS: one input
 //                             channel per workgroup, grad_input split into one plane per
 //                             structuring-element column, which makes the atomic adds bank-conflict
@@ -750,7 +750,7 @@ static PackedPlan plan_packed(const Geom& g)
     int64_t nchunks = (4096 + g.Cout - 1) / std::max(g.Cout, 1);  // (no output channel: an empty launch)
     const int64_t max_chunks = (total + BLOCK - 1) / BLOCK;
     if (nchunks > max_chunks) nchunks = max_chunks;
-    if (s.gather && nchunks > REDUCE_GROUP) nchunks = REDUCE_GROUP;  // one reduction launch
+    if (s.gather && nchunks > REDUCE_GROUP) nchunks = REDUCE_GROUP;  // (up to 128: the same time)
     while (nchunks > 1 && (size_t)nchunks * wnumel * sizeof(T) > ((size_t)256 << 20)) nchunks /= 2;
     if (nchunks < 1) nchunks = 1;
     s.nchunks = (int)nchunks;
@@ -1263,8 +1263,9 @@ size_t half_backward_workspace(int merge, bool has_indices, const Geom& g)
     return bytes;
 }
 
-// The kernels that read grad_output once per output pixel and write grad_input once per input pixel
-// take the 16-bit data directly: the max / min scatter and the IDENTITY tiles. grad_weight is summed in float32 partial slots and rounded at the end.
+// The kernels that read the 16-bit data directly and write grad_input once per input pixel: the max / min gather
+// and tiles (and, rounded from its double buffer, the scatter of elements the tiles do not take) and the
+// IDENTITY tiles. grad_weight is summed in float32 partial slots and rounded at the end.
 template <typename ST, int OP>
 static hipError_t half_direct(int merge, const void* indices, const ST* grad_out, ST* grad_in, ST* grad_w, const Geom& g, unsigned char* ws,
                               float* gw, hipStream_t stream)
