@@ -25,6 +25,11 @@ from morphocore_amd.functional.smorph import element, w_tilde  # noqa: E402
     (torch.float32, (2, 2, 3, 30, 130, 4, 5)),   # even height
     (torch.float32, (1, 2, 4, 1, 70, 3, 7)),     # a plane of one row
     (torch.float32, (40, 8, 6, 8, 70, 5, 3)),    # enough tiles: one slice
+    # Output-channel slices of several channels (1024 workgroups over 16 planes of 8 strips: 8 slices):
+    (torch.float64, (2, 8, 20, 32, 60, 5, 5)),   # six slices of three channels and one of two
+    (torch.float64, (2, 8, 21, 32, 60, 3, 3)),   # seven of three
+    (torch.float32, (2, 8, 20, 32, 60, 9, 9)),
+    (torch.float32, (2, 8, 21, 32, 60, 5, 3)),
     (torch.float64, (1, 2, 3, 20, 70, 6, 6)),    # not unrolled
     (torch.float32, (1, 3, 2, 7, 21, 13, 13)),   # not unrolled, most taps outside the image
 ])

@@ -1,7 +1,7 @@
 """The smorph forward of launches with few workgroups (four waves, four input channels), whose values are the
-reference's bit for bit, and the output-channel slices of the backward behind it: channel counts that are
-no multiple of four, planes narrower than a wave, rows of several widths, launches on both sides of
-the limit, slices of unequal and of full length.
+reference's bit for bit, and the backward behind it: channel counts that are no multiple of four, planes
+narrower than a wave, rows of several widths, launches on both sides of the limit. (The output-channel
+slices of the generic backward: test_gpu_smorph_generic.py.)
 """
 import numpy as np
 import pytest
@@ -31,17 +31,17 @@ SHAPES = [
     (torch.float64, (2, 5, 8, 65, 64, 3, 3)),     # 1664 waves: this kernel
     (torch.float64, (1, 4, 48, 128, 64, 3, 3)),   # 6144: this kernel
     (torch.float64, (1, 4, 48, 129, 64, 3, 3)),   # 6192: the other
-    (torch.float32, (1, 2, 8, 12, 40, 11, 11)),   # backward: two slices of four output channels
-    (torch.float32, (1, 2, 9, 12, 40, 7, 7)),     # of five and four
-    (torch.float32, (1, 2, 11, 12, 40, 5, 5)),    # of six and five
-    (torch.float32, (1, 2, 29, 12, 40, 3, 3)),    # of fifteen and fourteen
+    (torch.float32, (1, 2, 8, 12, 40, 11, 11)),   # two input channels: the static kernels
+    (torch.float32, (1, 2, 9, 12, 40, 7, 7)),
+    (torch.float32, (1, 2, 11, 12, 40, 5, 5)),
+    (torch.float32, (1, 2, 29, 12, 40, 3, 3)),
 ]
 
 
 @pytest.mark.parametrize("saved", [True, False], ids=["saved-stats", "recomputed"])
 @pytest.mark.parametrize("merge", ["sum", "mean", "max", "min"])
 @pytest.mark.parametrize("dtype,shape", SHAPES, ids=[str(s[0])[6:] + "-" + "x".join(map(str, s[1])) for s in SHAPES])
-def test_rows_forward_and_sliced_backward(dtype, shape, merge, saved, monkeypatch):
+def test_rows_forward_and_backward(dtype, shape, merge, saved, monkeypatch):
     if not saved and (dtype == torch.float64 or shape[-1] == 9):
         pytest.skip("no statistics are saved for this element")
     monkeypatch.setenv("MORPHOCORE_AMD_SAVED_STATS_LIMIT", "-1" if saved else "0")
