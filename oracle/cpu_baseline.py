@@ -18,7 +18,6 @@ import sys
 import time
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-ROOT = os.path.dirname(HERE)
 REF_LIB = os.path.join(HERE, "_ref", "libmorphocore_ref.so")
 
 MERGES = {"max": 0, "min": 1, "sum": 2, "mean": 3, "identity": 5}
@@ -94,11 +93,10 @@ def run_reference(spec, threads):
 
 def run_port(spec, threads):
     os.environ["OMP_NUM_THREADS"] = str(threads)
-    sys.path.insert(0, ROOT)
     import numpy as np
     import torch
 
-    from oracle import oracle as O
+    import oracle as O  # (this script's folder leads sys.path: oracle.py, not the folder above it)
 
     x, ws, dtype = _inputs(spec, torch)
     xn = x.numpy()
@@ -126,7 +124,17 @@ def run_port(spec, threads):
             gm, _ = O.morpho_backward(ops_[1], MERGES["identity"], padding, 0.0, mid, wk[ops_[1]], np.ones_like(out))
             O.morpho_backward(ops_[0], MERGES["identity"], padding, 0.0, xn, wk[ops_[0]], gm)
             return out.size
-        raise ValueError("the port baseline covers single operators and the opening / closing pair")
+        if spec["kind"] == "stack":
+            alpha = np.full((xn.shape[1], xn.shape[1]), 5.0, dtype=xn.dtype)
+            wt, we = O.smorph_w_tilde(wn[1], alpha, "sum"), np.ascontiguousarray(wn[2][:, :, ::-1, ::-1])
+            y1, i1 = O.morpho_forward(O.DILATION, MERGES["max"], padding, 0.0, xn, wn[0], save_indices=True)
+            y2 = O.smorph_forward(MERGES["sum"], y1, wt, alpha)
+            out, i3 = O.morpho_forward(O.EROSION, MERGES["min"], padding, 0.0, y2, we, save_indices=True)
+            g2, _ = O.morpho_backward(O.EROSION, MERGES["min"], padding, 0.0, y2, we, np.ones_like(out), indices=i3)
+            g1 = O.smorph_backward(MERGES["sum"], y1, wt, alpha, g2)[0]
+            O.morpho_backward(O.DILATION, MERGES["max"], padding, 0.0, xn, wn[0], g1, indices=i1)
+            return out.size * 3
+        raise ValueError("the port baseline covers single operators, the opening / closing pair and the stack")
 
     return step
 

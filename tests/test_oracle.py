@@ -9,8 +9,11 @@
   smorph, and the reference's known-answer padding tests (test_padding.py:95-143);
 * the oracle's exponential against libm within the accuracy its method promises.
 """
+import json
 import math
 import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -593,3 +596,22 @@ def test_smorph_term_magnitudes(dtype):
     gw = O.smorph_scm_backward(x, w, alpha, beta, g)[1]
     assert np.all(mw >= np.abs(gw) * (1 - tol)) and np.all(ma >= np.abs(ga) * (1 - tol)) and np.all(mb >= np.abs(gb) * (1 - tol))
     assert np.array_equal(O.smorph_scm_term_magnitudes(x, w, alpha, beta, -g)[2], mb)
+
+
+@pytest.mark.parametrize("spec", [
+    dict(kind="morpho", op="erosion", merge="sum", w=[4, 3, 3, 3]),
+    dict(kind="smorph", merge="mean", w=[4, 3, 3, 3], alpha=1.0, alpha_shape=[4, 3]),
+    dict(kind="pair", op="erosion", w=[3, 1, 3, 3]),
+    dict(kind="stack", w=[3, 3, 3, 3]),
+])
+def test_cpu_baseline_runs_on_the_oracle(spec):
+    """The bench's CPU leg as the bench starts it: a script of its own, on the oracle where the reference's
+    extension is not built."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    spec = dict(spec, dtype="f32", x=[1, 3, 12, 12], w_std=0.1, threads=2, min_seconds=0.0, max_steps=1)
+    r = subprocess.run([sys.executable, os.path.join(root, "oracle", "cpu_baseline.py"), json.dumps(spec)], capture_output=True, text=True,
+                       timeout=120, cwd=root)
+    assert r.returncode == 0, r.stderr[-1000:]
+    out = json.loads(r.stdout.strip().splitlines()[-1])
+    assert out["steps"] == 1 and out["seconds_per_step"] > 0
+    assert out["output_elements"] == (3 if spec["kind"] == "stack" else 1) * spec["w"][0] * 144
