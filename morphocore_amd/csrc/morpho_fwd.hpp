@@ -922,8 +922,7 @@ static hipError_t launch_generic(FwdParams<ST> p, hipStream_t stream)
 // idle and every workgroup's serial latency (its channel loop, the winner rescans of its pixels) is the
 // kernel time: such launches take one output channel per workgroup and 4, 2 or 1 rows per wave, the
 // most that leaves small_rows().four or .two workgroups and no wave without rows. More rows per wave share each LDS read of the window and
-// of the element; fewer make more workgroups, and keep fewer windows in registers where every tap is tracked
-// (11x11 is faster by one row at every size).
+// of the element; fewer make more workgroups, and keep fewer windows in registers where every tap is tracked.
 constexpr int64_t SMALL_GRID = 1024;
 
 struct SmallRows
@@ -933,16 +932,18 @@ struct SmallRows
 
 // Measured over 1100 random launches below SMALL_GRID (3x3 to 11x11, float32 and bfloat16): time over that of the
 // best of the three, geometric mean, by these limits | by one row always:
-// values 1.006 | 1.21, identity values 1.005 | 1.13, max / min winners 1.01 | 1.16, taps 1.01 | 1.02,
-// identity taps 1.01 | 1.05. Float32 (us, at 4, 2, 1 rows): values, 7x7 at (4, 8 -> 8, 128, 128) 18.8 20.6 30.4 (512,
+// values 1.006 | 1.25, identity values 1.006 | 1.13, max / min winners 1.01 | 1.12, taps 1.01 | 1.04,
+// identity taps 1.01 | 1.06. Float32 (us, at 4, 2, 1 rows): values, 7x7 at (4, 8 -> 8, 128, 128) 18.8 20.6 30.4 (512,
 // 1024, 2048 workgroups), 5x5 at (1, 16 -> 16, 64, 64) 17.8 12.9 10.6 (64, 128, 256); taps, 7x7 at
 // (2, 11 -> 38, 94, 14) 35.4 36.1 43.2 (456, 912, 1824), 9x9 at (11, 5 -> 6, 19, 162) 26.9 22.0 19.3
 // (396, 594, 990), 11x11 at (5, 28 -> 8, 60, 75) 186 187 157 (320, 640, 1200).
-template <int MODE, int KS>
+// (Taps of several channels of 7x7 and larger take 4 rows only where 16-row tiles hold at most 8% more rows than
+// the alternative's: 7x7 at (3, 27 -> 31, 249, 38) 210 234 277, but 9x9 at (8, 2 -> 50, 22, 102) 33.4 26.7 29.9.)
+template <int MODE, int KS, int MK>
 constexpr SmallRows small_rows()
 {
     constexpr int64_t never = INT64_MAX;
-    if (MODE == FWD_TAPS) return KS <= 5 ? SmallRows{640, 384} : (KS <= 9 ? SmallRows{never, 512} : SmallRows{never, never});
+    if (MODE == FWD_TAPS) return KS <= 5 ? SmallRows{640, 384} : SmallRows{MK == MK_IDENT ? never : 640, KS <= 9 ? 512 : never};
     if (MODE == FWD_PACKED) return KS <= 5 ? SmallRows{768, 512} : SmallRows{640, 256};
     return SmallRows{448, KS == 3 ? 384 : 192};
 }
@@ -972,9 +973,11 @@ static hipError_t launch_static(FwdParams<ST> p, hipStream_t stream)
                 p.t = make_tiling(p.g, rh);
                 return blocks = (int64_t)p.g.B * p.t.nty * p.t.ntx * p.nog;
             };
-            constexpr SmallRows rows = small_rows<MODE, KS>();
+            constexpr SmallRows rows = small_rows<MODE, KS, MK>();
+            const auto tiled_rows = [&](int rh) { return (int64_t)make_tiling(p.g, rh).nty * NWAVES * rh; };
+            const bool fits = 12 * tiled_rows(RH) <= 13 * tiled_rows(KS <= 9 ? 2 : 1);
             if constexpr (rows.four < INT64_MAX)
-                if (p.g.H > NWAVES * RH / 2 && with_rows(RH) >= rows.four)
+                if (p.g.H > NWAVES * RH / 2 && (MODE != FWD_TAPS || KS <= 5 || fits) && with_rows(RH) >= rows.four)
                 {
                     morpho_fwd_static<ST, OP, MK, KS, KS, 1, RH, MODE><<<(unsigned)blocks, BLOCK, 0, stream>>>(p);
                     return hipGetLastError();
