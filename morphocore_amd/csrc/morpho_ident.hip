@@ -1,4 +1,4 @@
-// Dilation / erosion with the IDENTITY merge (each channel with its own element: configs[3]'s layer),
+// Dilation / erosion with the IDENTITY merge (each channel with its own element),
 // 3x3 and 5x5 elements, as streaming kernels over row bands of whole image rows (reference semantics:
 // morpho_op_cpu_kernels.hxx:202-296 for the strict first-tap scan, morpho_op_cpu_backward.hxx:90-156
 // for the routing). The work is ~1 flop per byte moved, so these kernels are bound by HBM: each

@@ -379,7 +379,7 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
 // receives ref, then 1 / sum, [B, Cout, H, W] each, for the backward. The c_i of one output channel
 // are Cin planes apart, so consecutive threads read consecutive pixels of each plane.
 // CREG > 0 (Cin <= CREG, checked by the launcher): the c_i are read once, into registers, and both
-// passes run from there (the two-pass form reads them from memory twice: 4.2 ms at configs[2]'s shape,
+// passes run from there (the two-pass form reads them from memory twice: 4.2 ms at (8, 64 -> 64, 256, 256),
 // 8.6 GB of pair outputs per pass).
 template <typename T, int CREG>
 __global__ __launch_bounds__(BLOCK) void smorph_soft_merge_kernel(const T* __restrict__ pout, const T* __restrict__ beta, T* __restrict__ out,

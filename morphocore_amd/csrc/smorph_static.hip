@@ -333,7 +333,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(KH * KW >
         else if constexpr (KW > 7)
         {
             // 11x11: the border tiles keep the select (the keep factors of the select-free masked sums
-            // spill registers there: 60 bytes per lane, measured 1.5% slower on configs[4]).
+            // spill registers there: 60 bytes per lane, measured 1.5% slower at (8, 64, 512, 512)).
             ref = smorph_ref<KH, KW, true>(xb, w, dil, tm);
             if (za)
                 smorph_sums<KH, KW, true, true>(xb, w, a, ref, tm, S, Wsum);
