@@ -200,6 +200,7 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
         const int y0 = h0 + ph - (g.KH - 1), x0 = w0 + pw - (g.KW - 1);
         const int wc = w0 + lane;
         const int iy0 = h0 + wave * RH + ph, ix = wc + pw;
+        const bool live = h0 + wave * RH < g.H;  // else no row of this wave is in the image
         __syncthreads();
         stage_tile(tile, p.x + ((int64_t)b * g.Cin + i) * plane, g, t, y0, x0, false, T(0));
         if constexpr (!GGIN)
@@ -235,102 +236,105 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
 #pragma unroll
                 for (int j = 0; j < NW; ++j) wnext[j] = wn[min((int)threadIdx.x + j * BLOCK, K - 1)];
             }
-            T ref[RH], S[RH], Wsum[RH], outp[RH], scaled[RH], asum[RH];
-            bool in[RH];
-            T bsum = T(0);
-            if (inside)
-                smorph_pair_stats<T, RH, KWS, false>(tbase, t.pitch, wg, wp, a, g, iy0, ix, ref, S, Wsum);
-            else
-                smorph_pair_stats<T, RH, KWS, true>(tbase, t.pitch, wg, wp, a, g, iy0, ix, ref, S, Wsum);
-#pragma unroll
-            for (int r = 0; r < RH; ++r)
+            if (live)
             {
-                const int h = h0 + wave * RH + r;
-                in[r] = h < g.H && wc < g.W;
-                const int64_t oi = ((int64_t)b * g.Cout + o) * plane + (int64_t)h * g.W + wc;
-                T gv = in[r] ? p.gout[oi] * p.scale : T(0);
-                const T inv = T(1) / S[r];
-                outp[r] = Wsum[r] * inv;
-                if constexpr (MK == MK_MAX || MK == MK_MIN)
-                {
-                    if (in[r])
-                    {
-                        const T cnt = p.counts[oi];
-                        gv = gv / (cnt > T(0) ? cnt : T(1));
-                        if (!is_winner(outp[r], p.out[oi])) gv = T(0);
-                    }
-                }
-                if constexpr (MK == MK_SMOOTH)
-                {
-                    // Channel i's share of the soft merge, from the forward's ref and 1 / sum.
-                    if (in[r])
-                    {
-                        const T bt = p.beta[o];
-                        const T sref = p.sstats[oi], sinv = p.sstats[(int64_t)g.B * g.Cout * plane + oi], fin = p.out[oi];
-                        const T c = outp[r];
-                        const T pp = exp_ref((c - sref) * bt, lo) * sinv;
-                        bsum = bsum + pp * (c - sref) * (c - fin) * gv;
-                        gv = gv * fma(bt * pp, c - fin, pp);
-                    }
-                }
-                scaled[r] = gv * inv;
-                asum[r] = T(0);
-            }
-            const int KW = KWS > 0 ? KWS : g.KW;
-            auto route = [&](int kh, int kw) {
-                const int k = kh * KW + kw;
-                const T wk = KWS > 0 ? wp[k] : wg[k];
+                T ref[RH], S[RH], Wsum[RH], outp[RH], scaled[RH], asum[RH];
+                bool in[RH];
+                T bsum = T(0);
+                if (inside)
+                    smorph_pair_stats<T, RH, KWS, false>(tbase, t.pitch, wg, wp, a, g, iy0, ix, ref, S, Wsum);
+                else
+                    smorph_pair_stats<T, RH, KWS, true>(tbase, t.pitch, wg, wp, a, g, iy0, ix, ref, S, Wsum);
 #pragma unroll
                 for (int r = 0; r < RH; ++r)
                 {
-                    // Every in-image tap of an in-image pixel routes, also with a zero gradient
-                    // (so that a NaN of the pair reaches the gradients, as in the reference).
-                    const bool routes = in[r] && (inside || tap_in_image(iy0 + r, ix, kh, kw, g));
-                    const T v = tbase[(r - kh) * t.pitch - kw] + wk;
-                    // The routing's exponential: the hardware one in float32 (the sums above,
-                    // and so the output, use the reference's).
-                    T e;
-                    if constexpr (sizeof(T) == 4)
-                        e = exp_route((v - ref[r]) * a);
-                    else
-                        e = exp_ref((v - ref[r]) * a, lo);
-                    const T pg = e * scaled[r];
-                    const T centered = v - outp[r];
-                    // c = pg (1 + a centered) and the alpha term pg (v - ref) centered share pg centered.
-                    const T q = pg * centered;
-                    // A tap that does not route adds zeros (its own cell and bin exist): no branch per tap, which
-                    // also pays where rows are not unrolled (6x6 backward at (1, 67 -> 50, 93, 28) 1573 -> 1048 us).
-                    const T c = keep_if(fma(a, q, pg), routes);
-                    asum[r] = fma(keep_if(q, routes), keep_if(v - ref[r], routes), asum[r]);
-                    if constexpr (GGIN)
+                    const int h = h0 + wave * RH + r;
+                    in[r] = h < g.H && wc < g.W;
+                    const int64_t oi = ((int64_t)b * g.Cout + o) * plane + (int64_t)h * g.W + wc;
+                    T gv = in[r] ? p.gout[oi] * p.scale : T(0);
+                    const T inv = T(1) / S[r];
+                    outp[r] = Wsum[r] * inv;
+                    if constexpr (MK == MK_MAX || MK == MK_MIN)
                     {
-                        if (routes) global_add(&gplane[(int64_t)(iy0 + r - kh) * g.W + (ix - kw)], (Acc)c);
+                        if (in[r])
+                        {
+                            const T cnt = p.counts[oi];
+                            gv = gv / (cnt > T(0) ? cnt : T(1));
+                            if (!is_winner(outp[r], p.out[oi])) gv = T(0);
+                        }
                     }
-                    else
+                    if constexpr (MK == MK_SMOOTH)
                     {
-                        lds_add(&gtile[(wave * RH + r + g.KH - 1 - kh) * t.pitch + lane + g.KW - 1 - kw], (Acc)c);
+                        // Channel i's share of the soft merge, from the forward's ref and 1 / sum.
+                        if (in[r])
+                        {
+                            const T bt = p.beta[o];
+                            const T sref = p.sstats[oi], sinv = p.sstats[(int64_t)g.B * g.Cout * plane + oi], fin = p.out[oi];
+                            const T c = outp[r];
+                            const T pp = exp_ref((c - sref) * bt, lo) * sinv;
+                            bsum = bsum + pp * (c - sref) * (c - fin) * gv;
+                            gv = gv * fma(bt * pp, c - fin, pp);
+                        }
                     }
-                    lds_add(&bins[k * p.ncopy + copy], (Acc)c);
+                    scaled[r] = gv * inv;
+                    asum[r] = T(0);
                 }
-            };
-            for (int kh = 0; kh < g.KH; ++kh)
-            {
-                if constexpr (KWS > 0)
-                {
+                const int KW = KWS > 0 ? KWS : g.KW;
+                auto route = [&](int kh, int kw) {
+                    const int k = kh * KW + kw;
+                    const T wk = KWS > 0 ? wp[k] : wg[k];
 #pragma unroll
-                    for (int kw = 0; kw < KWS; ++kw) route(kh, kw);
-                }
-                else
+                    for (int r = 0; r < RH; ++r)
+                    {
+                        // Every in-image tap of an in-image pixel routes, also with a zero gradient
+                        // (so that a NaN of the pair reaches the gradients, as in the reference).
+                        const bool routes = in[r] && (inside || tap_in_image(iy0 + r, ix, kh, kw, g));
+                        const T v = tbase[(r - kh) * t.pitch - kw] + wk;
+                        // The routing's exponential: the hardware one in float32 (the sums above,
+                        // and so the output, use the reference's).
+                        T e;
+                        if constexpr (sizeof(T) == 4)
+                            e = exp_route((v - ref[r]) * a);
+                        else
+                            e = exp_ref((v - ref[r]) * a, lo);
+                        const T pg = e * scaled[r];
+                        const T centered = v - outp[r];
+                        // c = pg (1 + a centered) and the alpha term pg (v - ref) centered share pg centered.
+                        const T q = pg * centered;
+                        // A tap that does not route adds zeros (its own cell and bin exist): no branch per tap, which
+                        // also pays where rows are not unrolled (6x6 backward at (1, 67 -> 50, 93, 28) 1573 -> 1048 us).
+                        const T c = keep_if(fma(a, q, pg), routes);
+                        asum[r] = fma(keep_if(q, routes), keep_if(v - ref[r], routes), asum[r]);
+                        if constexpr (GGIN)
+                        {
+                            if (routes) global_add(&gplane[(int64_t)(iy0 + r - kh) * g.W + (ix - kw)], (Acc)c);
+                        }
+                        else
+                        {
+                            lds_add(&gtile[(wave * RH + r + g.KH - 1 - kh) * t.pitch + lane + g.KW - 1 - kw], (Acc)c);
+                        }
+                        lds_add(&bins[k * p.ncopy + copy], (Acc)c);
+                    }
+                };
+                for (int kh = 0; kh < g.KH; ++kh)
                 {
-                    for (int kw = 0; kw < g.KW; ++kw) route(kh, kw);
+                    if constexpr (KWS > 0)
+                    {
+#pragma unroll
+                        for (int kw = 0; kw < KWS; ++kw) route(kh, kw);
+                    }
+                    else
+                    {
+                        for (int kw = 0; kw < g.KW; ++kw) route(kh, kw);
+                    }
                 }
+                T as = T(0);
+#pragma unroll
+                for (int r = 0; r < RH; ++r) as += asum[r];
+                if (as != T(0)) lds_add(&abins[copy], (Acc)as);
+                if constexpr (MK == MK_SMOOTH)
+                    if (bsum != T(0)) lds_add(&bbins[copy], (Acc)bsum);
             }
-            T as = T(0);
-#pragma unroll
-            for (int r = 0; r < RH; ++r) as += asum[r];
-            if (as != T(0)) lds_add(&abins[copy], (Acc)as);
-            if constexpr (MK == MK_SMOOTH)
-                if (bsum != T(0)) lds_add(&bbins[copy], (Acc)bsum);
             if constexpr (KWS > 0)
             {
 #pragma unroll
