@@ -480,15 +480,14 @@ struct SmorphBwdPlan
     size_t lds;
 };
 
-// Element widths whose rows the generic kernels unroll (any height): they run one row per wave, whose taps
-// hide each other's latency. Other widths take the default rows per wave, one after the other. Float64
-// 5x5 at (2, 8 -> 8, 64, 60): forward 168 -> 60 us, backward 288 -> 61 (with the output-channel slices);
-// its training step 528 -> 133 (with smorph_element).
-// They read the pair's element from LDS, at the same address in every lane: scalar loads share the LDS
-// reads' wait counter, and a scalar operand halves an instruction's rate. With it, and out-of-image taps masked
-// by their bits (a select of an exponential becomes a branch a tap), the backward of float64 11x11 at
-// (3, 7 -> 13, 105, 75) takes 1552 us, 1769 before; 5x5 at (2, 8 -> 8, 64, 60) 55, 62 before. (Elements of more
-// than 64 rows, which need the LDS for their tiles, are not unrolled.)
+// Element widths whose rows the generic kernels unroll (up to UNROLLED_KH rows): they run one row per wave, whose
+// taps hide each other's latency, and read the pair's element from LDS, at the same address in every lane (scalar
+// loads share the LDS reads' wait counter, and a scalar operand halves an instruction's rate). Other widths take
+// the default rows per wave, one after the other. Forward | backward in us, several rows per wave -> unrolled:
+// float64 5x5 at (2, 8 -> 8, 64, 60) 162 | 299 -> 24 (smorph_fwd_rows) | 55, 11x11 at (3, 7 -> 13, 105, 75)
+// 1260 | 3175 -> 425 (smorph_fwd_rows) | 1460; float32 9x9 at (3, 4 -> 5, 102, 219) 442 | 944 -> 72 | 193, at
+// (1, 8 -> 53, 269, 292) 2352 | 9669 -> 1400 | 4540, where the bins are flushed for eight times as many tiles.
+// (Elements of more than 64 rows, which need the LDS for their tiles, are not unrolled.)
 static bool smorph_unrolled(const Geom& g) { return g.KW <= 11 && g.KW >= 3 && g.KW % 2 == 1 && g.KH <= UNROLLED_KH; }
 // LDS of that element.
 template <typename T>

@@ -7,8 +7,8 @@
 // order: four times the workgroups for the same work and the same roundings. The 64 pixels are rows of up
 // to 64 columns, or two or more shorter rows where the plane is narrow, whose lanes the other forwards leave
 // idle. Bound by the exponentials' latency at these sizes.
-// Measured (us, before -> after): float64 5x5 at (2, 8 -> 8, 64, 60) 60 -> 29; float32 11x11 at
-// (1, 51 -> 51, 32, 28) 455 -> 318, saving statistics; float32 7x7 at (4, 56 -> 6, 48, 34) 225 -> 133.
+// Measured (us, before -> after): float64 5x5 at (2, 8 -> 8, 64, 60) 60 -> 24; float32, saving statistics, 11x11 at
+// (1, 51 -> 51, 32, 28) 432 -> 266 and 7x7 at (4, 56 -> 6, 48, 34) 219 -> 110.
 #include <algorithm>
 
 #include "smorph_common.hpp"
