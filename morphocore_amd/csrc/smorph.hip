@@ -269,7 +269,7 @@ __global__ __launch_bounds__(BLOCK) void smorph_bwd_kernel(const SmorphBwdParams
                         if (in[r])
                         {
                             const T bt = p.beta[o];
-                            const T sref = p.sstats[oi], sinv = p.sstats[(int64_t)g.B * g.Cout * plane + oi], fin = p.out[oi];
+                            const T sref = p.sstats[oi], sinv = p.sstats[p.nsoft + oi], fin = p.out[oi];
                             const T c = outp[r];
                             const T pp = exp_ref((c - sref) * bt, lo) * sinv;
                             bsum = bsum + pp * (c - sref) * (c - fin) * gv;
@@ -465,6 +465,10 @@ __global__ __launch_bounds__(BLOCK) void smorph_soft_merge_kernel(const T* __res
 // Launch
 // ------------------------------------------------------------------------------------------------
 
+// Bytes of double grad_input sums that a float32 backward holds: larger batches take them in turn (at least one
+// element's, which are twice the size of its input).
+constexpr size_t SMORPH_SUMS_BYTES = size_t(1) << 30;
+
 struct SmorphBwdPlan
 {
     Tiling t;
@@ -477,6 +481,7 @@ struct SmorphBwdPlan
     // Workspace: grad_weight, grad_alpha and (SMOOTH) grad_beta partials, the double grad_input sums of float
     // tensors, winner counts and merge target (MAX / MIN), reduction scratch.
     size_t part_a, part_b, gacc, counts, scratch, bytes;
+    int gbatch;  // generic kernel: batch elements whose grad_input sums the workspace holds
     size_t lds;
 };
 
@@ -572,7 +577,9 @@ static SmorphBwdPlan plan_smorph_bwd(int merge, const Geom& g, bool saved = fals
     const bool smooth = merge == MERGE_SMOOTH;
     s.gacc = s.part_b + (smooth ? s.part_b - s.part_a : 0);
     const bool rounded = !stat && sizeof(T) != sizeof(Acc);
-    s.counts = s.gacc + (rounded ? align_up((size_t)g.B * g.Cin * g.plane() * sizeof(Acc)) : 0);
+    const size_t gin_bytes = (size_t)g.Cin * g.plane() * sizeof(Acc);  // of one batch element
+    s.gbatch = rounded && gin_bytes > 0 ? (int)std::max<int64_t>(1, std::min<int64_t>(g.B, (int64_t)(SMORPH_SUMS_BYTES / gin_bytes))) : g.B;
+    s.counts = s.gacc + (rounded ? align_up(s.gbatch * gin_bytes) : 0);
     // MAX / MIN: winner counts, then the merge target, per output pixel.
     s.scratch = s.counts + (merge == MERGE_MAX || merge == MERGE_MIN ? align_up(2 * (size_t)g.B * g.Cout * g.plane() * sizeof(T)) : 0);
     auto reduction = [&](int slots, int64_t n) { return stat ? reduce_slots_scratch<T>(slots, n) : reduce_slots_scratch<Acc>(slots, n); };
@@ -626,25 +633,43 @@ static hipError_t launch_smorph_bwd_generic(const SmorphBwdPlan& s, const Smorph
     return hipGetLastError();
 }
 
-// Zeros for everything the generic backward adds to: the partial slots and the grad_input sums behind them (one
-// launch; double tensors sum into grad_input itself).
-template <typename T>
-static hipError_t clear_smorph_sums(const SmorphBwdPlan& s, const Geom& g, unsigned char* ws, T* grad_in, hipStream_t stream)
+// The generic backward: zeros for everything it adds to (the partial slots and the grad_input sums behind them, one
+// launch; double tensors sum into grad_input itself), the kernel, and the sums rounded into float32 grad_input, for
+// s.gbatch batch elements at a time.
+template <typename T, int MK>
+static hipError_t run_smorph_bwd_generic(const SmorphBwdPlan& s, const SmorphBwdParams<T, Acc>& p, unsigned char* ws, T* grad_in,
+                                         hipStream_t stream)
 {
+    const Geom& g = p.g;
+    const int64_t plane = g.plane(), gin_n = (int64_t)g.Cin * plane, out_n = (int64_t)g.Cout * plane;
+    hipError_t err;
     if constexpr (sizeof(T) == sizeof(Acc))
+        if ((err = fill_async<T>(grad_in, g.B * gin_n, T(0), stream)) != hipSuccess) return err;
+    if ((err = fill_async<Acc>(reinterpret_cast<Acc*>(ws), (int64_t)(s.counts / sizeof(Acc)), Acc(0), stream)) != hipSuccess) return err;
+    Acc* const gacc = reinterpret_cast<Acc*>(ws + s.gacc);
+    for (int b0 = 0; b0 < g.B; b0 += s.gbatch)
     {
-        const hipError_t err = fill_async<T>(grad_in, (int64_t)g.B * g.Cin * g.plane(), T(0), stream);
-        if (err != hipSuccess) return err;
+        SmorphBwdParams<T, Acc> q = p;
+        q.g.B = std::min(s.gbatch, g.B - b0);
+        q.x += b0 * gin_n;
+        q.gout += b0 * out_n;
+        if (q.out) q.out += b0 * out_n;
+        if (q.counts) q.counts += b0 * out_n;
+        if (q.sstats) q.sstats += b0 * out_n;
+        const int64_t slot0 = (int64_t)b0 * s.nstrips;
+        q.part_w += slot0 * g.Cout * g.Cw * g.taps();
+        q.part_a += slot0 * s.npairs;
+        if (q.part_b) q.part_b += slot0 * g.Cin * g.Cout;
+        if constexpr (sizeof(T) == sizeof(Acc))
+            q.gin = reinterpret_cast<Acc*>(grad_in) + b0 * gin_n;
+        else
+            q.gin = gacc;
+        if (b0 > 0 && sizeof(T) != sizeof(Acc))
+            if ((err = fill_async<Acc>(gacc, q.g.B * gin_n, Acc(0), stream)) != hipSuccess) return err;
+        if ((err = launch_smorph_bwd_generic<T, MK>(s, q, stream)) != hipSuccess) return err;
+        if constexpr (sizeof(T) != sizeof(Acc))
+            if ((err = round_async<T>(gacc, grad_in + b0 * gin_n, q.g.B * gin_n, stream)) != hipSuccess) return err;
     }
-    return fill_async<Acc>(reinterpret_cast<Acc*>(ws), (int64_t)(s.counts / sizeof(Acc)), Acc(0), stream);
-}
-
-// The double grad_input sums of float tensors, rounded.
-template <typename T>
-static hipError_t round_smorph_gin(const SmorphBwdPlan& s, const Geom& g, const unsigned char* ws, T* grad_in, hipStream_t stream)
-{
-    if constexpr (sizeof(T) != sizeof(Acc))
-        return round_async<T>(reinterpret_cast<const Acc*>(ws + s.gacc), grad_in, (int64_t)g.B * g.Cin * g.plane(), stream);
     return hipSuccess;
 }
 
@@ -801,20 +826,17 @@ hipError_t smorph_backward(int merge, const T* x, const T* w, const T* alpha, co
             return reduce(p);
         }
     }
-    auto p = params(Acc(0));
-    p.gin = sizeof(T) == sizeof(Acc) ? reinterpret_cast<Acc*>(grad_in) : reinterpret_cast<Acc*>(ws + s.gacc);
-    if ((err = clear_smorph_sums<T>(s, g, ws, grad_in, stream)) != hipSuccess) return err;
+    const auto p = params(Acc(0));
     switch (merge)
     {
         case MERGE_ADD:
-        case MERGE_AVERAGE: err = launch_smorph_bwd_generic<T, MK_SUM>(s, p, stream); break;
-        case MERGE_MAX: err = launch_smorph_bwd_generic<T, MK_MAX>(s, p, stream); break;
-        case MERGE_MIN: err = launch_smorph_bwd_generic<T, MK_MIN>(s, p, stream); break;
-        case MERGE_IDENTITY: err = launch_smorph_bwd_generic<T, MK_IDENT>(s, p, stream); break;
+        case MERGE_AVERAGE: err = run_smorph_bwd_generic<T, MK_SUM>(s, p, ws, grad_in, stream); break;
+        case MERGE_MAX: err = run_smorph_bwd_generic<T, MK_MAX>(s, p, ws, grad_in, stream); break;
+        case MERGE_MIN: err = run_smorph_bwd_generic<T, MK_MIN>(s, p, ws, grad_in, stream); break;
+        case MERGE_IDENTITY: err = run_smorph_bwd_generic<T, MK_IDENT>(s, p, ws, grad_in, stream); break;
         default: return hipErrorInvalidValue;
     }
     if (err != hipSuccess) return err;
-    if ((err = round_smorph_gin<T>(s, g, ws, grad_in, stream)) != hipSuccess) return err;
     return reduce(p);
 }
 
@@ -935,6 +957,7 @@ hipError_t smorph_scm_backward(const T* x, const T* w, const T* alpha, const T* 
         p.part_b = reinterpret_cast<PT*>(ws + s.part_b);
         p.beta = beta;
         p.sstats = sstats;
+        p.nsoft = (int64_t)g.B * g.Cout * g.plane();
         p.g = g;
         p.t = s.t;
         p.nstrips = s.nstrips;
@@ -973,11 +996,8 @@ hipError_t smorph_scm_backward(const T* x, const T* w, const T* alpha, const T* 
             if ((err = launch_smorph_bwd_static(MK_SMOOTH, p, stream)) != hipSuccess) return err;
             return reduce(p);
         }
-    auto p = params(Acc(0));
-    p.gin = sizeof(T) == sizeof(Acc) ? reinterpret_cast<Acc*>(grad_in) : reinterpret_cast<Acc*>(ws + s.gacc);
-    if ((err = clear_smorph_sums<T>(s, g, ws, grad_in, stream)) != hipSuccess) return err;
-    if ((err = launch_smorph_bwd_generic<T, MK_SMOOTH>(s, p, stream)) != hipSuccess) return err;
-    if ((err = round_smorph_gin<T>(s, g, ws, grad_in, stream)) != hipSuccess) return err;
+    const auto p = params(Acc(0));
+    if ((err = run_smorph_bwd_generic<T, MK_SMOOTH>(s, p, ws, grad_in, stream)) != hipSuccess) return err;
     return reduce(p);
 }
 

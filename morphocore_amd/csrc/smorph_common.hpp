@@ -208,6 +208,7 @@ struct SmorphBwdParams
     // [slot][Cin][Cout].
     const T* __restrict__ beta;
     const T* __restrict__ sstats;
+    int64_t nsoft;  // generic kernel: elements between the two (B may be a chunk of the batch)
     PT* __restrict__ part_b;
     Geom g;
     Tiling t;

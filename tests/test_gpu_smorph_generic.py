@@ -151,3 +151,27 @@ def test_float32_slots_of_many_tiles_are_rounded_once(KH, KW):
     large[:, :, 46] = -large[:, :, 33]
     for got, want in list(zip(_gradients(x, w, alpha, small + large), _gradients(x, w, alpha, small)))[1:]:
         assert normwise_error(got, want) <= ONCE
+
+
+@pytest.mark.parametrize("merge", ["sum", "max", "identity", "smooth"])
+def test_float32_batches_whose_sums_exceed_the_workspace_bound(merge):
+    """Three batch elements of 544 MB of double grad_input sums each are taken one after the other: each gets the
+    gradients it has alone, and the element those summed over the batch."""
+    B, C, H, W, KH, KW = 3, 1, 8192, 8300, 1, 3
+    gen = torch.Generator(device="cuda").manual_seed(95)
+    x, g = (torch.randn(B, C, H, W, device="cuda", generator=gen) for _ in range(2))
+    w = seeded(96, C, C, KH, KW, kind="randn", scale=0.2).cuda()
+    alpha, beta = seeded(97, C, C, kind="randn").cuda(), seeded(98, C, kind="randn").cuda()
+
+    def grads(xs, gs):
+        leaves = [t.clone().requires_grad_() for t in (xs, w, alpha) + ((beta,) if merge == "smooth" else ())]
+        out = torch.ops.morphocore.smorph_scm(*leaves) if merge == "smooth" else torch.ops.morphocore.smorph(*leaves, O.MERGES[merge])
+        return torch.autograd.grad(out, leaves, gs)
+
+    whole = grads(x, g)
+    alone = [grads(x[b:b + 1], g[b:b + 1]) for b in range(B)]
+    for b in range(B):
+        assert torch.equal(whole[0][b], alone[b][0][0])
+    for k in range(1, len(whole)):
+        want = sum(a[k].double() for a in alone)
+        assert normwise_error(whole[k].cpu().numpy(), want.cpu().numpy()) <= 1e-6
